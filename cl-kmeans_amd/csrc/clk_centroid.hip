@@ -20,6 +20,7 @@
 // the FP64 global-atomic pass (of grid values, so exact as well) remains for
 // k too large for that.  `masses` is not read, as in the reference kernels.
 #include "clk_common.hpp"
+#include "clk_finalize.hpp"
 #include "clk_grid.hpp"
 #include "clk_kernels.hpp"
 
@@ -479,7 +480,7 @@ int run_centroid_update(clk_context *ctx, const clk_kernel_config *cfg, uint64_t
                                (uint32_t)d, (uint32_t)k, labels, sg, ps);
             CLK_HIP_CHECK(hipGetLastError());
         }
-        return launch_reduce_f64(ctx, ps, gx, dk, sums, true, stream);
+        return launch_merge_sums(ctx, ps, gx, dk, sums, stream);
     }
     if (strategy == CLK_CENTROID_FEATURE_SUM_PARDIM) {
         uint64_t lf = (cfg && cfg->local_features) ? cfg->local_features : 1;
@@ -529,7 +530,7 @@ int run_centroid_update(clk_context *ctx, const clk_kernel_config *cfg, uint64_t
                                stream, points, n, (uint32_t)d, (uint32_t)k, labels, sg, ps);
             CLK_HIP_CHECK(hipGetLastError());
         }
-        return launch_reduce_f64(ctx, ps, gxs, dk, sums, true, stream);
+        return launch_merge_sums(ctx, ps, gxs, dk, sums, stream);
     }
     if (!kern)
         return launch_accumulate_global(ctx, d, n, k, points, labels, sg, sums, nullptr, stream);
@@ -548,7 +549,7 @@ int run_centroid_update(clk_context *ctx, const clk_kernel_config *cfg, uint64_t
                                (uint32_t)d, (uint32_t)k, labels, sg, ps);
         CLK_HIP_CHECK(hipGetLastError());
     }
-    return launch_reduce_f64(ctx, ps, gx, dk, sums, true, stream);
+    return launch_merge_sums(ctx, ps, gx, dk, sums, stream);
 }
 
 }  // namespace clk

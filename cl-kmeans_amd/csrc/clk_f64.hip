@@ -20,6 +20,7 @@
 // buffers with global FP64 / uint64 atomics (order not fixed).  Labels are
 // bit-exact either way; sums differ from a serial sum only by FP64 rounding.
 #include "clk_common.hpp"
+#include "clk_finalize.hpp"
 #include "clk_kernels.hpp"
 
 #include <algorithm>
@@ -32,11 +33,13 @@ template <int DMAX, bool LABEL, bool SUMS, bool MASS, bool TILE>
 __global__ void __launch_bounds__(1024)
 f64_pass_kernel(const double *__restrict__ pts, uint64_t n, uint32_t d, uint32_t k,
                 const double *__restrict__ cen, uint64_t *__restrict__ labels,
-                double *__restrict__ part_sums, uint32_t *__restrict__ part_masses,
-                double *__restrict__ sums, uint64_t *__restrict__ masses)
+                double *__restrict__ part, double *__restrict__ sums, uint64_t *__restrict__ masses,
+                double *__restrict__ max_shift)
 {
     extern __shared__ __align__(16) double smem64[];
     const uint32_t B = blockDim.x, tid = threadIdx.x;
+    if (max_shift && blockIdx.x == 0 && tid == 0)
+        *max_shift = 0.0;  // the merge raises it
     double *cen_lds = smem64;                                        // LABEL: [k][DMAX]
     double *tile = cen_lds + (LABEL ? (size_t)k * DMAX : 0);         // SUMS && TILE: [d][k]
     uint32_t *cnt = reinterpret_cast<uint32_t *>(tile + (SUMS && TILE ? (size_t)d * k : 0));  // MASS && TILE
@@ -108,12 +111,16 @@ f64_pass_kernel(const double *__restrict__ pts, uint64_t n, uint32_t d, uint32_t
 
     if constexpr (TILE && (SUMS || MASS)) {
         __syncthreads();
-        if constexpr (SUMS)
+        // the partial row: the sums [d][k], then the masses [k]
+        double *row = part + (size_t)blockIdx.x * ((SUMS ? (size_t)d * k : 0) + (MASS ? k : 0));
+        if constexpr (SUMS) {
             for (uint32_t i = tid; i < d * k; i += B)
-                part_sums[(size_t)blockIdx.x * d * k + i] = tile[i];
+                row[i] = tile[i];
+            row += (size_t)d * k;
+        }
         if constexpr (MASS)
             for (uint32_t i = tid; i < k; i += B)
-                part_masses[(size_t)blockIdx.x * k + i] = cnt[i];
+                row[i] = (double)cnt[i];
     }
 }
 
@@ -155,20 +162,6 @@ f64_pass_global_kernel(const double *__restrict__ pts, uint64_t n, uint32_t d, u
         if constexpr (MASS)
             atomicAdd(reinterpret_cast<unsigned long long *>(&masses[lab]), 1ull);
     }
-}
-
-// masses[c] += sum over rows of part[row * k + c] (fixed order).
-__global__ void __launch_bounds__(256)
-reduce_masses_u64_kernel(const uint32_t *__restrict__ part, uint64_t rows, uint32_t k,
-                         uint64_t *__restrict__ masses)
-{
-    const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= k)
-        return;
-    uint64_t s = 0;
-    for (uint64_t r = 0; r < rows; ++r)
-        s += part[r * k + c];
-    masses[c] += s;
 }
 
 // centroids[f,c] = sums[f,c] / (double)masses[c] (0/0 = NaN for an empty
@@ -217,7 +210,7 @@ __global__ void add_u64_kernel(uint64_t *__restrict__ fst, const uint64_t *__res
 }
 
 using PassKernel = void (*)(const double *, uint64_t, uint32_t, uint32_t, const double *, uint64_t *,
-                            double *, uint32_t *, double *, uint64_t *);
+                            double *, double *, uint64_t *, double *);
 
 template <bool LABEL, bool SUMS, bool MASS, bool TILE>
 PassKernel pick_pass(int dmax)
@@ -254,11 +247,31 @@ int check_f64_sizes(uint64_t d, uint64_t n, uint64_t k)
     return CLK_OK;
 }
 
-// One pass: labels (LABEL) and/or accumulation into sums / masses.
+uint64_t f64_tile_bytes(uint64_t d, uint64_t k, bool sums, bool mass)
+{
+    return (sums ? d * k * 8 : 0) + (mass ? k * 4 : 0);
+}
+
+// Whether the fused pass's centroids and tile fit the work-group's LDS.
+bool f64_fused_tile_fits(const clk_context *ctx, uint64_t d, uint64_t k)
+{
+    const int dmax = dmax_f64(d);
+    return dmax && k * dmax * 8 + f64_tile_bytes(d, k, true, true) <= ctx->lds_per_block;
+}
+
+// The outputs of a whole iteration (clk_lloyd_step_f64).
+struct StepOut {
+    double *centroids;
+    double *max_shift;
+};
+
+// One pass: labels (LABEL) and/or accumulation into sums / masses.  With
+// `step` (a fused pass whose tile fits) sums and masses are overwritten and
+// the centroids divided in the same two launches.
 int run_f64_pass(clk_context *ctx, const clk_kernel_config *cfg, bool label, bool want_sums,
                  bool want_mass, uint64_t d, uint64_t n, uint64_t k, const double *points,
                  const double *centroids, uint64_t *labels, double *sums, uint64_t *masses,
-                 hipStream_t stream, const char *name)
+                 hipStream_t stream, const char *name, const StepOut *step = nullptr)
 {
     if (n == 0)
         return CLK_OK;
@@ -268,7 +281,7 @@ int run_f64_pass(clk_context *ctx, const clk_kernel_config *cfg, bool label, boo
     const int B = (int)b;
     const int dmax = dmax_f64(d);
     const uint64_t cen_bytes = label ? k * (uint64_t)std::max(dmax, 1) * 8 : 0;
-    const uint64_t tile_bytes = (want_sums ? d * k * 8 : 0) + (want_mass ? k * 4 : 0);
+    const uint64_t tile_bytes = f64_tile_bytes(d, k, want_sums, want_mass);
     const bool fits_cen = dmax != 0 && cen_bytes <= ctx->lds_per_block;
     const bool tile = fits_cen && cen_bytes + tile_bytes <= ctx->lds_per_block;
     PassKernel kern = nullptr;
@@ -288,30 +301,44 @@ int run_f64_pass(clk_context *ctx, const clk_kernel_config *cfg, bool label, boo
                     : kern ? auto_grid(ctx, (const void *)kern, B, lds, n)
                            : std::min<uint64_t>(need, (uint64_t)ctx->num_cus * 8);
     grid = std::max<uint64_t>(1, std::min<uint64_t>(grid, 1u << 16));
-    KernelTimer t(ctx, name, stream);
     if (kern) {
-        double *ps = nullptr;
-        uint32_t *pm = nullptr;
-        if (tile && want_sums) {
-            CLK_TRY(ensure_scratch(ctx->part_sums, grid * d * k * sizeof(double)));
-            ps = static_cast<double *>(ctx->part_sums.ptr);
+        const uint64_t nv = (want_sums ? d : 0) + (want_mass ? 1 : 0);
+        double *part = nullptr;
+        if (tile && nv) {
+            CLK_TRY(ensure_scratch(ctx->part_sums, grid * nv * k * sizeof(double)));
+            part = static_cast<double *>(ctx->part_sums.ptr);
         }
-        if (tile && want_mass) {
-            CLK_TRY(ensure_scratch(ctx->part_masses, grid * k * sizeof(uint32_t)));
-            pm = static_cast<uint32_t *>(ctx->part_masses.ptr);
-        }
-        hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(B), lds, stream, points, n, (uint32_t)d,
-                           (uint32_t)k, centroids, labels, ps, pm, sums, masses);
-        CLK_HIP_CHECK(hipGetLastError());
-        if (tile && want_sums)
-            CLK_TRY(launch_reduce_f64(ctx, ps, grid, d * k, sums, true, stream));
-        if (tile && want_mass) {
-            hipLaunchKernelGGL(reduce_masses_u64_kernel, dim3((unsigned)div_up(k, 256)), dim3(256), 0, stream,
-                               pm, grid, (uint32_t)k, masses);
+        {
+            KernelTimer t(ctx, name, stream);
+            hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(B), lds, stream, points, n, (uint32_t)d,
+                               (uint32_t)k, centroids, labels, part, sums, masses,
+                               step ? step->max_shift : nullptr);
             CLK_HIP_CHECK(hipGetLastError());
         }
-        return CLK_OK;
+        if (!part)
+            return CLK_OK;
+        MergeF64 m;
+        m.part = part;
+        m.rows = (uint32_t)grid;
+        m.mass = want_mass;
+        if (want_mass) {
+            m.d = want_sums ? (uint32_t)d : 0;
+            m.k = k;
+        } else {  // sums alone: one row of d*k values
+            m.d = 1;
+            m.k = d * k;
+        }
+        m.sums = sums;
+        m.masses = masses;
+        if (step) {
+            m.divide = true;
+            m.centroids = step->centroids;
+            m.old_centroids = centroids;
+            m.max_shift = step->max_shift;
+        }
+        return launch_merge(ctx, m, step ? "FinalizeDivide" : "ReduceVectorParcol", stream);
     }
+    KernelTimer t(ctx, name, stream);
     // beyond the register buckets or the LDS: global memory and atomics
     const int sel = (label ? 4 : 0) | (want_sums ? 2 : 0) | (want_mass ? 1 : 0);
     const dim3 g((unsigned)grid), bl(B);
@@ -387,9 +414,10 @@ extern "C" int clk_centroid_update_f64(clk_context *ctx, const clk_kernel_config
                         sums, nullptr, as_stream(stream), "CentroidUpdate");
 }
 
-extern "C" int clk_fused_f64(clk_context *ctx, const clk_kernel_config *cfg, uint64_t d, uint64_t n, uint64_t k,
-                             const double *points, const double *old_centroids, double *sums, uint64_t *labels,
-                             uint64_t *masses, void *stream)
+// clk_fused_f64, or with `step` the whole iteration (f64_fused_tile_fits).
+static int fused_f64(clk_context *ctx, const clk_kernel_config *cfg, uint64_t d, uint64_t n, uint64_t k,
+                     const double *points, const double *old_centroids, double *sums, uint64_t *labels,
+                     uint64_t *masses, void *stream, const StepOut *step = nullptr)
 {
     CLK_TRY(enter(ctx));
     CLK_TRY(require_stage(cfg, CLK_STAGE_FUSED, "clk_fused_f64: config is not a fused-stage config"));
@@ -400,7 +428,14 @@ extern "C" int clk_fused_f64(clk_context *ctx, const clk_kernel_config *cfg, uin
     CLK_REQUIRE(n == 0 || (points && old_centroids && sums && labels && masses), CLK_ERR_INVALID_ARGUMENT,
                 "fused_f64: null buffer");
     return run_f64_pass(ctx, cfg, true, true, true, d, n, k, points, old_centroids, labels, sums, masses,
-                        as_stream(stream), "FusedClusterMerge");
+                        as_stream(stream), "FusedClusterMerge", step);
+}
+
+extern "C" int clk_fused_f64(clk_context *ctx, const clk_kernel_config *cfg, uint64_t d, uint64_t n, uint64_t k,
+                             const double *points, const double *old_centroids, double *sums, uint64_t *labels,
+                             uint64_t *masses, void *stream)
+{
+    return fused_f64(ctx, cfg, d, n, k, points, old_centroids, sums, labels, masses, stream);
 }
 
 extern "C" int clk_matrix_divide_f64(clk_context *ctx, uint64_t d, uint64_t k, const double *sums,
@@ -427,6 +462,10 @@ extern "C" int clk_lloyd_step_f64(clk_context *ctx, const clk_kernel_config *cfg
     CLK_REQUIRE(new_centroids && new_centroids != old_centroids, CLK_ERR_INVALID_ARGUMENT,
                 "lloyd_step_f64: new_centroids must be set and must not alias old_centroids");
     CLK_REQUIRE(sums && masses, CLK_ERR_INVALID_ARGUMENT, "lloyd_step_f64: null buffer");
+    if (n != 0 && f64_fused_tile_fits(ctx, d, k)) {
+        const StepOut step{new_centroids, max_shift};
+        return fused_f64(ctx, cfg, d, n, k, points, old_centroids, sums, labels, masses, stream, &step);
+    }
     CLK_TRY(clk_fill_zero(ctx, sums, d * k * sizeof(double), stream));
     CLK_TRY(clk_fill_zero(ctx, masses, k * sizeof(uint64_t), stream));
     CLK_TRY(clk_fused_f64(ctx, cfg, d, n, k, points, old_centroids, sums, labels, masses, stream));

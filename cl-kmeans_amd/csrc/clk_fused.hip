@@ -18,10 +18,10 @@
 // (ds_add_u32), flushed into acc (ds_add_u64) every 64 values a cell can
 // take; feature_sum straight into acc.  All additions are exact integer
 // additions, so the sums do not depend on the grid or the order.  At the end
-// acc (times the unit) and the summed mass columns are written as
-// per-work-group FP64 / uint32 partials; a column reduction adds the
-// partials into the caller's sums and masses (exact: every partial is a
-// multiple of the unit below 2^53 units).
+// acc (times the unit) and the summed mass columns are written as the
+// work-group's FP64 partial row; the merge kernel (clk_finalize.hpp) adds the
+// rows into the caller's sums and masses (exact: every partial sum is a
+// multiple of the unit below 2^53 units) and, for a whole iteration, divides.
 #include "clk_common.hpp"
 #include "clk_finalize.hpp"
 #include "clk_grid.hpp"
@@ -45,11 +45,13 @@ template <int DMAX, int VEC, int BLOCK, bool PRIVATE, bool EXACT, bool BOUNDED>
 __global__ void __launch_bounds__(BLOCK > 0 ? BLOCK : (DMAX >= 64 ? 512 : 1024))
 fused_tile_kernel(const float *__restrict__ pts, uint64_t n, uint32_t d, uint32_t k,
                   const float *__restrict__ cen, uint32_t *__restrict__ labels, GridRef grid,
-                  double *__restrict__ part_sums, uint32_t *__restrict__ part_masses)
+                  double *__restrict__ part, double *__restrict__ max_shift)
 {
     extern __shared__ __align__(16) float smem[];
     const uint32_t B = BLOCK > 0 ? BLOCK : blockDim.x;
     const uint32_t tid = threadIdx.x;
+    if (max_shift && blockIdx.x == 0 && tid == 0)
+        *max_shift = 0.0;  // the merge raises it
     const uint32_t cols = PRIVATE ? B : 1;
     const uint32_t dk = d * k;
     const uint32_t rows = PRIVATE ? k * (d + 1) : k;
@@ -253,20 +255,16 @@ fused_tile_kernel(const float *__restrict__ pts, uint64_t n, uint32_t d, uint32_
         flush();
     __syncthreads();
 
-    for (uint32_t r = tid; r < k * (d + 1); r += B) {
-        // r < k: masses; then the d*k sums in [d][k] order
-        if (r < k) {
-            part_masses[(uint64_t)blockIdx.x * k + r] =
-                PRIVATE ? lds_row_sum_u32(tile + (uint64_t)r * (d + 1) * cols, cols, r) : tile[r];
-        } else {
-            const uint32_t i = r - k, f = i / k;
-            part_sums[(uint64_t)blockIdx.x * dk + i] = cell_value(acc[i], grid_unit(scl[f]), flg[i]);
-        }
-    }
+    // the partial row: d*k sums in [d][k] order, then the k masses
+    double *const row = part + (uint64_t)blockIdx.x * (dk + k);
+    for (uint32_t i = tid; i < dk; i += B)
+        row[i] = cell_value(acc[i], grid_unit(scl[i / k]), flg[i]);
+    for (uint32_t c = tid; c < k; c += B)
+        row[dk + c] = (double)(PRIVATE ? lds_row_sum_u32(tile + (uint64_t)c * (d + 1) * cols, cols, c) : tile[c]);
 }
 
 using FusedKernel = void (*)(const float *, uint64_t, uint32_t, uint32_t, const float *,
-                             uint32_t *, GridRef, double *, uint32_t *);
+                             uint32_t *, GridRef, double *, double *);
 
 // Points per work-item at most (VEC x DMAX values in registers, no spills).
 constexpr int fused_vec_cap(int dmax) { return dmax >= 32 ? 1 : dmax >= 16 ? 2 : 4; }
@@ -423,16 +421,15 @@ int run_fused(clk_context *ctx, const clk_kernel_config *cfg, uint64_t d, uint64
     if (lds > 65536)
         CLK_HIP_CHECK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     GridRef sgrid;
-    double *psums = nullptr;
-    uint32_t *pmasses = nullptr;
+    double *part = nullptr;
     if (ext) {
-        // [per-call grid d words, 256-aligned] [partial sums] [partial masses]:
-        // as many work-groups as the rows that fit (grid-stride: any count
-        // gives the same results)
+        // [per-call grid d words, 256-aligned] [partial rows]: as many
+        // work-groups as the rows that fit (grid-stride: any count gives the
+        // same results)
         const size_t head = ctx->grid_pinned ? 0 : ((d + 1) * sizeof(uint32_t) + 255) / 256 * 256;
-        const size_t row = d * k * sizeof(double) + k * sizeof(uint32_t);
+        const size_t row = (d + 1) * k * sizeof(double);
         const size_t fit = ext->bytes > head ? (ext->bytes - head) / row : 0;
-        CLK_REQUIRE(fit >= 1, CLK_ERR_SIZE, "lloyd_step_noalloc: k*(8d+4) exceeds the static scratch");
+        CLK_REQUIRE(fit >= 1, CLK_ERR_SIZE, "lloyd_step_noalloc: 8k(d+1) exceeds the static scratch");
         grid = std::min<uint64_t>(grid, fit);
         if (ctx->grid_pinned) {
             CLK_TRY(resolve_grid(ctx, d, n, points, stream, &sgrid));
@@ -443,30 +440,15 @@ int run_fused(clk_context *ctx, const clk_kernel_config *cfg, uint64_t d, uint64
             sgrid.bits = grid_bits(n);
             sgrid.own = 1;
         }
-        psums = reinterpret_cast<double *>(ext->ptr + head);
-        pmasses = reinterpret_cast<uint32_t *>(psums + grid * d * k);
+        part = reinterpret_cast<double *>(ext->ptr + head);
     } else {
         if (grid_in)
             sgrid = *grid_in;
         else
             CLK_TRY(resolve_grid(ctx, d, n, points, stream, &sgrid));
-        CLK_TRY(ensure_scratch(ctx->part_sums, grid * d * k * sizeof(double)));
-        CLK_TRY(ensure_scratch(ctx->part_masses, grid * k * sizeof(uint32_t)));
-        psums = static_cast<double *>(ctx->part_sums.ptr);
-        pmasses = static_cast<uint32_t *>(ctx->part_masses.ptr);
+        CLK_TRY(ensure_scratch(ctx->part_sums, grid * (d + 1) * k * sizeof(double)));
+        part = static_cast<double *>(ctx->part_sums.ptr);
     }
-    FinalizeArgs fa;
-    fa.part_sums = psums;
-    fa.part_masses = pmasses;
-    fa.rows = (uint32_t)grid;
-    fa.sums = sums;
-    fa.masses = masses;
-    fa.centroids = new_centroids;
-    fa.old_centroids = max_shift ? old_centroids : nullptr;
-    fa.max_shift = max_shift;
-    fa.d = (uint32_t)d;
-    fa.k = (uint32_t)k;
-    fa.mode = mode;
     {
         KernelTimer t(ctx,
                       !use_private ? "FusedFeatureSum"
@@ -474,23 +456,22 @@ int run_fused(clk_context *ctx, const clk_kernel_config *cfg, uint64_t d, uint64
                                    : "FusedClusterMerge",
                       stream);
         hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(B), lds, stream, points, n, (uint32_t)d,
-                           (uint32_t)k, old_centroids, labels, sgrid, psums, pmasses);
+                           (uint32_t)k, old_centroids, labels, sgrid, part, max_shift);
         CLK_HIP_CHECK(hipGetLastError());
     }
-    const size_t fin_lds = d * k * sizeof(double) + k * sizeof(uint32_t) + 12 * 1024 + 16;
-    if (fin_lds <= ctx->lds_per_block)
-        return launch_finalize(ctx, fa, stream);
-    // d*k beyond the one-work-group merge: column reduction, then divide.
-    if (mode == 2) {
-        CLK_TRY(clk_fill_zero(ctx, sums, d * k * sizeof(double), stream));
-        CLK_TRY(clk_fill_zero(ctx, masses, k * sizeof(uint32_t), stream));
-    }
-    CLK_TRY(launch_reduce_partials(ctx, fa.part_sums, d * k, sums, fa.part_masses, k, masses, grid,
-                                   stream));
-    if (mode == 2)
-        return clk_matrix_divide_row(ctx, d, k, sums, masses, new_centroids,
-                                     max_shift ? old_centroids : nullptr, max_shift, stream);
-    return CLK_OK;
+    MergeF32 m;
+    m.part = part;
+    m.rows = (uint32_t)grid;
+    m.d = (uint32_t)d;
+    m.k = k;
+    m.mass = true;
+    m.sums = sums;
+    m.masses = masses;
+    m.divide = mode == 2;
+    m.centroids = new_centroids;
+    m.old_centroids = old_centroids;
+    m.max_shift = max_shift;
+    return launch_merge(ctx, m, mode == 2 ? "FinalizeDivide" : "ReduceVectorParcol", stream);
 }
 
 int lloyd_step_with_grid(clk_context *ctx, const clk_kernel_config *cfg, uint64_t d, uint64_t n, uint64_t k,

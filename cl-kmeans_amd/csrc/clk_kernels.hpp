@@ -5,22 +5,11 @@
 
 namespace clk {
 
-// out[row] (+)= sum over col of in[col * rows + row], fixed order.
+// out[row] = sum over col of in[col * rows + row], fixed order.
 int launch_reduce_f64(clk_context *ctx, const double *in, uint64_t cols, uint64_t rows,
-                      double *out, bool accumulate, hipStream_t stream);
+                      double *out, hipStream_t stream);
 int launch_reduce_u32(clk_context *ctx, const uint32_t *in, uint64_t cols, uint64_t rows,
-                      uint32_t *out, bool accumulate, hipStream_t stream);
-
-// sums[r] += sum over col of ps[col*rows_s + r] (FP64) and
-// masses[r] += sum over col of pm[col*rows_m + r] (uint32), one launch.
-int launch_reduce_partials(clk_context *ctx, const double *ps, uint64_t rows_s, double *sums,
-                           const uint32_t *pm, uint64_t rows_m, uint32_t *masses, uint64_t cols,
-                           hipStream_t stream);
-
-struct FinalizeArgs;
-// Merge per-work-group partials into sums/masses (mode 1 accumulate, mode 2
-// overwrite + FP64 divide + optional shift): one work-group launch.
-int launch_finalize(clk_context *ctx, const FinalizeArgs &a, hipStream_t stream);
+                      uint32_t *out, hipStream_t stream);
 
 // Smallest register bucket >= d among 1,2,4,8,16,32,64; 0 when d > 64.
 inline int dmax_bucket(uint64_t d)

@@ -10,6 +10,7 @@
 // Integer arithmetic: every strategy gives identical, exact masses.  Labels
 // >= k are skipped.
 #include "clk_common.hpp"
+#include "clk_finalize.hpp"
 #include "clk_kernels.hpp"
 
 #include <algorithm>
@@ -199,7 +200,13 @@ int run_mass_update(clk_context *ctx, const clk_kernel_config *cfg, uint64_t n, 
                                n, (uint32_t)k, pm);
             CLK_HIP_CHECK(hipGetLastError());
         }
-        return launch_reduce_u32(ctx, pm, grid, k, masses, true, stream);
+        MergeU32 m;
+        m.part = pm;
+        m.rows = (uint32_t)grid;
+        m.k = k;
+        m.mass = true;
+        m.masses = masses;
+        return launch_merge(ctx, m, "ReduceVectorParcol", stream);
     }
     default:
         set_error("mass_update: unknown strategy id");

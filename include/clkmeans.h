@@ -183,7 +183,7 @@ int clk_lloyd_step(clk_context *ctx, const clk_kernel_config *cfg, uint64_t d,
  * points unless one is pinned) lives in one static device array of
  * CLK_NOALLOC_SCRATCH_BYTES per GPU, held until the process ends; the
  * persistent grid is clamped to the partial rows that fit.  CLK_ERR_SIZE when
- * one row, k*(8d+4) bytes, does not fit; CLK_ERR_UNSUPPORTED when k*d needs
+ * one row, 8k(d+1) bytes, does not fit; CLK_ERR_UNSUPPORTED when k*d needs
  * the separate labeling / mass / centroid stages (beyond the LDS tiles).
  * Every call on one GPU shares the array and leaves its contents there:
  * calls that overlap in time on one GPU race (order them on one stream).
