@@ -410,15 +410,23 @@ int run_fused(clk_context *ctx, const clk_kernel_config *cfg, uint64_t d, uint64
 
     const bool b256 = (B == 256);
     const bool exact = (uint64_t)dmax == d;
+    // The bounded pass is the faster one on settled labels where it keeps two
+    // work-groups per CU and the points dwarf its fixed costs (16M points,
+    // d=4 k=10: 84 us against 110-124 with split labels; d=8 k=8 123 / 146-188;
+    // but d=4 k=16, one work-group: 185 / 105-125, and 1M points d=4 k=10:
+    // 26 / 18-20).
+    const bool split = !(run_bounded && n >= (4u << 20) && 2 * priv_bytes <= ctx->lds_per_block) &&
+                       split_labeling_pays(ctx, cfg, d, n, k, true);
     FusedKernel kern = !use_private ? pick_fused<false, false>(dmax, exact, vec, b256)
                        : run_bounded ? pick_fused<true, true>(dmax, exact, vec, b256)
                                      : pick_fused<true, false>(dmax, exact, vec, b256);
     const size_t lds = use_private ? priv_bytes : shared_bytes;
     const uint64_t groups = n / vec;
     uint64_t grid = (cfg && cfg->global_size[0]) ? div_up(cfg->global_size[0], (uint64_t)B)
-                                                 : auto_grid(ctx, (const void *)kern, B, lds, groups);
+                    : split ? fused_split_rows(ctx, d, n, k)
+                            : auto_grid(ctx, (const void *)kern, B, lds, groups);
     grid = std::max<uint64_t>(1, std::min<uint64_t>(grid, 1u << 20));
-    if (lds > 65536)
+    if (lds > 65536 && !split)
         CLK_HIP_CHECK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     GridRef sgrid;
     double *part = nullptr;
@@ -449,12 +457,14 @@ int run_fused(clk_context *ctx, const clk_kernel_config *cfg, uint64_t d, uint64
         CLK_TRY(ensure_scratch(ctx->part_sums, grid * (d + 1) * k * sizeof(double)));
         part = static_cast<double *>(ctx->part_sums.ptr);
     }
-    {
-        KernelTimer t(ctx,
-                      !use_private ? "FusedFeatureSum"
-                      : run_bounded ? "FusedClusterMergeBounded"
-                                   : "FusedClusterMerge",
-                      stream);
+    const char *name = !use_private  ? "FusedFeatureSum"
+                       : run_bounded ? "FusedClusterMergeBounded"
+                                     : "FusedClusterMerge";
+    if (split) {
+        CLK_TRY(launch_fused_split(ctx, name, d, n, k, points, old_centroids, labels, sgrid, grid, part, max_shift,
+                                   stream));
+    } else {
+        KernelTimer t(ctx, name, stream);
         hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(B), lds, stream, points, n, (uint32_t)d,
                            (uint32_t)k, old_centroids, labels, sgrid, part, max_shift);
         CLK_HIP_CHECK(hipGetLastError());

@@ -28,6 +28,19 @@ int launch_labeling(clk_context *ctx, const clk_kernel_config *cfg, uint64_t d, 
                     uint64_t k, const float *points, const float *centroids, uint32_t *labels,
                     hipStream_t stream, bool bounded = false);
 
+// Split-operand MFMA labels (clk_split.hip): whether the labeling pass or
+// (fused) the fused pass takes them at these sizes, and the passes.  The fused
+// pass writes `rows` partial rows [d + 1][k] to part.
+bool split_labeling_pays(const clk_context *ctx, const clk_kernel_config *cfg, uint64_t d, uint64_t n, uint64_t k,
+                         bool fused);
+int launch_labeling_split(clk_context *ctx, uint64_t d, uint64_t n, uint64_t k, const float *points,
+                          const float *centroids, uint32_t *labels, hipStream_t stream);
+struct GridRef;
+uint64_t fused_split_rows(clk_context *ctx, uint64_t d, uint64_t n, uint64_t k);
+int launch_fused_split(clk_context *ctx, const char *name, uint64_t d, uint64_t n, uint64_t k, const float *points,
+                       const float *centroids, uint32_t *labels, const GridRef &grid, uint64_t rows, double *part,
+                       double *max_shift, hipStream_t stream);
+
 // Labels from x·cᵀ on MFMA (16-bit operands, FP32 accumulation) with an exact
 // FP32 relabel of near ties: the same labels as launch_labeling.  Supported
 // for d <= 128 and n < 2^32 when the 16-bit centroid table fits in LDS.
@@ -50,7 +63,6 @@ int run_centroid_update(clk_context *ctx, const clk_kernel_config *cfg, uint64_t
 // sums[f,c] += x_f (the grid value of x_f, clk_grid.hpp) and masses[c] += 1
 // for every point, with FP64 / u32 global atomics (any k*d; exact, so the
 // order of the atomics does not matter).  masses may be null.
-struct GridRef;
 int launch_accumulate_global(clk_context *ctx, uint64_t d, uint64_t n, uint64_t k,
                              const float *points, const uint32_t *labels, const GridRef &grid,
                              double *sums, uint32_t *masses, hipStream_t stream);

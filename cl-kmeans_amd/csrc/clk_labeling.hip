@@ -295,6 +295,8 @@ int launch_labeling(clk_context *ctx, const clk_kernel_config *cfg, uint64_t d, 
     const uint64_t B = (cfg && cfg->local_size[0]) ? cfg->local_size[0] : 256;
     CLK_REQUIRE(B <= (uint64_t)ctx->max_threads_per_block, CLK_ERR_INVALID_ARGUMENT,
                 "labeling: local_size exceeds the device limit");
+    if (!bounded && split_labeling_pays(ctx, cfg, d, n, k, false))
+        return launch_labeling_split(ctx, d, n, k, points, centroids, labels, stream);
     const int dmax = dmax_bucket(d);
     const uint64_t cen_plain = dmax ? ((k * dmax + 3) & ~3ull) * 4 : 0;
     // the bounded variant adds k keep thresholds; beyond LDS it runs as the

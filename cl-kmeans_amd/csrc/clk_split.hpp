@@ -1,0 +1,509 @@
+// Labeling on the matrix cores with split operands: scores of about FP32
+// accuracy from FP16 MFMA, so that few points need the exact scan.  One
+// launch, no scratch memory: each work-group builds the operand table of the
+// centroids in LDS.  The labels equal the sequential-fma scan's
+// (lloyd_fused_feature_sum.cl:213-239, kmeans_naive.cpp:49-63) bit for bit.
+//
+// Scores.  With a power of two s that puts max |c| into [2^12, 2^13), every
+// coordinate is split into two FP16 parts: s x = xh + xl (toward zero),
+// -2 s c = ch + cl (to nearest).  The MFMA accumulator starts at
+// RN(||s c||^2), so S_c = ||s c||^2 - 2 s^2 x.c up to a bounded error.
+// K = 32 of one 16x16x32 MFMA holds, for P padded features:
+//   P = 4, 8 all four products xh ch, xh cl, xl ch, xl cl of the features;
+//   P = 16   two MFMAs, (ch | cl) against (xh | xh) and (xl | xl);
+//   P >= 32  three MFMAs per 32 features: xh ch, xl ch, xh cl.
+// Scores may be negative: they are ranked as floats.  A key is the score with
+// its low bits replaced by an index.
+//
+// Error of one score (u = 2^-24, X >= ||s x|| over the padded features, C >= max ||s c||, N >= C^2):
+//   split of x   Rx = 2^-20 X + 1.01 * 2^-24 sqrt(d)  (toward zero: 2^-10
+//                relative per part, subnormal spacing 2^-24)
+//   split of c   Rc = 2^-22 2C + 1.01 * 2^-25 sqrt(d)
+//   inputs       (X + Rx) Rc + Rx 2C; P >= 32 also the dropped xl cl:
+//                (2^-10 X + 2^-24 sqrt(d)) (2^-11 2C + 2^-25 sqrt(d))
+//   summation    g (N + 1.004 X 2C), g = 2(T+1)u / (1 - 2(T+1)u) for the T
+//                products that are not padding (adding 0 is exact), each
+//                addition rounding or truncating
+//   norm         2u N
+// E = 1.01 x the sum + a bound on flushed denormals.  An FP16 subnormal must
+// reach the product: every launch checks that the matrix core keeps them, and
+// without that every point takes the exact scan.
+//
+// Margin.  vb, vs: the two smallest keys; tr the relative key error 2^(bits -
+// 23); e_c the reference's FP32 distance, within eps = (d+3)u relative (plus
+// d 2^-125 absolute) of ||x-c||^2.  With D = vb + tr|vb| + E + X^2 >= the
+// scaled ||x-c_b||^2,
+//   vs - vb > 1.01 (2E + tr'(|vb| + |vs|) + 2.1 eps D + 2 s^2 d 2^-125),
+// tr' = tr / (1 - tr),
+// makes c_b the strict, unique minimum of e_c.  Every other point -- and every
+// point with a coordinate that is not finite or too large for FP16 -- scans
+// all centroids with the reference's arithmetic, the 64 lanes of its wave
+// taking a centroid each.
+#pragma once
+
+#include "clk_common.hpp"
+#include "clk_mfma_device.hpp"
+
+namespace clk {
+namespace split {
+
+using mfma::f32v4;
+using mfma::u16x8;
+
+typedef __fp16 h16x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+
+constexpr float kNever = 3.0e38f;  // norm of a padded or non-finite centroid
+
+template <int P>
+struct Shape {
+    static constexpr int nkb = P < 32 ? 1 : P / 32;       // K-blocks of 32 features
+    static constexpr int nops = P < 32 ? 1 : 2 * nkb;     // operand vectors per tile of 16 centroids
+    static constexpr int terms = P < 32 ? 4 : 3;  // products per feature
+    static constexpr int planes = P < 32 ? P / 4 : 0;  // LDS exchange, u16x8 [64] each
+};
+
+// LDS of one work-group of `waves` waves: table, norms, FP32 centroids
+// (P < 32: [k][P], 0 past d), statistics, exchange.
+template <int P>
+__host__ __device__ constexpr size_t table_bytes(uint32_t ntiles)
+{
+    return (size_t)ntiles * Shape<P>::nops * 64 * sizeof(u16x8);
+}
+constexpr uint32_t kStatWords = 16;
+template <int P>
+__host__ __device__ constexpr size_t rows_bytes(uint32_t ntiles)
+{
+    return P < 32 ? (size_t)ntiles * 16 * P * sizeof(float) : 0;
+}
+template <int P>
+__host__ __device__ constexpr size_t lds_bytes(uint32_t ntiles, uint32_t waves)
+{
+    return table_bytes<P>(ntiles) + rows_bytes<P>(ntiles) + (size_t)ntiles * 16 * sizeof(float) +
+           kStatWords * sizeof(float) +
+           (size_t)waves * Shape<P>::planes * 64 * sizeof(u16x8);
+}
+
+__device__ __forceinline__ float min_f(float a, float b)
+{
+    float r;
+    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float max_f(float a, float b)
+{
+    float r;
+    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float min3_f(float a, float b, float c)
+{
+    float r;
+    asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+__device__ __forceinline__ float med3_f(float a, float b, float c)
+{
+    float r;
+    asm("v_med3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+
+// Two keys into (best, second): the two smallest of the four.
+__device__ __forceinline__ void push2(float &best, float &second, float a, float b)
+{
+    const float m = med3_f(best, a, b);
+    best = min3_f(best, a, b);
+    second = min_f(second, m);
+}
+
+__device__ __forceinline__ void merge_pair(float &b, float &s, float b2, float s2)
+{
+    s = min3_f(max_f(b, b2), s, s2);
+    b = min_f(b, b2);
+}
+
+// Swap the upper half-wave of a with the lower half-wave of b / the odd rows
+// of 16 lanes of a with the even rows of b.
+__device__ __forceinline__ void swap32(float &a, float &b)
+{
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void swap16(float &a, float &b)
+{
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+}
+
+// What the work-group's table says, wave-uniform.
+struct Table {
+    const u16x8 *ops;
+    const float *norm;
+    const float *rows;
+    uint32_t ntiles, kmask;
+    float scale;    // s
+    // the margin: t0 + tX ||s x|| + tx2 ||s x||^2 + tk (|vb| + |vs|)
+    float t0, tX, tx2, tk;
+    bool ok;
+};
+
+// The margin's coefficients (see the header; each is rounded up by far more
+// than the rounding of its evaluation and of the margin's).
+template <int P>
+__device__ __forceinline__ void set_margin(Table &t, float N, uint32_t d, uint32_t bits)
+{
+    constexpr float up = 1.0f + 1e-4f;
+    const float C2 = 2.0f * sqrtf(N) * up, sd = sqrtf((float)d) * up;
+    const float T = (float)(Shape<P>::terms * d);
+    const float g0 = 2.0f * (T + 1.0f) * mfma::kU;
+    const float gamma = g0 / (1.0f - g0) * up;
+    constexpr float alpha = 0x1p-20f;
+    const float beta = 1.01f * 0x1p-24f * sd;
+    const float Rc = 0x1p-22f * C2 + 1.01f * 0x1p-25f * sd;
+    float e1 = (1.0f + alpha) * Rc + alpha * C2 + gamma * 1.004f * C2;
+    float e0 = beta * (Rc + C2) + (gamma + 2.0f * mfma::kU) * N;
+    if constexpr (P >= 32) {
+        const float m = 0x1p-11f * C2 + 0x1p-25f * sd;
+        e1 += 0x1p-10f * m;
+        e0 += 0x1p-24f * sd * m;
+    }
+    e1 *= 1.01f;
+    e0 = 1.01f * e0 + (T + 2.0f) * 0x1p-125f;
+    const float eps = (float)(d + 3) * mfma::kU * up;
+    const float tr0 = __uint_as_float((bits - 23 + 127) << 23), tr = tr0 / (1.0f - tr0) * up;
+    const float under = t.scale * t.scale * (float)d * 0x1p-125f;
+    t.t0 = up * (1.01f * ((2.0f + 2.1f * eps) * e0 + 2.0f * under) + 1e-30f);
+    t.tX = up * 1.01f * (2.0f + 2.1f * eps) * e1;
+    t.tx2 = up * 1.01f * 2.1f * eps;
+    t.tk = up * 1.01f * (tr + 2.1f * eps * (1.0f + tr));
+}
+
+// Build the table of cen [d][k] (whole work-group; ends with a barrier).
+template <int P>
+__device__ __forceinline__ Table stage(const float *__restrict__ cen, uint32_t d, uint32_t k, uint32_t ntiles,
+                                       char *lds)
+{
+    using Sh = Shape<P>;
+    Table t;
+    u16x8 *ops = reinterpret_cast<u16x8 *>(lds);
+    float *norm = reinterpret_cast<float *>(lds + table_bytes<P>(ntiles));
+    float *rows = norm + ntiles * 16;
+    uint32_t *stat = reinterpret_cast<uint32_t *>(rows + rows_bytes<P>(ntiles) / sizeof(float));
+    const uint32_t tid = threadIdx.x, B = blockDim.x;
+    if (tid < kStatWords)
+        stat[tid] = 0;
+    __syncthreads();
+    // stat[0]: max |c| over the finite coordinates
+    uint32_t m = 0;
+#pragma unroll 4
+    for (uint32_t i = tid; i < d * k; i += B) {
+        const uint32_t u = __float_as_uint(__builtin_fabsf(cen[i]));
+        m = (u < 0x7F800000u && u > m) ? u : m;
+    }
+    for (int o = 32; o >= 1; o /= 2)
+        m = max(m, (uint32_t)__shfl_xor((int)m, o));
+    if (tid % 64 == 0 && m)
+        atomicMax(&stat[0], m);
+    __syncthreads();
+    const int ex = max((int)(stat[0] >> 23) - 127, -88);  // max |c| < 2^(ex + 1)
+    t.ok = ex <= 56;  // distances of points that FP16 holds stay far below FLT_MAX
+    const float s = __uint_as_float((uint32_t)(12 - (t.ok ? ex : 0) + 127) << 23);
+    t.scale = s;
+    for (uint32_t e = tid; e < ntiles * Sh::nops * 64; e += B) {
+        const uint32_t lane = e % 64, op = (e / 64) % Sh::nops, tile = e / (64 * Sh::nops);
+        const uint32_t c = tile * 16 + lane % 16, h = lane / 16;
+        const bool low = P == 8 ? (h & 1) != 0 : P == 16 ? h >= 2 : (op & 1) != 0;
+        const uint32_t f0 = P <= 8 ? 0 : P == 16 ? 8 * (h & 1) : (op / 2) * 32 + 8 * h;
+        u16x8 v;
+#pragma unroll
+        for (uint32_t j = 0; j < 8; ++j) {
+            // P = 4: (ch | cl) in the first two quarters, zeros in the others
+            const uint32_t f = P == 4 ? j % 4 : f0 + j;
+            const bool lo = P == 4 ? j >= 4 : low;
+            const bool in = c < k && f < d && (P != 4 || h < 2);
+            float x = cen[in ? (size_t)f * k + c : 0];
+            x = in && __builtin_fabsf(x) <= FLT_MAX ? -2.0f * s * x : 0.0f;
+            _Float16 p = (_Float16)x;
+            if (lo)
+                p = (_Float16)(x - (float)p);
+            v[j] = __builtin_bit_cast(uint16_t, p);
+        }
+        ops[e] = v;
+    }
+    if constexpr (P < 32)
+        for (uint32_t i = tid; i < k * P; i += B) {
+            const uint32_t c = i % k, f = i / k;
+            rows[c * P + f] = f < d ? cen[(size_t)f * k + c] : 0.0f;
+        }
+    uint32_t nmax = 0;
+    for (uint32_t c = tid; c < ntiles * 16; c += B) {
+        double q = 0.0;
+        bool fin = c < k;
+        const float *col = cen + (fin ? c : 0);
+#pragma unroll 8
+        for (uint32_t f = 0; f < d; ++f) {
+            const float v = col[(size_t)f * k];
+            fin = fin && __builtin_fabsf(v) <= FLT_MAX;
+            const double w = (double)(v * s);
+            q = __builtin_fma(w, w, q);
+        }
+        norm[c] = fin ? (float)q : kNever;
+        const uint32_t u = __float_as_uint((float)(q * (1.0 + 1e-6)));
+        nmax = fin && u > nmax ? u : nmax;
+    }
+    for (int o = 32; o >= 1; o /= 2)
+        nmax = max(nmax, (uint32_t)__shfl_xor((int)nmax, o));
+    if (tid % 64 == 0 && nmax)
+        atomicMax(&stat[1], nmax);
+    {  // does the matrix core keep FP16 subnormals?  32 x 2^-20 x 1
+        u16x8 a, b;
+        for (int j = 0; j < 8; ++j) {
+            a[j] = mfma::to16<true>(0x1p-20f);
+            b[j] = mfma::to16<true>(1.0f);
+        }
+        const f32v4 r = mfma::mma16<true>(a, b, f32v4{0.0f, 0.0f, 0.0f, 0.0f});
+        t.ok = t.ok && r[0] == 0x1p-15f;
+    }
+    __syncthreads();
+    t.ops = ops;
+    t.norm = norm;
+    t.rows = rows;
+    t.ntiles = ntiles;
+    uint32_t bits = 4;
+    while ((1u << bits) < ntiles * 16)
+        ++bits;
+    t.kmask = (1u << bits) - 1u;
+    set_margin<P>(t, __uint_as_float(stat[1]), d, bits);
+    return t;
+}
+
+// Two scaled coordinates -> their high and low FP16 parts, packed.
+__device__ __forceinline__ void split2(float a, float b, uint32_t &hi, uint32_t &lo)
+{
+    const h16x2 h = __builtin_amdgcn_cvt_pkrtz(a, b);
+    const h16x2 l = __builtin_amdgcn_cvt_pkrtz(a - (float)h[0], b - (float)h[1]);
+    hi = __builtin_bit_cast(uint32_t, h);
+    lo = __builtin_bit_cast(uint32_t, l);
+}
+
+// The wave's 64 points as B operands, four groups of 16.
+template <int P>
+struct PointOps {
+    u16x8 hi[4][Shape<P>::nkb];
+    u16x8 lo[P <= 8 ? 1 : 4][Shape<P>::nkb];  // P <= 8: hi holds both parts
+};
+
+// P <= 16: lane = point, coordinates x (past d any of
+// the point's coordinates again: the centroids are 0 there).  buf: this wave's
+// exchange planes.  Returns a bound >= ||s x||^2.
+template <int P>
+__device__ __forceinline__ float build_points(const float (&x)[P], float s, u16x8 *buf, uint32_t lane,
+                                              PointOps<P> &o)
+{
+    static_assert(P < 32, "lane = point form");
+    float x2 = 0.0f;
+    uint32_t hi[P / 2], lo[P / 2];
+#pragma unroll
+    for (int f = 0; f < P; f += 2) {
+        const float a = x[f] * s, b = x[f + 1] * s;
+        x2 = __builtin_fmaf(a, a, x2);
+        x2 = __builtin_fmaf(b, b, x2);
+        split2(a, b, hi[f / 2], lo[f / 2]);
+    }
+    const uint32_t q = lane % 16, h = lane / 16;
+    mfma::wave_lds_order();  // the previous step's reads are done
+    if constexpr (P == 4) {
+        buf[lane] = __builtin_bit_cast(u16x8, v4u{hi[0], hi[1], lo[0], lo[1]});
+        mfma::wave_lds_order();
+        typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+        const v2u *half = reinterpret_cast<const v2u *>(buf);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const v2u w = half[(g * 16 + q) * 2 + (h & 1)];
+            o.hi[g][0] = __builtin_bit_cast(u16x8, v4u{w.x, w.y, w.x, w.y});
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < P / 8; ++i) {
+            buf[i * 64 + lane] = __builtin_bit_cast(u16x8, v4u{hi[4 * i], hi[4 * i + 1], hi[4 * i + 2], hi[4 * i + 3]});
+            buf[(P / 8 + i) * 64 + lane] =
+                __builtin_bit_cast(u16x8, v4u{lo[4 * i], lo[4 * i + 1], lo[4 * i + 2], lo[4 * i + 3]});
+        }
+        mfma::wave_lds_order();
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            if constexpr (P == 8) {
+                o.hi[g][0] = buf[(h / 2) * 64 + g * 16 + q];
+            } else {
+                o.hi[g][0] = buf[(h & 1) * 64 + g * 16 + q];
+                o.lo[g][0] = buf[(2 + (h & 1)) * 64 + g * 16 + q];
+            }
+        }
+    }
+    return x2 * (1.0f + (float)(2 * P + 8) * mfma::kU);
+}
+
+// P >= 32: lane (q, h) holds raw[g][kb*8 + j] = feature kb*32 + 8h + j of
+// point g*16 + q (past d as above).  Returns a bound >= ||s x||^2 of this
+// lane's own point (lane 16h + q).
+template <int P>
+__device__ __forceinline__ float build_points(const float (&raw)[4][Shape<P>::nkb * 8], float s, uint32_t lane,
+                                              PointOps<P> &o)
+{
+    static_assert(P >= 32, "matrix layout");
+    float mine = 0.0f;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        float x2 = 0.0f;
+#pragma unroll
+        for (int kb = 0; kb < Shape<P>::nkb; ++kb) {
+            v4u hi, lo;
+#pragma unroll
+            for (int j = 0; j < 8; j += 2) {
+                const float a = raw[g][kb * 8 + j] * s, b = raw[g][kb * 8 + j + 1] * s;
+                x2 = __builtin_fmaf(a, a, x2);
+                x2 = __builtin_fmaf(b, b, x2);
+                uint32_t h, l;
+                split2(a, b, h, l);
+                hi[j / 2] = h;
+                lo[j / 2] = l;
+            }
+            o.hi[g][kb] = __builtin_bit_cast(u16x8, hi);
+            o.lo[g][kb] = __builtin_bit_cast(u16x8, lo);
+        }
+        x2 += mfma::xor_swizzle<16>(x2);
+        x2 += __shfl_xor(x2, 32);
+        mine = (uint32_t)g == lane / 16 ? x2 : mine;
+    }
+    return mine * (1.0f + (float)(2 * P + 8) * mfma::kU);
+}
+
+// The two smallest keys of this lane's own point over all centroids.  A key's
+// low bits hold (4 tile + i) * 4 + h for row 4h + i of a tile: the tile and
+// row parts are the same for all lanes (scalar operands), h is put in once
+// after the last tile; centroid_of undoes it.
+__device__ __forceinline__ uint32_t centroid_of(float key, uint32_t kmask)
+{
+    const uint32_t l = __float_as_uint(key) & kmask;
+    return (l & ~15u) | ((l & 3u) << 2) | ((l >> 2) & 3u);
+}
+
+template <int P>
+__device__ __forceinline__ void rank_points(const Table &t, const PointOps<P> &x, uint32_t lane, float &best,
+                                            float &second)
+{
+    using Sh = Shape<P>;
+    const uint32_t h = lane / 16;
+    float b[4], s[4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+        b[g] = s[g] = FLT_MAX;
+    const uint32_t vkeep = mfma::opaque_v(~t.kmask);
+    for (uint32_t tile = 0; tile < t.ntiles; ++tile) {
+        const f32v4 nrm = *reinterpret_cast<const f32v4 *>(t.norm + tile * 16 + 4 * h);
+        f32v4 acc[4];
+#pragma unroll
+        for (int kb = 0; kb < Sh::nkb; ++kb) {
+            if constexpr (P < 32) {
+                const u16x8 a = t.ops[tile * 64 + lane];
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+                    acc[g] = mfma::mma16<true>(a, x.hi[g][0], nrm);
+                if constexpr (P == 16)
+#pragma unroll
+                    for (int g = 0; g < 4; ++g)
+                        acc[g] = mfma::mma16<true>(a, x.lo[g][0], acc[g]);
+            } else {
+                const u16x8 ah = t.ops[(tile * Sh::nops + 2 * kb) * 64 + lane];
+                const u16x8 al = t.ops[(tile * Sh::nops + 2 * kb + 1) * 64 + lane];
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+                    acc[g] = mfma::mma16<true>(ah, x.hi[g][kb], kb == 0 ? nrm : acc[g]);
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+                    acc[g] = mfma::mma16<true>(ah, x.lo[g][kb], acc[g]);
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+                    acc[g] = mfma::mma16<true>(al, x.hi[g][kb], acc[g]);
+            }
+        }
+        uint32_t idx[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            idx[i] = mfma::opaque_s((4 * tile + i) * 4);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            float key[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                key[i] = __uint_as_float((__float_as_uint(acc[g][i]) & vkeep) | idx[i]);
+            push2(b[g], s[g], key[0], key[1]);
+            push2(b[g], s[g], key[2], key[3]);
+        }
+    }
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+        b[g] = __uint_as_float(__float_as_uint(b[g]) | h);
+    // The four lanes of a column hold the four row quarters of every group:
+    // after two exchanges lane row h holds group h, merged.
+    swap32(b[0], b[2]);
+    swap32(s[0], s[2]);
+    merge_pair(b[0], s[0], b[2], s[2]);
+    swap32(b[1], b[3]);
+    swap32(s[1], s[3]);
+    merge_pair(b[1], s[1], b[3], s[3]);
+    swap16(b[0], b[1]);
+    swap16(s[0], s[1]);
+    merge_pair(b[0], s[0], b[1], s[1]);
+    best = b[0];
+    second = s[0];
+}
+
+// Margin test of this lane's own point; lab = the best key's centroid.
+__device__ __forceinline__ bool decide(const Table &t, float x2, float best, float second, uint32_t k, uint32_t &lab)
+{
+    const float X = __builtin_amdgcn_sqrtf(x2);  // within one ulp
+    const float ab = __builtin_fabsf(best);
+    float tau = __builtin_fmaf(t.tX, X, t.t0);
+    tau = __builtin_fmaf(t.tx2, x2, tau);
+    tau = __builtin_fmaf(t.tk, ab + __builtin_fabsf(second), tau);
+    lab = centroid_of(best, t.kmask);
+    // NaN fails every test; 4.2e9 < 65504^2; a key of denormal size is not
+    // trusted to keep its index
+    return t.ok && x2 < 4.2e9f && best < 1e37f && ab > 1e-30f && second - best > tau && lab < k;
+}
+
+// The reference's scan of one point over all centroids, a centroid per lane
+// and round; dist_to(col) gives the point's distance to the centroid whose
+// column of cen [d][k] starts at col.
+template <typename DistTo>
+__device__ __forceinline__ uint32_t exact_scan(const float *__restrict__ cen, uint32_t k, uint32_t lane,
+                                               DistTo &&dist_to)
+{
+    float best = FLT_MAX;
+    uint32_t bi = 0;
+    for (uint32_t c0 = 0; c0 < k; c0 += 64) {
+        const uint32_t c = c0 + lane;
+        const float dist = dist_to(cen + min(c, k - 1));
+        if (c < k && dist < best) {
+            best = dist;
+            bi = c;
+        }
+    }
+    // smallest distance, lowest index on equal distances; none below FLT_MAX
+    // gives label 0
+    uint32_t hi = __float_as_uint(best);
+    for (int o = 32; o >= 1; o /= 2) {
+        const uint32_t h2 = (uint32_t)__shfl_xor((int)hi, o), i2 = (uint32_t)__shfl_xor((int)bi, o);
+        const bool take = h2 < hi || (h2 == hi && i2 < bi);
+        hi = take ? h2 : hi;
+        bi = take ? i2 : bi;
+    }
+    return hi < __float_as_uint(FLT_MAX) ? bi : 0u;
+}
+
+}  // namespace split
+}  // namespace clk

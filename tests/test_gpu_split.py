@@ -1,0 +1,72 @@
+"""Split-operand MFMA labels (clk_split.hpp) at the edges of its shapes: the
+labels, masses and grid-exact sums equal the oracle's, exactly."""
+import numpy as np
+import pytest
+
+import clkmeans
+from clkmeans import hip
+from oracle import oracle as O
+from tests.helpers import dev, zeros
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [  # n, d, k: operand forms of 8, 16, 32 .. 128 features, tile and batch remainders
+    (5000, 1, 130), (4096, 2, 64), (4097, 3, 100), (70001, 7, 33), (6000, 8, 16), (5555, 8, 17), (4160, 9, 31),
+    (30003, 13, 48), (5000, 16, 97), (4500, 17, 15), (9001, 24, 48), (4100, 32, 256), (6001, 33, 40), (4200, 64, 129),
+    (4111, 65, 30), (4100, 96, 65), (4099, 97, 33), (4096, 128, 100), (5000, 5, 1200), (4300, 30, 700),
+]
+
+
+def points(n, d, k, kind, seed):
+    rng = np.random.default_rng(seed)
+    if kind == "blobs":  # overlapping: many undecided points
+        return clkmeans.generate_blobs(n, d, k, sigma=2.0, box=8.0, seed=seed)[0]
+    if kind == "lattice":  # exact ties and duplicated centroids
+        return rng.integers(-3, 4, (d, n)).astype(np.float32)
+    if kind == "offset":  # large norms against small gaps
+        return (rng.standard_normal((d, n)) + 300.0).astype(np.float32)
+    p = rng.standard_normal((d, n)).astype(np.float32)  # "special"
+    p *= np.float32(2.0) ** rng.integers(-130, 100, n).astype(np.float32)
+    p[0, 7::53], p[d - 1, 9::59], p[0, 11::61] = np.nan, np.inf, -np.inf
+    return p
+
+
+def centroids(pts, k, kind):
+    c = np.ascontiguousarray(pts[:, np.arange(k) * 2 % pts.shape[1]])
+    if kind == "special":
+        c[~np.isfinite(c)] = 1.0
+        c[0, k // 2] = np.nan
+        c[0, k // 3] = np.inf
+    return c
+
+
+@pytest.mark.parametrize("kind", ["blobs", "lattice", "offset", "special"])
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "n%d_d%d_k%d" % s)
+def test_split_labels_and_sums(gpu_ctx, shape, kind):
+    n, d, k = shape
+    pts = points(n, d, k, kind, n + d + k)
+    cen = centroids(pts, k, kind)
+    ref = O.label(pts, cen)
+    dp, dc = dev(pts), dev(cen)
+    labels = dev(np.full(n, 0xFFFFFFFF, np.uint32))
+    gpu_ctx.labeling(gpu_ctx.config(clkmeans.STAGE_LABELING, "unroll_vector"), d, n, k, dp, dc, labels)
+    hip.synchronize()
+    np.testing.assert_array_equal(labels.to_host(), ref)
+    labels = dev(np.full(n, 0xFFFFFFFF, np.uint32))
+    sums, masses = zeros((d, k), np.float64), zeros(k, np.uint32)
+    gpu_ctx.fused(gpu_ctx.config(clkmeans.STAGE_FUSED, "feature_sum"), d, n, k, dp, dc, sums, labels, masses)
+    hip.synchronize()
+    np.testing.assert_array_equal(labels.to_host(), ref)
+    np.testing.assert_array_equal(masses.to_host(), O.mass(ref, k))
+    np.testing.assert_array_equal(sums.to_host(), O.sums_grid(pts, ref, k, O.grid_scales(pts)))
+
+
+@pytest.mark.parametrize("scale", [2.0 ** -100, 2.0 ** -40, 2.0 ** 40, 2.0 ** 60])
+def test_split_scales(gpu_ctx, scale):
+    n, d, k = 8000, 6, 60
+    pts = (clkmeans.generate_blobs(n, d, k, sigma=1.0, box=10.0, seed=3)[0] * np.float32(scale)).astype(np.float32)
+    cen = np.ascontiguousarray(pts[:, :k])
+    labels = zeros(n, np.uint32)
+    gpu_ctx.labeling(gpu_ctx.config(clkmeans.STAGE_LABELING, "unroll_vector"), d, n, k, dev(pts), dev(cen), labels)
+    hip.synchronize()
+    np.testing.assert_array_equal(labels.to_host(), O.label(pts, cen))
