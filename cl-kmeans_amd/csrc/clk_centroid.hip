@@ -9,16 +9,20 @@
 //                       (lloyd_feature_sum_pardim.cl's points x feature tiles)
 //   feature_sum         one LDS accumulator [d][k] shared by the work-group,
 //                       work-items stride over the flattened feature-major
-//                       matrix (coalesced rows); the smallest LDS footprint
+//                       matrix (coalesced rows)
+// With an automatic launch geometry every strategy takes the kernel that is
+// fastest for the sizes (the results are the same): cluster_merge's private
+// tile for a few cells, else the cell kernel below, which shares the
+// accumulators of a slice of features; the strategies' own kernels serve the
+// launch geometries that name them.
 // Every coordinate is rounded to its grid integer and added exactly
 // (clk_grid.hpp): the private int32 columns flush into the work-group's
 // int64 accumulator (ds_add_u64) at least every 64 values, shared
 // accumulators take ds_add_u64 directly.  The work-group's sums (times the
-// unit) form its FP64 partial row; a column reduction adds the rows (exact).
-// So every strategy and geometry gives the same bits.  For large k*d (when
-// neither fits) every strategy uses the cluster-major slice kernel below;
-// the FP64 global-atomic pass (of grid values, so exact as well) remains for
-// k too large for that.  `masses` is not read, as in the reference kernels.
+// unit) form its FP64 partial row; the merge adds the rows (exact).  So every
+// strategy and geometry gives the same bits.  The FP64 global-atomic pass (of
+// grid values, so exact as well) remains for k beyond the LDS.  `masses` is
+// not read, as in the reference kernels.
 #include "clk_common.hpp"
 #include "clk_finalize.hpp"
 #include "clk_grid.hpp"
@@ -296,101 +300,159 @@ cu_feature_sum_kernel(const float *__restrict__ pts, uint64_t n, uint32_t d, uin
         part[(uint64_t)blockIdx.x * rows + i] = cell_value(h.acc[i], grid_unit(h.scl[i / k]), h.flg[i]);
 }
 
-// Cluster-major feature slices for large k*d.  blockIdx.y selects features
-// [4*blockIdx.y, +4); the work-group shares one int64 accumulator [k][4] in
-// LDS.  A wave takes 64 consecutive points (lane = point: 4 coalesced
-// feature loads and the label) and adds each point's grid integers into its
-// cluster's row with ds_add_u64 (exact, so no ordering between lanes or
-// waves is needed).  The accumulator (times the units) is the work-group's
-// partial row.
-constexpr uint32_t kSliceF = 4, kSliceWaves = 4, kSlicePrefetch = 8;
+// Cells of a feature slice: blockIdx.y selects features [F*blockIdx.y, +F),
+// the work-group shares int64 accumulators [R][F][k] in LDS.  A wave takes 64
+// consecutive points per step (lane = point: F coalesced loads and the label)
+// and adds each point's grid integers into its cluster's cells with ds_add_u64
+// (exact, so no ordering between lanes or waves is needed); R replicas (lane
+// mod R) thin out the same-cell additions of a wave when k is small.
+// Bound by the points' bytes from a few million points on: 16M points d=64
+// k=1024 648 us (6.4 TB/s; 32-bit flags, four features per slice and a quarter
+// more label reads took 730), d=32 k=256 339 us (6.2 TB/s).  Against the
+// kernels it replaces: 400k points d=32 k=256 168 -> 16 us (a 64-bit division
+// per element), 10M d=5 k=20 78 -> 46 us (one private-tile work-group per CU).
+constexpr uint32_t kCellWaves = 8;
 
-size_t slice_lds_bytes(uint64_t k)
+// LDS of a cell kernel: scales [F] | cells | flag bytes.
+size_t cell_lds_bytes(uint32_t F, uint64_t k, uint32_t R)
 {
-    return (size_t)acc_head_words(kSliceF, (uint32_t)k) * 4;
+    return ((size_t)F * 4 + 15) / 16 * 16 + (size_t)R * F * k * 8 + (F * k + 3) / 4 * 4;
 }
 
-__global__ void __launch_bounds__(64 * kSliceWaves)
-cu_slice_kernel(const float *__restrict__ pts, uint64_t n, uint32_t d, uint32_t k,
-                const uint32_t *__restrict__ labels, GridRef grid, double *__restrict__ part)
+template <int F>
+__global__ void __launch_bounds__(64 * kCellWaves)
+cu_cell_kernel(const float *__restrict__ pts, uint64_t n, uint32_t d, uint32_t k, const uint32_t *__restrict__ labels,
+               GridRef grid, uint32_t R, double *__restrict__ part)
 {
-    extern __shared__ __align__(16) float lds_sl[];
-    typedef float f4 __attribute__((ext_vector_type(4)));
+    extern __shared__ __align__(16) char lds_cell[];
+    constexpr uint32_t B = 64 * kCellWaves;
+    constexpr int kRing = F >= 16 ? 2 : F >= 8 ? 4 : 8;  // steps in flight
     // the wave index as a scalar: tile indices and the loop below are then
-    // wave-uniform, so the prefetch ring needs no divergent control flow
+    // wave-uniform, so the ring needs no divergent control flow
     const uint32_t tid = threadIdx.x, lane = tid % 64;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid / 64));
-    const uint32_t f0 = blockIdx.y * kSliceF;
-    const uint32_t nf = min(kSliceF, d - f0);
-    const AccHead h = acc_head(lds_sl, kSliceF, k, f0, d, grid, tid, blockDim.x);
+    const uint32_t f0 = blockIdx.y * F;
+    const uint32_t nf = min((uint32_t)F, d - f0), cells = F * k;
+    float *scl = reinterpret_cast<float *>(lds_cell);
+    long long *acc = reinterpret_cast<long long *>(lds_cell + (F * 4 + 15) / 16 * 16);
+    uint32_t *flg = reinterpret_cast<uint32_t *>(acc + (size_t)R * cells);  // a byte per cell
+    for (uint32_t j = tid; j < F; j += B)
+        scl[j] = j < nf ? grid_scale(grid.gmax[f0 + j], grid.bits) : 1.0f;
+    for (uint32_t i = tid; i < R * cells; i += B)
+        acc[i] = 0;
+    for (uint32_t i = tid; i < (cells + 3) / 4; i += B)
+        flg[i] = 0u;
     __syncthreads();
-    float sc[kSliceF];
+    float sc[F];
 #pragma unroll
-    for (uint32_t j = 0; j < kSliceF; ++j)
-        sc[j] = h.scl[j];
+    for (int j = 0; j < F; ++j)
+        sc[j] = __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(scl[j])));
+    const bool on_grid = grid.own != 0 && grid.gmax[d] == 0;
+    long long *const mine = acc + (size_t)(lane & (R - 1)) * cells;
     const uint64_t tiles = (n + 63) / 64;
-    const uint64_t tstride = (uint64_t)gridDim.x * kSliceWaves;
+    const uint64_t stride = (uint64_t)gridDim.x * kCellWaves;
     // Every load is unconditional and in bounds (a tile past the end reads
-    // the last tile, a feature past the slice reads its last feature; such
-    // values are never added), so no branch separates a load from its use
-    // and the loads of later tiles stay in flight.
-    auto load = [&](uint64_t tile, f4 &v, uint32_t &L) {
-        const uint64_t p = min(min(tile, tiles - 1) * 64 + lane, n - 1);
+    // the last tile, a point past the end the last point, a feature past the
+    // slice its last feature; such values are never added), so no branch
+    // separates a load from its use and the later tiles' loads stay in flight.
+    auto load = [&](uint64_t tile, float (&v)[F], uint32_t &L) {
+        const uint64_t at = tile < tiles ? tile : tiles - 1;
+        const uint64_t left = n - 1 - at * 64;
+        const uint32_t off = min(lane, left < 63 ? (uint32_t)left : 63u);
+        const float *base = pts + at * 64 + (uint64_t)f0 * n;
 #pragma unroll
-        for (uint32_t j = 0; j < kSliceF; ++j)
-            v[j] = pts[(uint64_t)(f0 + min(j, nf - 1)) * n + p];
-        L = labels[p];
+        for (int j = 0; j < F; ++j)
+            v[j] = stream_load(base + (uint64_t)min((uint32_t)j, nf - 1) * n + off);
+        L = (labels + at * 64)[off];  // other slices read them too: cached
     };
-    // A ring of kSlicePrefetch tiles in registers: the loads of the next
-    // kSlicePrefetch tiles of this wave are in flight while one is added
-    // (one tile alone leaves too few bytes in flight to cover HBM latency).
-    // The ring is indexed by the unrolled slot, so it stays in registers.
-    f4 vr[kSlicePrefetch];
-    uint32_t Lr[kSlicePrefetch];
-    const uint64_t first = (uint64_t)blockIdx.x * kSliceWaves + wave;
-    // this wave's tiles first + i*tstride, i < mine: full rounds of the ring
-    // in a loop with no early exit (so every path into its head has issued
-    // the same loads), then the partial last round
-    const uint64_t mine = first < tiles ? (tiles - first + tstride - 1) / tstride : 0;
-    const uint64_t rounds = mine / kSlicePrefetch;
-    const uint32_t rest = (uint32_t)(mine % kSlicePrefetch);
-    auto add = [&](uint64_t tile, f4 v, uint32_t L) {
-        const bool valid = tile * 64 + lane < n && L < k;
-        if (valid) {
+    auto add = [&](uint64_t tile, const float (&v)[F], uint32_t L) {
+        if (tile * 64 + lane >= n || L >= k)
+            return;
+        if (on_grid) {
 #pragma unroll
-            for (uint32_t j = 0; j < kSliceF; ++j)
-                if (j < nf) {
+            for (int j = 0; j < F; ++j)
+                if (j < (int)nf)
+                    lds_add64(mine + j * k + L, (long long)grid_q_on(v[j], sc[j]));
+        } else {
+#pragma unroll
+            for (int j = 0; j < F; ++j)
+                if (j < (int)nf) {
                     bool ok;
                     const int32_t q = grid_q(v[j], sc[j], ok);
-                    lds_add64(h.acc + j * k + L, (long long)q);
-                    if (__builtin_expect(!ok, 0))
-                        lds_or(h.flg + j * k + L, special_flag(v[j]));
+                    lds_add64(mine + j * k + L, (long long)q);
+                    if (__builtin_expect(!ok, 0)) {
+                        const uint32_t i = j * k + L;
+                        lds_or(flg + i / 4, special_flag(v[j]) << 8 * (i % 4));
+                    }
                 }
         }
     };
+    // this wave's tiles first + i*stride, i < count: full rounds of the ring
+    // in a loop with no early exit, then the partial last round
+    const uint64_t first = (uint64_t)blockIdx.x * kCellWaves + wave;
+    const uint64_t count = first < tiles ? (tiles - first + stride - 1) / stride : 0;
+    const uint64_t rounds = count / kRing;
+    const uint32_t rest = (uint32_t)(count % kRing);
+    float v[kRing][F];
+    uint32_t L[kRing];
 #pragma unroll
-    for (uint32_t s = 0; s < kSlicePrefetch; ++s)
-        load(first + s * tstride, vr[s], Lr[s]);
-    uint64_t base = first;
-    for (uint64_t r = 0; r < rounds; ++r, base += kSlicePrefetch * tstride) {
+    for (int s = 0; s < kRing; ++s)
+        load(first + s * stride, v[s], L[s]);
+    uint64_t at = first;
+    for (uint64_t r = 0; r < rounds; ++r, at += kRing * stride) {
 #pragma unroll
-        for (uint32_t s = 0; s < kSlicePrefetch; ++s) {
-            const uint64_t tile = base + s * tstride;  // wave-uniform, < tiles
-            add(tile, vr[s], Lr[s]);
+        for (int s = 0; s < kRing; ++s) {
+            const uint64_t tile = at + s * stride;  // wave-uniform, < tiles
+            add(tile, v[s], L[s]);
             // refill the slot once its tile is added: its registers are free
-            load(tile + kSlicePrefetch * tstride, vr[s], Lr[s]);
+            load(tile + kRing * stride, v[s], L[s]);
         }
     }
 #pragma unroll
-    for (uint32_t s = 0; s < kSlicePrefetch; ++s)
-        if (s < rest)
-            add(base + s * tstride, vr[s], Lr[s]);
+    for (int s = 0; s < kRing; ++s)
+        if (s < (int)rest)
+            add(at + s * stride, v[s], L[s]);
     __syncthreads();
-    for (uint32_t i = tid; i < k * nf; i += blockDim.x) {
-        const uint32_t j = i / k, c = i % k;
-        part[(uint64_t)blockIdx.x * ((uint64_t)d * k) + (uint64_t)(f0 + j) * k + c] =
-            cell_value(h.acc[i], grid_unit(h.scl[j]), h.flg[i]);
+    double *const row = part + (uint64_t)blockIdx.x * ((uint64_t)d * k) + (uint64_t)f0 * k;
+    for (uint32_t i = tid; i < nf * k; i += B) {
+        long long q = 0;
+        for (uint32_t r = 0; r < R; ++r)
+            q += acc[(size_t)r * cells + i];
+        row[i] = cell_value(q, grid_unit(scl[i / k]), (flg[i / 4] >> 8 * (i % 4)) & 7u);
     }
+}
+
+using CellKernel = void (*)(const float *, uint64_t, uint32_t, uint32_t, const uint32_t *, GridRef, uint32_t, double *);
+
+struct CellPlan {
+    CellKernel kern = nullptr;
+    uint32_t F = 0, R = 1;
+    size_t lds = 0;
+};
+
+// The widest slice whose cells leave a CU two work-groups (every wave slot):
+// each slice reads the labels again, and loads of more features overlap.
+// Else the narrowest slice that fits at all.  Replicas as far as a CU keeps
+// its two work-groups and k is small enough for a wave's labels to meet.
+CellPlan cell_plan(const clk_context *ctx, uint64_t d, uint64_t k)
+{
+    CellPlan p;
+    const uint32_t widest = d >= 16 ? 16 : d > 4 ? 8 : d > 2 ? 4 : (uint32_t)d;
+    for (uint32_t F = widest; F >= 1 && !p.F; F /= 2)
+        if (cell_lds_bytes(F, k, 1) <= ctx->lds_per_block / 2 || (F == 1 && cell_lds_bytes(1, k, 1) <= ctx->lds_per_block))
+            p.F = F;
+    switch (p.F) {
+    case 1: p.kern = cu_cell_kernel<1>; break;
+    case 2: p.kern = cu_cell_kernel<2>; break;
+    case 4: p.kern = cu_cell_kernel<4>; break;
+    case 8: p.kern = cu_cell_kernel<8>; break;
+    case 16: p.kern = cu_cell_kernel<16>; break;
+    default: return p;
+    }
+    while (p.R < 8 && p.R * k < 128 && cell_lds_bytes(p.F, k, 2 * p.R) <= ctx->lds_per_block / 2)
+        p.R *= 2;
+    p.lds = cell_lds_bytes(p.F, k, p.R);
+    return p;
 }
 
 using CmKernel = void (*)(const float *, uint64_t, uint32_t, uint32_t, const uint32_t *, GridRef, double *);
@@ -431,6 +493,18 @@ CmKernel pick_cm(int dmax, int vec, bool b256)
     }
 }
 
+const char *const kCellNames[] = {"CentroidUpdateFeatureSum", "CentroidUpdateFeatureSumPardim",
+                                  "CentroidUpdateClusterMerge"};
+
+// Whether cluster_merge's private tile beats the shared cells: only on the
+// largest data, with two work-groups per CU and enough cells (2^27 points,
+// d=4 k=10: 421 us against 433; k=16: 439 / 459; but d=4 k=3 540 / 433, d=2
+// k=10 277 / 261, and 16M points d=4 k=10 60 / 55).
+bool private_pays(const clk_context *ctx, uint64_t n, uint64_t dk, uint64_t lds)
+{
+    return n >= (64u << 20) && dk >= 32 && 2 * lds <= ctx->lds_per_block;
+}
+
 }  // namespace
 
 int run_centroid_update(clk_context *ctx, const clk_kernel_config *cfg, uint64_t d, uint64_t n,
@@ -463,8 +537,12 @@ int run_centroid_update(clk_context *ctx, const clk_kernel_config *cfg, uint64_t
     uint32_t tf = 1;
     uint64_t gx = 0;
 
-    if (strategy == CLK_CENTROID_CLUSTER_MERGE && dmax && dk < (1ull << 24) &&
-        head + dk * B * 4 <= ctx->lds_per_block) {
+    // a launch geometry of the caller's names the strategy's own kernel
+    const bool automatic = !(cfg && (cfg->global_size[0] || (cfg->local_size[0] && cfg->local_size[0] != 256)));
+    const bool private_fits = dmax && dk < (1ull << 24) && head + dk * B * 4 <= ctx->lds_per_block;
+    const CellPlan cells = cell_plan(ctx, d, k);
+    const bool take_cells = cells.kern && automatic && !(private_fits && private_pays(ctx, n, dk, head + dk * B * 4));
+    if (!take_cells && private_fits && (automatic || strategy == CLK_CENTROID_CLUSTER_MERGE)) {
         const int vec = std::min(pick_vector_width(cfg ? cfg->vector_length : 4), cm_vec_cap(dmax));
         CmKernel kc = pick_cm(dmax, vec, B == 256);
         lds = head + dk * B * 4;
@@ -482,7 +560,7 @@ int run_centroid_update(clk_context *ctx, const clk_kernel_config *cfg, uint64_t
         }
         return launch_merge_sums(ctx, ps, gx, dk, sums, stream);
     }
-    if (strategy == CLK_CENTROID_FEATURE_SUM_PARDIM) {
+    if (!take_cells && strategy == CLK_CENTROID_FEATURE_SUM_PARDIM) {
         uint64_t lf = (cfg && cfg->local_features) ? cfg->local_features : 1;
         tf = (uint32_t)((cfg && cfg->thread_features) ? cfg->thread_features : 1);
         lf = std::min<uint64_t>(lf, d);
@@ -499,9 +577,7 @@ int run_centroid_update(clk_context *ctx, const clk_kernel_config *cfg, uint64_t
             name = "CentroidUpdateFeatureSumPardim";
         }
     }
-    if (!kern && (strategy == CLK_CENTROID_FEATURE_SUM || strategy == CLK_CENTROID_CLUSTER_MERGE ||
-                  strategy == CLK_CENTROID_FEATURE_SUM_PARDIM) &&
-        dk < (1ull << 24) && head <= ctx->lds_per_block) {
+    if (!kern && !take_cells && dk < (1ull << 24) && head <= ctx->lds_per_block) {
         kern = (const void *)cu_feature_sum_kernel;
         lds = head;
         block = dim3((unsigned)B);
@@ -510,24 +586,22 @@ int run_centroid_update(clk_context *ctx, const clk_kernel_config *cfg, uint64_t
         grid = dim3((unsigned)gx);
         name = "CentroidUpdateFeatureSum";
     }
-    if (!kern && slice_lds_bytes(k) <= ctx->lds_per_block) {
-        // Large k*d: cluster-major feature slices, every strategy.
-        const size_t sl = slice_lds_bytes(k);
-        if (sl > 65536)
-            CLK_HIP_CHECK(hipFuncSetAttribute((const void *)cu_slice_kernel,
-                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)sl));
-        const uint64_t gy = div_up(d, (uint64_t)kSliceF);
-        // at least four work-groups per CU over the slices, a quarter
-        // k-th of the points per work-group (partial rows stay few)
-        uint64_t gxs = std::max<uint64_t>(div_up(n, 64 * k * kSliceWaves), div_up(4 * (uint64_t)ctx->num_cus, gy));
-        gxs = std::max<uint64_t>(1, std::min<uint64_t>(gxs, div_up(n, 64 * kSliceWaves)));
-        gxs = std::min<uint64_t>(gxs, 65535);
+    if (!kern && cells.kern) {
+        if (cells.lds > 65536)
+            CLK_HIP_CHECK(hipFuncSetAttribute((const void *)cells.kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                              (int)cells.lds));
+        // a resident grid over the slices; a work-group takes at least 4k
+        // points (it writes F*k doubles)
+        const uint64_t gy = div_up(d, (uint64_t)cells.F);
+        uint64_t gxs = auto_grid(ctx, (const void *)cells.kern, 64 * kCellWaves, cells.lds, n * gy) / gy;
+        gxs = std::min<uint64_t>(gxs, div_up(n, std::max<uint64_t>(4 * k, 64 * kCellWaves)));
+        gxs = std::max<uint64_t>(1, std::min<uint64_t>(gxs, 65535));
         CLK_TRY(ensure_scratch(ctx->part_sums, gxs * dk * sizeof(double)));
         double *ps = static_cast<double *>(ctx->part_sums.ptr);
         {
-            KernelTimer t(ctx, "CentroidUpdateSlices", stream);
-            hipLaunchKernelGGL(cu_slice_kernel, dim3((unsigned)gxs, (unsigned)gy), dim3(64 * kSliceWaves), sl,
-                               stream, points, n, (uint32_t)d, (uint32_t)k, labels, sg, ps);
+            KernelTimer t(ctx, kCellNames[strategy], stream);
+            hipLaunchKernelGGL(cells.kern, dim3((unsigned)gxs, (unsigned)gy), dim3(64 * kCellWaves), cells.lds,
+                               stream, points, n, (uint32_t)d, (uint32_t)k, labels, sg, cells.R, ps);
             CLK_HIP_CHECK(hipGetLastError());
         }
         return launch_merge_sums(ctx, ps, gxs, dk, sums, stream);
