@@ -317,8 +317,10 @@ bool split_labeling_pays(const clk_context *ctx, const clk_kernel_config *cfg, u
     // with one or two features the plain scan's 2d + 3 operations per centroid
     // stay below the ranking's.  Fused step: d=4 k=3 33 / 34, k=10 25 / 29,
     // k=50 36 / 47; d=16 k=5 61 / 50, k=10 52 / 73; d=32 k=32 88 / 190.
+    // One feature and many clusters: the gaps sink below the keys' truncation
+    // (274k points k=238: 81 / 45) and the plain scan costs 5 per centroid.
     if (fused)
-        return n >= 512 && k >= 6 && split_plan<true>(ctx, d, k).kern != nullptr;
+        return n >= 512 && k >= 6 && (d > 1 || k <= 32) && split_plan<true>(ctx, d, k).kern != nullptr;
     const uint64_t bucket = d <= 4 ? 4 : d <= 8 ? 8 : d <= 16 ? 16 : div_up(d, (uint64_t)32) * 32;
     return n >= 4096 && d >= 3 && k * (2 * bucket + 3) >= 300 + 20 * bucket &&
            split_plan<false>(ctx, d, k).kern != nullptr;
