@@ -124,6 +124,64 @@ mass_lds_kernel(const uint32_t *__restrict__ labels, uint64_t n, uint32_t k,
             PRIVATE ? lds_row_sum_u32(hist + (uint64_t)c * cols, cols, c) : hist[c];
 }
 
+// One LDS histogram [R][k] per work-group (lane mod R picks the replica:
+// fewer same-cell additions within a wave when k is small).  A wave takes
+// 1024 labels per step, sixteen per lane in four independent 128-bit loads
+// (4-byte aligned).  DIRECT: the counts go to masses with one atomic per
+// cluster and work-group; else to the work-group's partial row.
+constexpr uint32_t kHistWaves = 8;
+
+template <bool DIRECT>
+__global__ void __launch_bounds__(64 * kHistWaves)
+mass_hist_kernel(const uint32_t *__restrict__ labels, uint64_t n, uint32_t k, uint32_t R, uint32_t *__restrict__ out)
+{
+    extern __shared__ __align__(16) uint32_t hist_r[];
+    constexpr uint32_t B = 64 * kHistWaves;
+    const uint32_t tid = threadIdx.x;
+    for (uint32_t i = tid; i < R * k; i += B)
+        hist_r[i] = 0u;
+    __syncthreads();
+    uint32_t *const mine = hist_r + (tid & (R - 1)) * k;
+    const uint64_t n4 = n / 4;
+    const uint64_t stride = (uint64_t)gridDim.x * B;
+    auto count4 = [&](const gu32x4 &v) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (v[j] < k)
+                lds_add(mine + v[j], 1u);
+    };
+    const gu32x4 *l4 = reinterpret_cast<const gu32x4 *>(labels);
+    uint64_t i = (uint64_t)blockIdx.x * B + tid;
+    for (; i + 3 * stride < n4; i += 4 * stride) {
+        gu32x4 v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            v[u] = stream_load(l4 + i + u * stride);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            count4(v[u]);
+    }
+    for (; i < n4; i += stride)
+        count4(stream_load(l4 + i));
+    if (blockIdx.x == 0 && tid < n % 4) {  // the last n % 4 labels
+        const uint32_t c = labels[n4 * 4 + tid];
+        if (c < k)
+            lds_add(mine + c, 1u);
+    }
+    __syncthreads();
+    for (uint32_t c = tid; c < k; c += B) {
+        uint32_t s = 0;
+        for (uint32_t r = 0; r < R; ++r)
+            s += hist_r[r * k + c];
+        if constexpr (DIRECT) {
+            if (s)
+                atomicAdd(&out[c], s);
+        } else {
+            out[(uint64_t)blockIdx.x * k + c] = s;
+        }
+    }
+}
+
 using MassKernel = void (*)(const uint32_t *, uint64_t, uint32_t, uint32_t *);
 
 MassKernel pick_lds(int vec, bool priv)
@@ -134,6 +192,9 @@ MassKernel pick_lds(int vec, bool priv)
     return vec == 4 ? mass_lds_kernel<4, false> : vec == 2 ? mass_lds_kernel<2, false>
                                                             : mass_lds_kernel<1, false>;
 }
+
+const char *const kMassNames[] = {"MassUpdateGlobalAtomic", "MassUpdatePartGlobal", "MassUpdatePartLocal",
+                                  "MassUpdatePartPrivate"};
 
 }  // namespace
 
@@ -150,6 +211,46 @@ int run_mass_update(clk_context *ctx, const clk_kernel_config *cfg, uint64_t n, 
                 "mass_update: local_size exceeds the device limit");
     const int vec = pick_vector_width(cfg ? cfg->vector_length : 4);
     const uint64_t user_grid = (cfg && cfg->global_size[0]) ? div_up(cfg->global_size[0], B) : 0;
+
+    // An automatic launch geometry takes the histogram kernel under every
+    // strategy (the counts are exact integers): the per-label global atomics of
+    // global_atomic and part_global meet on a few addresses, at about 45 ns
+    // each (20M labels, k=36: 50 ms per call; this kernel and the merge about
+    // 35 us).
+    const bool automatic = !(cfg && (cfg->global_size[0] || (cfg->local_size[0] && cfg->local_size[0] != 256)));
+    if (automatic && strategy >= CLK_MASS_GLOBAL_ATOMIC && strategy <= CLK_MASS_PART_PRIVATE &&
+        k * 4 <= 65536) {
+        uint32_t R = 1;
+        while (R < 16 && R * k < 512)
+            R *= 2;
+        const size_t lds = (size_t)R * k * 4;
+        const char *name = kMassNames[strategy];
+        // As many work-groups as four loads per lane fill.  Up to 32 add
+        // straight into the masses (same-address atomics: 32 x 45 ns, against
+        // the merge's launch).
+        uint64_t grid = auto_grid(ctx, (const void *)mass_hist_kernel<false>, 64 * kHistWaves, lds, div_up(n, 16));
+        const bool direct = grid <= 32;
+        uint32_t *out = masses;
+        if (!direct) {
+            CLK_TRY(ensure_scratch(ctx->part_masses, grid * k * sizeof(uint32_t)));
+            out = static_cast<uint32_t *>(ctx->part_masses.ptr);
+        }
+        {
+            KernelTimer t(ctx, name, stream);
+            hipLaunchKernelGGL(direct ? mass_hist_kernel<true> : mass_hist_kernel<false>, dim3((unsigned)grid),
+                               dim3(64 * kHistWaves), lds, stream, labels, n, (uint32_t)k, R, out);
+            CLK_HIP_CHECK(hipGetLastError());
+        }
+        if (direct)
+            return CLK_OK;
+        MergeU32 m;
+        m.part = out;
+        m.rows = (uint32_t)grid;
+        m.k = k;
+        m.mass = true;
+        m.masses = masses;
+        return launch_merge(ctx, m, "ReduceVectorParcol", stream);
+    }
 
     // LDS-fit fallbacks: private -> local -> part_global.
     if (strategy == CLK_MASS_PART_PRIVATE && k * B * 4 > ctx->lds_per_block)
