@@ -138,31 +138,8 @@ split_kernel(const float *__restrict__ pts, uint64_t n, uint32_t d, uint32_t k, 
                 open = 0;
             }
         }
-        while (open) {
-            const int src = (int)__builtin_ctzll(open);
-            open &= open - 1;
-            const uint64_t ps = bt * 64 + (uint32_t)src;
-            const uint32_t r = exact_scan(cen, k, lane, [&](const float *col) {
-                float dist = 0.0f;
-                for (uint32_t f0 = 0; f0 < d; f0 += 8) {
-                    float xv[8], cv[8];  // eight features' loads at once
-#pragma unroll
-                    for (uint32_t j = 0; j < 8; ++j) {
-                        const uint32_t f = min(f0 + j, d - 1);
-                        xv[j] = pts[(uint64_t)f * n + ps];
-                        cv[j] = col[(size_t)f * k];
-                    }
-#pragma unroll
-                    for (uint32_t j = 0; j < 8; ++j)
-                        if (f0 + j < d) {
-                            const float u = xv[j] - cv[j];
-                            dist = __builtin_fmaf(u, u, dist);
-                        }
-                }
-                return dist;
-            });
-            lab = (int)lane == src ? r : lab;
-        }
+        if (open)
+            exact_scan(open, pts + bt * 64, n, cen, d, k, lane, lab);
         if (p < n)
             stream_store(lab, labels + p);
         if constexpr (FUSED) {
@@ -316,11 +293,13 @@ bool split_labeling_pays(const clk_context *ctx, const clk_kernel_config *cfg, u
     // k=16 17.8 / 20.8; d=16 k=16 31 / 39; d=32 k=10 60 / 55, k=16 55 / 65;
     // with one or two features the plain scan's 2d + 3 operations per centroid
     // stay below the ranking's.  Fused step: d=4 k=3 33 / 34, k=10 25 / 29,
-    // k=50 36 / 47; d=16 k=5 61 / 50, k=10 52 / 73; d=32 k=32 88 / 190.
+    // k=50 36 / 47; d=16 k=5 61 / 50, k=10 52 / 73; d=32 k=32 88 / 190; 300k
+    // points d=4 k=5 14 / 19, d=16 k=3 22 / 35; 20k points d=4 k=5 11 / 16.
     // One feature and many clusters: the gaps sink below the keys' truncation
     // (274k points k=238: 81 / 45) and the plain scan costs 5 per centroid.
     if (fused)
-        return n >= 512 && k >= 6 && (d > 1 || k <= 32) && split_plan<true>(ctx, d, k).kern != nullptr;
+        return (k >= 6 || (n <= (1u << 20) && k >= 2)) && (d > 1 || k <= 32) &&
+               split_plan<true>(ctx, d, k).kern != nullptr;
     const uint64_t bucket = d <= 4 ? 4 : d <= 8 ? 8 : d <= 16 ? 16 : div_up(d, (uint64_t)32) * 32;
     return n >= 4096 && d >= 3 && k * (2 * bucket + 3) >= 300 + 20 * bucket &&
            split_plan<false>(ctx, d, k).kern != nullptr;

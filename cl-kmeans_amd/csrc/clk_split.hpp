@@ -37,8 +37,7 @@
 // tr' = tr / (1 - tr),
 // makes c_b the strict, unique minimum of e_c.  Every other point -- and every
 // point with a coordinate that is not finite or too large for FP16 -- scans
-// all centroids with the reference's arithmetic, the 64 lanes of its wave
-// taking a centroid each.
+// all centroids with the reference's arithmetic.
 #pragma once
 
 #include "clk_common.hpp"
@@ -476,33 +475,70 @@ __device__ __forceinline__ bool decide(const Table &t, float x2, float best, flo
     return t.ok && x2 < 4.2e9f && best < 1e37f && ab > 1e-30f && second - best > tau && lab < k;
 }
 
-// The reference's scan of one point over all centroids, a centroid per lane
-// and round; dist_to(col) gives the point's distance to the centroid whose
-// column of cen [d][k] starts at col.
-template <typename DistTo>
-__device__ __forceinline__ uint32_t exact_scan(const float *__restrict__ cen, uint32_t k, uint32_t lane,
-                                               DistTo &&dist_to)
+// The reference's scan, over all centroids, of the wave's points whose bit is
+// set in open: 64 / G points at a time, G lanes each (8 <= G <= 64, a lane per
+// centroid while k <= G), sixteen features' loads in flight.  base: the
+// coordinate of feature 0 of the wave's point 0, the rows n apart.  lab of
+// lane i becomes the label of point i.
+__device__ __forceinline__ void exact_scan(uint64_t open, const float *__restrict__ base, uint64_t n,
+                                           const float *__restrict__ cen, uint32_t d, uint32_t k, uint32_t lane,
+                                           uint32_t &lab)
 {
-    float best = FLT_MAX;
-    uint32_t bi = 0;
-    for (uint32_t c0 = 0; c0 < k; c0 += 64) {
-        const uint32_t c = c0 + lane;
-        const float dist = dist_to(cen + min(c, k - 1));
-        if (c < k && dist < best) {
-            best = dist;
-            bi = c;
+    uint32_t G = 8;
+    while (G < k && G < 64)
+        G *= 2;
+    while (open) {
+        uint64_t rest = open;
+        uint32_t src = 0;  // this lane's point
+        for (uint32_t i = 0; i < 64 / G && rest; ++i) {
+            const uint32_t bit = (uint32_t)__builtin_ctzll(rest);
+            rest &= rest - 1;
+            src = lane / G >= i ? bit : src;  // groups past the last point repeat it
+        }
+        const float *x = base + src;
+        float best = FLT_MAX;
+        uint32_t bi = 0;
+        for (uint32_t c0 = 0; c0 < k; c0 += G) {
+            const uint32_t c = c0 + lane % G;
+            const float *col = cen + min(c, k - 1);
+            float dist = 0.0f;
+            for (uint32_t f0 = 0; f0 < d; f0 += 16) {
+                float xv[16], cv[16];
+#pragma unroll
+                for (uint32_t j = 0; j < 16; ++j) {
+                    const uint32_t f = min(f0 + j, d - 1);
+                    xv[j] = x[(uint64_t)f * n];
+                    cv[j] = col[(size_t)f * k];
+                }
+#pragma unroll
+                for (uint32_t j = 0; j < 16; ++j)
+                    if (f0 + j < d) {
+                        const float u = xv[j] - cv[j];
+                        dist = __builtin_fmaf(u, u, dist);
+                    }
+            }
+            if (c < k && dist < best) {
+                best = dist;
+                bi = c;
+            }
+        }
+        // smallest distance, lowest index on equal distances; none below
+        // FLT_MAX gives label 0
+        uint32_t hi = __float_as_uint(best);
+        for (uint32_t o = G / 2; o >= 1; o /= 2) {
+            const uint32_t h2 = (uint32_t)__shfl_xor((int)hi, (int)o), i2 = (uint32_t)__shfl_xor((int)bi, (int)o);
+            const bool take = h2 < hi || (h2 == hi && i2 < bi);
+            hi = take ? h2 : hi;
+            bi = take ? i2 : bi;
+        }
+        const uint32_t found = hi < __float_as_uint(FLT_MAX) ? bi : 0u;
+        for (uint32_t i = 0; i < 64 / G && open; ++i) {
+            const uint32_t bit = (uint32_t)__builtin_ctzll(open);
+            open &= open - 1;
+            const uint32_t r = (uint32_t)__builtin_amdgcn_readlane((int)found, (int)(i * G));
+            lab = lane == bit ? r : lab;
         }
     }
-    // smallest distance, lowest index on equal distances; none below FLT_MAX
-    // gives label 0
-    uint32_t hi = __float_as_uint(best);
-    for (int o = 32; o >= 1; o /= 2) {
-        const uint32_t h2 = (uint32_t)__shfl_xor((int)hi, o), i2 = (uint32_t)__shfl_xor((int)bi, o);
-        const bool take = h2 < hi || (h2 == hi && i2 < bi);
-        hi = take ? h2 : hi;
-        bi = take ? i2 : bi;
-    }
-    return hi < __float_as_uint(FLT_MAX) ? bi : 0u;
 }
 
 }  // namespace split
