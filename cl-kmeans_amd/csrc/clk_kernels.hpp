@@ -33,7 +33,7 @@ int launch_labeling(clk_context *ctx, const clk_kernel_config *cfg, uint64_t d, 
 // pass writes `rows` partial rows [d + 1][k] to part.
 bool split_labeling_pays(const clk_context *ctx, const clk_kernel_config *cfg, uint64_t d, uint64_t n, uint64_t k,
                          bool fused);
-int launch_labeling_split(clk_context *ctx, uint64_t d, uint64_t n, uint64_t k, const float *points,
+int launch_labeling_split(clk_context *ctx, const char *name, uint64_t d, uint64_t n, uint64_t k, const float *points,
                           const float *centroids, uint32_t *labels, hipStream_t stream);
 struct GridRef;
 uint64_t fused_split_rows(clk_context *ctx, uint64_t d, uint64_t n, uint64_t k);

@@ -295,8 +295,14 @@ int launch_labeling(clk_context *ctx, const clk_kernel_config *cfg, uint64_t d, 
     const uint64_t B = (cfg && cfg->local_size[0]) ? cfg->local_size[0] : 256;
     CLK_REQUIRE(B <= (uint64_t)ctx->max_threads_per_block, CLK_ERR_INVALID_ARGUMENT,
                 "labeling: local_size exceeds the device limit");
-    if (!bounded && split_labeling_pays(ctx, cfg, d, n, k, false))
-        return launch_labeling_split(ctx, d, n, k, points, centroids, labels, stream);
+    // Split-operand labels for the bounded variant too: the keep test spares
+    // the scan only where no point of a wave fails it, and its thresholds cost
+    // k^2 d in every work-group (settled labels, 1M points: d=4 k=64 25 us
+    // against 16, d=16 k=40 44 / 25, d=32 k=100 287 / 50; 941k d=6 k=421
+    // 654 / 80).
+    if (split_labeling_pays(ctx, cfg, d, n, k, false))
+        return launch_labeling_split(ctx, bounded ? "LabelingUnrollVectorBounded" : "LabelingUnrollVector", d, n, k,
+                                     points, centroids, labels, stream);
     const int dmax = dmax_bucket(d);
     const uint64_t cen_plain = dmax ? ((k * dmax + 3) & ~3ull) * 4 : 0;
     // the bounded variant adds k keep thresholds; beyond LDS it runs as the

@@ -304,15 +304,17 @@ bool split_labeling_pays(const clk_context *ctx, const clk_kernel_config *cfg, u
     return n >= 4096 && d >= 3 && k * (2 * bucket + 3) >= 300 + 20 * bucket &&
            split_plan<false>(ctx, d, k).kern != nullptr;
 }
-int launch_labeling_split(clk_context *ctx, uint64_t d, uint64_t n, uint64_t k, const float *points,
+
+int launch_labeling_split(clk_context *ctx, const char *name, uint64_t d, uint64_t n, uint64_t k, const float *points,
                           const float *centroids, uint32_t *labels, hipStream_t stream)
 {
     const SplitPlan p = split_plan<false>(ctx, d, k);
     CLK_REQUIRE(p.kern && n > 0, CLK_ERR_UNSUPPORTED, "split labeling: sizes");
     CLK_TRY(allow_lds(p));
-    KernelTimer t(ctx, "LabelingUnrollVector", stream);
+    KernelTimer t(ctx, name, stream);
     hipLaunchKernelGGL(p.kern, dim3((unsigned)split_grid(ctx, p, n)), dim3(p.block), p.lds, stream, points, n,
-                       (uint32_t)d, (uint32_t)k, centroids, labels, p.ntiles, GridRef{}, 1u, nullptr, nullptr);
+                       (uint32_t)d, (uint32_t)k, centroids, labels, p.ntiles, GridRef{}, 1u,
+                       nullptr, nullptr);
     CLK_HIP_CHECK(hipGetLastError());
     return CLK_OK;
 }
