@@ -78,6 +78,12 @@ struct clk_context {
     char *noalloc_scratch = nullptr;  // this device's static scratch (clk_lloyd_step_noalloc)
     uint64_t grid_d = 0, grid_n = 0;
     const void *grid_src = nullptr;  // the points a grid was pinned from (null: from maxima)
+    struct Occupancy {
+        const void *kernel;
+        int block, per_cu;
+        size_t lds;
+    };
+    std::vector<Occupancy> occupancies;  // auto_grid's answers: the query costs more than a launch
     int mfma_subnormals = -1;     // bit 0 FP16, bit 1 BF16: MFMA keeps subnormal inputs (-1 unknown)
     bool profiling = false;
     int32_t iteration = -1;

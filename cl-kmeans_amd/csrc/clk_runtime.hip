@@ -85,10 +85,18 @@ uint64_t auto_grid(clk_context *ctx, const void *kernel, int block, size_t dyn_l
                    uint64_t work_items)
 {
     int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, block, dyn_lds) !=
-            hipSuccess ||
-        per_cu < 1)
-        per_cu = 1;
+    for (const clk_context::Occupancy &o : ctx->occupancies)
+        if (o.kernel == kernel && o.block == block && o.lds == dyn_lds)
+            per_cu = o.per_cu;
+    if (per_cu == 0) {
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, block, dyn_lds) !=
+                hipSuccess ||
+            per_cu < 1)
+            per_cu = 1;
+        if (ctx->occupancies.size() >= 64)  // sizes that keep changing
+            ctx->occupancies.clear();
+        ctx->occupancies.push_back({kernel, block, per_cu, dyn_lds});
+    }
     uint64_t grid = (uint64_t)per_cu * (uint64_t)ctx->num_cus;
     uint64_t need = div_up(std::max<uint64_t>(work_items, 1), (uint64_t)block);
     return std::max<uint64_t>(1, std::min(grid, need));

@@ -11,6 +11,7 @@
 #include <memory>
 #include <stdexcept>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "clkmeans.h"
@@ -48,6 +49,13 @@ public:
         check_hip(hipEventCreate(&h), "hipEventCreate");
         e.h_ = std::shared_ptr<ihipEvent_t>(h, [](hipEvent_t x) { (void)hipEventDestroy(x); });
         check_hip(hipEventRecord(h, stream), "hipEventRecord");
+        return e;
+    }
+    // The event of an operator that records one at its end anyway (its timing).
+    static Event share(std::shared_ptr<ihipEvent_t> h)
+    {
+        Event e;
+        e.h_ = std::move(h);
         return e;
     }
     bool valid() const { return (bool)h_; }

@@ -15,10 +15,10 @@ const char *const kExperimentSuffix = "_expm";
 const char *const kMeasurementsSuffix = "_mnts";
 const char *const kEventsSuffix = "_evnt";
 
-std::shared_ptr<ihipEvent_t> make_event()
+std::shared_ptr<ihipEvent_t> make_event(unsigned flags)
 {
     hipEvent_t e;
-    if (hipEventCreate(&e) != hipSuccess)
+    if (hipEventCreateWithFlags(&e, flags) != hipSuccess)
         throw std::runtime_error("hipEventCreate failed");
     return std::shared_ptr<ihipEvent_t>(e, [](hipEvent_t x) { (void)hipEventDestroy(x); });
 }
@@ -36,14 +36,15 @@ uint64_t elapsed_ns(hipEvent_t a, hipEvent_t b)
 TimedEvent TimedEvent::begin(hipStream_t s)
 {
     TimedEvent t;
-    t.start = make_event();
+    // only its time is read: no write-back of the caches to the host
+    t.start = make_event(hipEventDisableSystemFence);
     (void)hipEventRecord(t.start.get(), s);
     return t;
 }
 
 void TimedEvent::finish(hipStream_t s)
 {
-    end = make_event();
+    end = make_event(hipEventDefault);
     (void)hipEventRecord(end.get(), s);
 }
 

@@ -140,7 +140,7 @@ Event timed_enqueue(const Queue &q, Measurement::DataPoint &dp, const WaitList &
     te = Measurement::TimedEvent::begin(q.get());
     fn(q.get());
     te.finish(q.get());
-    return Event::record(q.get());
+    return Event::share(te.end);
 }
 
 template <typename T>
