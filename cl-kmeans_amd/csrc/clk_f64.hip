@@ -19,6 +19,9 @@
 // Where the tile does not fit, the pass adds straight into the caller's
 // buffers with global FP64 / uint64 atomics (order not fixed).  Labels are
 // bit-exact either way; sums differ from a serial sum only by FP64 rounding.
+// Where the scan's operations bound the pass, labels come from split-operand
+// MFMA scores (clk_split.hpp): 200k points d=20 k=64 labeling 58 -> 19 us, 5M
+// d=4 k=10 fused 58 -> 43 us.
 #include "clk_common.hpp"
 #include "clk_finalize.hpp"
 #include "clk_kernels.hpp"
@@ -265,6 +268,27 @@ struct StepOut {
     double *max_shift;
 };
 
+// The partial rows of a pass into sums / masses, and with step the divide.
+int merge_f64(clk_context *ctx, const double *part, uint64_t rows, uint64_t d, uint64_t k, bool mass, double *sums,
+              uint64_t *masses, const double *old_centroids, const StepOut *step, hipStream_t stream)
+{
+    MergeF64 m;
+    m.part = part;
+    m.rows = (uint32_t)rows;
+    m.mass = mass;
+    m.d = mass ? (uint32_t)d : 1;
+    m.k = mass ? k : d * k;  // sums alone: one row of d*k values
+    m.sums = sums;
+    m.masses = masses;
+    if (step) {
+        m.divide = true;
+        m.centroids = step->centroids;
+        m.old_centroids = old_centroids;
+        m.max_shift = step->max_shift;
+    }
+    return launch_merge(ctx, m, step ? "FinalizeDivide" : "ReduceVectorParcol", stream);
+}
+
 // One pass: labels (LABEL) and/or accumulation into sums / masses.  With
 // `step` (a fused pass whose tile fits) sums and masses are overwritten and
 // the centroids divided in the same two launches.
@@ -295,6 +319,16 @@ int run_f64_pass(clk_context *ctx, const clk_kernel_config *cfg, bool label, boo
         default: break;
         }
     }
+    const uint64_t split = label ? split_rows_f64(ctx, cfg, d, n, k, want_sums) : 0;
+    if (split && !want_sums)
+        return launch_split_f64(ctx, name, d, n, k, points, centroids, labels, split, nullptr, nullptr, stream);
+    if (split && tile) {
+        CLK_TRY(ensure_scratch(ctx->part_sums, split * (d + 1) * k * sizeof(double)));
+        double *part = static_cast<double *>(ctx->part_sums.ptr);
+        CLK_TRY(launch_split_f64(ctx, name, d, n, k, points, centroids, labels, split, part,
+                                 step ? step->max_shift : nullptr, stream));
+        return merge_f64(ctx, part, split, d, k, true, sums, masses, centroids, step, stream);
+    }
     const size_t lds = tile ? (size_t)(cen_bytes + tile_bytes) : (size_t)cen_bytes;
     const uint64_t need = div_up(n, (uint64_t)B);
     uint64_t grid = (cfg && cfg->global_size[0]) ? div_up(cfg->global_size[0], (uint64_t)B)
@@ -317,26 +351,7 @@ int run_f64_pass(clk_context *ctx, const clk_kernel_config *cfg, bool label, boo
         }
         if (!part)
             return CLK_OK;
-        MergeF64 m;
-        m.part = part;
-        m.rows = (uint32_t)grid;
-        m.mass = want_mass;
-        if (want_mass) {
-            m.d = want_sums ? (uint32_t)d : 0;
-            m.k = k;
-        } else {  // sums alone: one row of d*k values
-            m.d = 1;
-            m.k = d * k;
-        }
-        m.sums = sums;
-        m.masses = masses;
-        if (step) {
-            m.divide = true;
-            m.centroids = step->centroids;
-            m.old_centroids = centroids;
-            m.max_shift = step->max_shift;
-        }
-        return launch_merge(ctx, m, step ? "FinalizeDivide" : "ReduceVectorParcol", stream);
+        return merge_f64(ctx, part, grid, want_sums ? d : 0, k, want_mass, sums, masses, centroids, step, stream);
     }
     KernelTimer t(ctx, name, stream);
     // beyond the register buckets or the LDS: global memory and atomics

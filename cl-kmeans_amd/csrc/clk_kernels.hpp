@@ -41,6 +41,14 @@ int launch_fused_split(clk_context *ctx, const char *name, uint64_t d, uint64_t 
                        const float *centroids, uint32_t *labels, const GridRef &grid, uint64_t rows, double *part,
                        double *max_shift, hipStream_t stream);
 
+// The same for double points: the number of work-groups (partial rows) of the
+// labeling or fused pass, 0 where it is not taken; part: non-null for the
+// fused pass.
+uint64_t split_rows_f64(clk_context *ctx, const clk_kernel_config *cfg, uint64_t d, uint64_t n, uint64_t k, bool fused);
+int launch_split_f64(clk_context *ctx, const char *name, uint64_t d, uint64_t n, uint64_t k, const double *points,
+                     const double *centroids, uint64_t *labels, uint64_t rows, double *part, double *max_shift,
+                     hipStream_t stream);
+
 // Labels from x·cᵀ on MFMA (16-bit operands, FP32 accumulation) with an exact
 // FP32 relabel of near ties: the same labels as launch_labeling.  Supported
 // for d <= 128 and n < 2^32 when the 16-bit centroid table fits in LDS.

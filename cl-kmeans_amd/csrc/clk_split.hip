@@ -14,6 +14,7 @@
 #include "clk_split.hpp"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace clk {
 namespace {
@@ -24,27 +25,30 @@ using namespace split;
 // registers.
 constexpr uint32_t split_waves(int P) { return P >= 96 ? 4 : 8; }
 
-// LDS words after the table of a fused pass: scales [P] | acc [R][d*k] int64
-// | flags [d*k] | counts [R][k].  R replicas (lane mod R) thin out the
-// same-cell atomics of a wave.
-__host__ __device__ inline size_t fused_tail_bytes(uint32_t P, uint32_t d, uint32_t k, uint32_t R)
+// LDS after the table of a fused pass: scales [P] | cells [R][d*k] | flags
+// [d*k] | counts [R][k].  Float points: int64 cells of grid integers
+// (clk_grid.hpp); double points: FP64 cells, no scales or flags.  R replicas
+// (lane mod R) thin out the same-cell atomics of a wave.
+__host__ __device__ inline size_t fused_tail_bytes(uint32_t P, uint32_t d, uint32_t k, uint32_t R, bool f64)
 {
-    return (size_t)P * 4 + (size_t)R * d * k * 8 + (size_t)d * k * 4 + (size_t)R * k * 4 + 16;
+    return (f64 ? 0 : (size_t)P * 4 + (size_t)d * k * 4) + (size_t)R * d * k * 8 + (size_t)R * k * 4 + 16;
 }
 
-// FUSED: labels, masses and grid-exact sums (clk_grid.hpp) in one pass, the
-// work-group's partial row to part (clk_finalize.hpp); else labels only.
+// FUSED: labels, masses and sums in one pass, the work-group's partial row to
+// part (clk_finalize.hpp); else labels only.
 // A wave takes 64 consecutive points per step.  P <= 16: lane = point, the
 // next step's coordinates loaded while this step is labelled.  P >= 32: lane
 // (q, h) holds features 8h .. 8h+7 of each K-block of the points q, 16+q,
 // 32+q, 48+q (the matrix core's layout).
-template <int P, bool FUSED>
+template <int P, bool FUSED, typename T, typename LabelT>
 __global__ void __launch_bounds__(64 * split_waves(P))
-split_kernel(const float *__restrict__ pts, uint64_t n, uint32_t d, uint32_t k, const float *__restrict__ cen,
-             uint32_t *__restrict__ labels, uint32_t ntiles, GridRef grid, uint32_t R, double *__restrict__ part,
+split_kernel(const T *__restrict__ pts, uint64_t n, uint32_t d, uint32_t k, const T *__restrict__ cen,
+             LabelT *__restrict__ labels, uint32_t ntiles, GridRef grid, uint32_t R, double *__restrict__ part,
              double *__restrict__ max_shift)
 {
     using Sh = Shape<P>;
+    constexpr bool f64 = sizeof(T) == 8;
+    using Cell = std::conditional_t<f64, double, long long>;
     constexpr uint32_t kWaves = split_waves(P);
     extern __shared__ __align__(16) char smem_split[];
     const uint32_t tid = threadIdx.x, lane = tid % 64, B = 64 * kWaves;
@@ -52,31 +56,34 @@ split_kernel(const float *__restrict__ pts, uint64_t n, uint32_t d, uint32_t k, 
     const uint32_t q = lane % 16, h = lane / 16;
     const uint32_t dk = d * k;
     // the exchange planes end the table's block; the fused tail follows
-    u16x8 *buf = reinterpret_cast<u16x8 *>(smem_split + lds_bytes<P>(ntiles, 0)) + wave * Sh::planes * 64;
-    char *tail = smem_split + lds_bytes<P>(ntiles, kWaves);
+    u16x8 *buf = reinterpret_cast<u16x8 *>(smem_split + lds_bytes<P, T>(ntiles, 0)) + wave * Sh::planes * 64;
+    char *tail = smem_split + lds_bytes<P, T>(ntiles, kWaves);
     float *scl = reinterpret_cast<float *>(tail);
-    long long *acc = reinterpret_cast<long long *>(scl + P);
+    Cell *acc = reinterpret_cast<Cell *>(scl + (f64 ? 0 : P));
     uint32_t *flg = reinterpret_cast<uint32_t *>(acc + (size_t)R * dk);
-    uint32_t *cnt = flg + dk;
+    uint32_t *cnt = flg + (f64 ? 0 : dk);
     if constexpr (FUSED) {
         if (max_shift && blockIdx.x == 0 && tid == 0)
             *max_shift = 0.0;  // the merge raises it
-        for (uint32_t f = tid; f < P; f += B)
-            scl[f] = f < d ? grid_scale(grid.gmax[f], grid.bits) : 1.0f;
         for (uint32_t i = tid; i < R * dk; i += B)
             acc[i] = 0;
-        for (uint32_t i = tid; i < dk; i += B)
-            flg[i] = 0u;
+        if constexpr (!f64) {
+            for (uint32_t f = tid; f < P; f += B)
+                scl[f] = f < d ? grid_scale(grid.gmax[f], grid.bits) : 1.0f;
+            for (uint32_t i = tid; i < dk; i += B)
+                flg[i] = 0u;
+        }
         for (uint32_t i = tid; i < R * k; i += B)
             cnt[i] = 0u;
     }
-    const Table t = stage<P>(cen, d, k, ntiles, smem_split);
-    const bool on_grid = FUSED && grid.own != 0 && grid.gmax[d] == 0;
+    const Table<T> t = stage<P, T>(cen, d, k, ntiles, smem_split);
+    const bool on_grid = FUSED && !f64 && grid.own != 0 && grid.gmax[d] == 0;
 
     constexpr int kOwn = P < 32 ? P : Sh::nkb * 8;  // coordinates per lane and point
     constexpr int kPts = P < 32 ? 1 : 4;            // points a lane holds parts of
-    float sc[FUSED ? kOwn : 1];
-    if constexpr (FUSED) {
+    constexpr bool kScales = FUSED && !f64;
+    float sc[kScales ? kOwn : 1];
+    if constexpr (kScales) {
 #pragma unroll
         for (int i = 0; i < kOwn; ++i) {
             sc[i] = scl[P < 32 ? i : (i / 8) * 32 + 8 * h + i % 8];
@@ -95,8 +102,8 @@ split_kernel(const float *__restrict__ pts, uint64_t n, uint32_t d, uint32_t k, 
 #pragma unroll
         for (int i = 0; i < kOwn; ++i)
             rows[i] = min(feature(i), d - 1) * (uint32_t)n;  // n * d <= 2^30
-    auto load = [&](uint64_t bt, float (&x)[kPts][kOwn]) {
-        const float *base = pts + bt * 64;                              // wave-uniform
+    auto load = [&](uint64_t bt, T (&x)[kPts][kOwn]) {
+        const T *base = pts + bt * 64;                              // wave-uniform
         const uint64_t left = n - 1 - bt * 64;
         const uint32_t last = left < 63 ? (uint32_t)left : 63u;
 #pragma unroll
@@ -111,15 +118,15 @@ split_kernel(const float *__restrict__ pts, uint64_t n, uint32_t d, uint32_t k, 
             }
         }
     };
-    auto step = [&](uint64_t bt, const float (&x)[kPts][kOwn]) {
+    auto step = [&](uint64_t bt, const T (&x)[kPts][kOwn]) {
         const uint64_t p = bt * 64 + lane;
         PointOps<P> ops;
         float x2, best, second;
         if constexpr (P < 32)
-            x2 = build_points<P>(x[0], t.scale, buf, lane, ops);
+            x2 = build_points<P, T>(x[0], t.scale, buf, lane, ops);
         else
-            x2 = build_points<P>(x, t.scale, lane, ops);
-        rank_points<P>(t, ops, lane, best, second);
+            x2 = build_points<P, T>(x, t.scale, lane, ops);
+        rank_points<P, T>(t, ops, lane, best, second);
         uint32_t lab;
         const bool sure = decide(t, x2, best, second, k, lab);
         uint64_t open = __ballot(!sure && p < n);
@@ -128,29 +135,31 @@ split_kernel(const float *__restrict__ pts, uint64_t n, uint32_t d, uint32_t k, 
             // for its own point (about k (2P + 3) instructions in all, against
             // about 150 for each point that the wave scans together).
             if (open && k * (2 * P + 3) <= 150u * (uint32_t)__builtin_popcountll(open)) {
-                float own[P][1];
-#pragma unroll
-                for (int f = 0; f < P; ++f)
-                    own[f][0] = f < (int)d ? x[0][f] : 0.0f;
-                uint32_t scanned[1];
-                argmin_lds<P, 1>(own, t.rows, k, scanned);
-                lab = sure ? lab : scanned[0];
+                const uint32_t scanned = scan_rows<P, T>(t, x[0], d, k);
+                lab = sure ? lab : scanned;
                 open = 0;
             }
         }
         if (open)
             exact_scan(open, pts + bt * 64, n, cen, d, k, lane, lab);
         if (p < n)
-            stream_store(lab, labels + p);
+            stream_store((LabelT)lab, labels + p);
         if constexpr (FUSED) {
-            long long *const mine = acc + (size_t)(lane & (R - 1)) * dk;
+            Cell *const mine = acc + (size_t)(lane & (R - 1)) * dk;
             if (p < n)
                 lds_add(cnt + (lane & (R - 1)) * k + lab, 1u);
 #pragma unroll
             for (int g = 0; g < kPts; ++g) {
                 const uint32_t lg = P < 32 ? lab : (uint32_t)__shfl((int)lab, (int)(g * 16 + q));
                 const bool in = bt * 64 + (P < 32 ? lane : g * 16 + q) < n;
-                if (on_grid) {
+                if constexpr (f64) {
+                    if (in) {
+#pragma unroll
+                        for (int i = 0; i < kOwn; ++i)
+                            if (feature(i) < d)
+                                atomicAdd(mine + feature(i) * k + lg, x[g][i]);
+                    }
+                } else if (on_grid) {
                     if (in) {
 #pragma unroll
                         for (int i = 0; i < kOwn; ++i)
@@ -174,9 +183,9 @@ split_kernel(const float *__restrict__ pts, uint64_t n, uint32_t d, uint32_t k, 
     const uint64_t batches = (n + 63) / 64;
     const uint64_t stride = (uint64_t)gridDim.x * kWaves;
     uint64_t bt = (uint64_t)blockIdx.x * kWaves + wave;
-    if constexpr (P <= 32) {
+    if constexpr (P <= 32 && !(f64 && FUSED && P == 32)) {
         // two register buffers: the next step's loads are in flight
-        float xa[kPts][kOwn], xb[kPts][kOwn];
+        T xa[kPts][kOwn], xb[kPts][kOwn];
         load(bt < batches ? bt : batches - 1, xa);
         while (bt < batches) {
             const uint64_t b1 = bt + stride;
@@ -190,7 +199,7 @@ split_kernel(const float *__restrict__ pts, uint64_t n, uint32_t d, uint32_t k, 
         }
     } else {
         for (; bt < batches; bt += stride) {
-            float x[kPts][kOwn];
+            T x[kPts][kOwn];
             load(bt, x);
             step(bt, x);
         }
@@ -199,10 +208,13 @@ split_kernel(const float *__restrict__ pts, uint64_t n, uint32_t d, uint32_t k, 
         __syncthreads();
         double *const row = part + (uint64_t)blockIdx.x * (dk + k);
         for (uint32_t i = tid; i < dk; i += B) {
-            long long s = 0;
+            Cell s = 0;
             for (uint32_t r = 0; r < R; ++r)
                 s += acc[(size_t)r * dk + i];
-            row[i] = cell_value(s, grid_unit(scl[i / k]), flg[i]);
+            if constexpr (f64)
+                row[i] = s;
+            else
+                row[i] = cell_value(s, grid_unit(scl[i / k]), flg[i]);
         }
         for (uint32_t c = tid; c < k; c += B) {
             uint32_t s = 0;
@@ -213,68 +225,88 @@ split_kernel(const float *__restrict__ pts, uint64_t n, uint32_t d, uint32_t k, 
     }
 }
 
-using SplitKernel = void (*)(const float *, uint64_t, uint32_t, uint32_t, const float *, uint32_t *, uint32_t, GridRef,
-                             uint32_t, double *, double *);
+template <typename T>
+using LabelOf = std::conditional_t<sizeof(T) == 8, uint64_t, uint32_t>;
+template <typename T>
+using SplitKernel = void (*)(const T *, uint64_t, uint32_t, uint32_t, const T *, LabelOf<T> *, uint32_t, GridRef, uint32_t,
+                             double *, double *);
 
+template <typename T>
 struct SplitPlan {
-    SplitKernel kern = nullptr;
+    SplitKernel<T> kern = nullptr;
     uint32_t block = 0;
     uint32_t ntiles = 0, R = 1;
     size_t lds = 0;
 };
 
-template <int P, bool FUSED>
-SplitPlan plan_for(const clk_context *ctx, uint64_t d, uint64_t k)
+template <int P, bool FUSED, typename T>
+SplitPlan<T> plan_for(const clk_context *ctx, uint64_t d, uint64_t k)
 {
-    SplitPlan p;
+    constexpr bool f64 = sizeof(T) == 8;
+    SplitPlan<T> p;
     p.ntiles = (uint32_t)div_up(k, (uint64_t)16);
     p.block = 64 * split_waves(P);
-    p.lds = lds_bytes<P>(p.ntiles, split_waves(P));
+    p.lds = lds_bytes<P, T>(p.ntiles, split_waves(P));
     if (FUSED) {
         // replicas only where they leave the CU its second work-group
         p.R = P < 32 ? 4 : 1;
-        while (p.R > 1 && p.lds + fused_tail_bytes(P, (uint32_t)d, (uint32_t)k, p.R) > ctx->lds_per_block / 2)
+        while (p.R > 1 && p.lds + fused_tail_bytes(P, (uint32_t)d, (uint32_t)k, p.R, f64) > ctx->lds_per_block / 2)
             p.R /= 2;
-        p.lds += fused_tail_bytes(P, (uint32_t)d, (uint32_t)k, p.R);
+        p.lds += fused_tail_bytes(P, (uint32_t)d, (uint32_t)k, p.R, f64);
     }
     if (p.lds <= ctx->lds_per_block)
-        p.kern = split_kernel<P, FUSED>;
+        p.kern = split_kernel<P, FUSED, T, LabelOf<T>>;
     return p;
 }
 
-template <bool FUSED>
-SplitPlan split_plan(const clk_context *ctx, uint64_t d, uint64_t k)
+template <bool FUSED, typename T>
+SplitPlan<T> split_plan(const clk_context *ctx, uint64_t d, uint64_t k)
 {
     if (d == 0 || k == 0 || k > 65536)
         return {};
     if (d <= 4)
-        return plan_for<4, FUSED>(ctx, d, k);
+        return plan_for<4, FUSED, T>(ctx, d, k);
     if (d <= 8)
-        return plan_for<8, FUSED>(ctx, d, k);
+        return plan_for<8, FUSED, T>(ctx, d, k);
     if (d <= 16)
-        return plan_for<16, FUSED>(ctx, d, k);
+        return plan_for<16, FUSED, T>(ctx, d, k);
     if (d <= 32)
-        return plan_for<32, FUSED>(ctx, d, k);
+        return plan_for<32, FUSED, T>(ctx, d, k);
     if constexpr (!FUSED) {
         if (d <= 64)
-            return plan_for<64, FUSED>(ctx, d, k);
+            return plan_for<64, FUSED, T>(ctx, d, k);
         if (d <= 96)
-            return plan_for<96, FUSED>(ctx, d, k);
+            return plan_for<96, FUSED, T>(ctx, d, k);
         if (d <= 128)
-            return plan_for<128, FUSED>(ctx, d, k);
+            return plan_for<128, FUSED, T>(ctx, d, k);
     }
     return {};
 }
 
-uint64_t split_grid(clk_context *ctx, const SplitPlan &p, uint64_t n)
+// Padded features of the plans.
+uint64_t split_bucket(uint64_t d)
+{
+    return d <= 4 ? 4 : d <= 8 ? 8 : d <= 16 ? 16 : div_up(d, (uint64_t)32) * 32;
+}
+
+template <typename T>
+uint64_t split_grid(clk_context *ctx, const SplitPlan<T> &p, uint64_t n)
 {
     return auto_grid(ctx, (const void *)p.kern, (int)p.block, p.lds, n);
 }
 
-int allow_lds(const SplitPlan &p)
+template <typename T>
+int launch_split(clk_context *ctx, const SplitPlan<T> &p, const char *name, uint64_t grid, uint64_t d, uint64_t n,
+                 uint64_t k, const T *points, const T *centroids, LabelOf<T> *labels, const GridRef &sgrid,
+                 double *part, double *max_shift, hipStream_t stream)
 {
+    CLK_REQUIRE(p.kern && n > 0, CLK_ERR_UNSUPPORTED, "split labels: sizes");
     if (p.lds > 65536)
         CLK_HIP_CHECK(hipFuncSetAttribute((const void *)p.kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)p.lds));
+    KernelTimer t(ctx, name, stream);
+    hipLaunchKernelGGL(p.kern, dim3((unsigned)grid), dim3(p.block), p.lds, stream, points, n, (uint32_t)d, (uint32_t)k,
+                       centroids, labels, p.ntiles, sgrid, p.R, part, max_shift);
+    CLK_HIP_CHECK(hipGetLastError());
     return CLK_OK;
 }
 
@@ -299,43 +331,69 @@ bool split_labeling_pays(const clk_context *ctx, const clk_kernel_config *cfg, u
     // (274k points k=238: 81 / 45) and the plain scan costs 5 per centroid.
     if (fused)
         return (k >= 6 || (n <= (1u << 20) && k >= 2)) && (d > 1 || k <= 32) &&
-               split_plan<true>(ctx, d, k).kern != nullptr;
-    const uint64_t bucket = d <= 4 ? 4 : d <= 8 ? 8 : d <= 16 ? 16 : div_up(d, (uint64_t)32) * 32;
+               split_plan<true, float>(ctx, d, k).kern != nullptr;
+    const uint64_t bucket = split_bucket(d);
     return n >= 4096 && d >= 3 && k * (2 * bucket + 3) >= 300 + 20 * bucket &&
-           split_plan<false>(ctx, d, k).kern != nullptr;
+           split_plan<false, float>(ctx, d, k).kern != nullptr;
 }
 
 int launch_labeling_split(clk_context *ctx, const char *name, uint64_t d, uint64_t n, uint64_t k, const float *points,
                           const float *centroids, uint32_t *labels, hipStream_t stream)
 {
-    const SplitPlan p = split_plan<false>(ctx, d, k);
-    CLK_REQUIRE(p.kern && n > 0, CLK_ERR_UNSUPPORTED, "split labeling: sizes");
-    CLK_TRY(allow_lds(p));
-    KernelTimer t(ctx, name, stream);
-    hipLaunchKernelGGL(p.kern, dim3((unsigned)split_grid(ctx, p, n)), dim3(p.block), p.lds, stream, points, n,
-                       (uint32_t)d, (uint32_t)k, centroids, labels, p.ntiles, GridRef{}, 1u,
-                       nullptr, nullptr);
-    CLK_HIP_CHECK(hipGetLastError());
-    return CLK_OK;
+    const SplitPlan<float> p = split_plan<false, float>(ctx, d, k);
+    return launch_split(ctx, p, name, p.kern ? split_grid(ctx, p, n) : 0, d, n, k, points, centroids, labels, GridRef{},
+                        nullptr, nullptr, stream);
 }
 
 uint64_t fused_split_rows(clk_context *ctx, uint64_t d, uint64_t n, uint64_t k)
 {
-    return split_grid(ctx, split_plan<true>(ctx, d, k), n);
+    return split_grid(ctx, split_plan<true, float>(ctx, d, k), n);
 }
 
 int launch_fused_split(clk_context *ctx, const char *name, uint64_t d, uint64_t n, uint64_t k, const float *points,
                        const float *centroids, uint32_t *labels, const GridRef &grid, uint64_t rows, double *part,
                        double *max_shift, hipStream_t stream)
 {
-    const SplitPlan p = split_plan<true>(ctx, d, k);
-    CLK_REQUIRE(p.kern && n > 0, CLK_ERR_UNSUPPORTED, "split fused pass: sizes");
-    CLK_TRY(allow_lds(p));
-    KernelTimer t(ctx, name, stream);
-    hipLaunchKernelGGL(p.kern, dim3((unsigned)rows), dim3(p.block), p.lds, stream, points, n, (uint32_t)d,
-                       (uint32_t)k, centroids, labels, p.ntiles, grid, p.R, part, max_shift);
-    CLK_HIP_CHECK(hipGetLastError());
-    return CLK_OK;
+    return launch_split(ctx, split_plan<true, float>(ctx, d, k), name, rows, d, n, k, points, centroids, labels, grid,
+                        part, max_shift, stream);
+}
+
+// ---- double points ---------------------------------------------------------
+
+uint64_t split_rows_f64(clk_context *ctx, const clk_kernel_config *cfg, uint64_t d, uint64_t n, uint64_t k, bool fused)
+{
+    if (cfg && (cfg->global_size[0] || (cfg->local_size[0] && cfg->local_size[0] != 256)))
+        return 0;
+    if (n == 0 || (d > 16 && n * d > (1ull << 30)))
+        return 0;
+    // Where the line lies (us, this pass against f64_pass_kernel).  Labeling:
+    // 2M points d=4 k=16 19 / 22, k=8 18 / 18; d=8 k=16 29 / 39; d=32 k=8 120 /
+    // 120, k=100 151 / 576; 200k d=8 k=32 8.5 / 12; 20k d=8 k=32 6.8 / 7.7, d=4
+    // k=100 10 / 8.  Fused step: 2M d=4 k=4 32 / 37; d=2 k=32 31 / 38, k=8 24 /
+    // 23; d=32 k=32 139 / 299; 200k d=8 k=4 16 / 17, d=4 k=16 15 / 15; 20k d=8
+    // k=32 12 / 13, k=16 12 / 10.  One feature: the plain scan always.
+    const uint64_t b = split_bucket(d), cost = k * (2 * b + 3);
+    bool pays;
+    if (d <= 2)
+        pays = fused && d == 2 && n >= 1000000 && k >= 32;
+    else if (n >= 1000000)
+        pays = fused || cost >= 150 + 10 * b;
+    else if (n >= 100000)
+        pays = fused ? b >= 8 || cost >= 300 : cost >= 300 + 20 * b;
+    else
+        pays = b >= 8 && cost >= 600;
+    if (!pays)
+        return 0;
+    const SplitPlan<double> p = fused ? split_plan<true, double>(ctx, d, k) : split_plan<false, double>(ctx, d, k);
+    return p.kern && k >= 2 ? split_grid(ctx, p, n) : 0;
+}
+
+int launch_split_f64(clk_context *ctx, const char *name, uint64_t d, uint64_t n, uint64_t k, const double *points,
+                     const double *centroids, uint64_t *labels, uint64_t rows, double *part, double *max_shift,
+                     hipStream_t stream)
+{
+    const SplitPlan<double> p = part ? split_plan<true, double>(ctx, d, k) : split_plan<false, double>(ctx, d, k);
+    return launch_split(ctx, p, name, rows, d, n, k, points, centroids, labels, GridRef{}, part, max_shift, stream);
 }
 
 }  // namespace clk

@@ -38,10 +38,15 @@
 // makes c_b the strict, unique minimum of e_c.  Every other point -- and every
 // point with a coordinate that is not finite or too large for FP16 -- scans
 // all centroids with the reference's arithmetic.
+//
+// Double points (T = double): s x and -2 s c are rounded to FP32 first, 2^-24
+// relative, which Rx and Rc include; eps = (d+3) 2^-53 and the scans are FP64.
 #pragma once
 
 #include "clk_common.hpp"
 #include "clk_mfma_device.hpp"
+
+#include <type_traits>
 
 namespace clk {
 namespace split {
@@ -62,7 +67,7 @@ struct Shape {
     static constexpr int planes = P < 32 ? P / 4 : 0;  // LDS exchange, u16x8 [64] each
 };
 
-// LDS of one work-group of `waves` waves: table, norms, FP32 centroids
+// LDS of one work-group of `waves` waves: table, norms, centroids as they are
 // (P < 32: [k][P], 0 past d), statistics, exchange.
 template <int P>
 __host__ __device__ constexpr size_t table_bytes(uint32_t ntiles)
@@ -70,15 +75,15 @@ __host__ __device__ constexpr size_t table_bytes(uint32_t ntiles)
     return (size_t)ntiles * Shape<P>::nops * 64 * sizeof(u16x8);
 }
 constexpr uint32_t kStatWords = 16;
-template <int P>
+template <int P, typename T>
 __host__ __device__ constexpr size_t rows_bytes(uint32_t ntiles)
 {
-    return P < 32 ? (size_t)ntiles * 16 * P * sizeof(float) : 0;
+    return P < 32 ? (size_t)ntiles * 16 * P * sizeof(T) : 0;
 }
-template <int P>
+template <int P, typename T>
 __host__ __device__ constexpr size_t lds_bytes(uint32_t ntiles, uint32_t waves)
 {
-    return table_bytes<P>(ntiles) + rows_bytes<P>(ntiles) + (size_t)ntiles * 16 * sizeof(float) +
+    return table_bytes<P>(ntiles) + rows_bytes<P, T>(ntiles) + (size_t)ntiles * 16 * sizeof(float) +
            kStatWords * sizeof(float) +
            (size_t)waves * Shape<P>::planes * 64 * sizeof(u16x8);
 }
@@ -138,10 +143,11 @@ __device__ __forceinline__ void swap16(float &a, float &b)
 }
 
 // What the work-group's table says, wave-uniform.
+template <typename T>
 struct Table {
     const u16x8 *ops;
     const float *norm;
-    const float *rows;
+    const T *rows;
     uint32_t ntiles, kmask;
     float scale;    // s
     // the margin: t0 + tX ||s x|| + tx2 ||s x||^2 + tk (|vb| + |vs|)
@@ -151,17 +157,18 @@ struct Table {
 
 // The margin's coefficients (see the header; each is rounded up by far more
 // than the rounding of its evaluation and of the margin's).
-template <int P>
-__device__ __forceinline__ void set_margin(Table &t, float N, uint32_t d, uint32_t bits)
+template <int P, typename T>
+__device__ __forceinline__ void set_margin(Table<T> &t, float N, uint32_t d, uint32_t bits)
 {
+    constexpr bool f64 = sizeof(T) == 8;
     constexpr float up = 1.0f + 1e-4f;
     const float C2 = 2.0f * sqrtf(N) * up, sd = sqrtf((float)d) * up;
-    const float T = (float)(Shape<P>::terms * d);
-    const float g0 = 2.0f * (T + 1.0f) * mfma::kU;
+    const float terms = (float)(Shape<P>::terms * d);
+    const float g0 = 2.0f * (terms + 1.0f) * mfma::kU;
     const float gamma = g0 / (1.0f - g0) * up;
-    constexpr float alpha = 0x1p-20f;
+    constexpr float alpha = f64 ? 0x1.2p-20f : 0x1p-20f;
     const float beta = 1.01f * 0x1p-24f * sd;
-    const float Rc = 0x1p-22f * C2 + 1.01f * 0x1p-25f * sd;
+    const float Rc = (f64 ? 0x1.5p-22f : 0x1p-22f) * C2 + 1.01f * 0x1p-25f * sd;
     float e1 = (1.0f + alpha) * Rc + alpha * C2 + gamma * 1.004f * C2;
     float e0 = beta * (Rc + C2) + (gamma + 2.0f * mfma::kU) * N;
     if constexpr (P >= 32) {
@@ -170,10 +177,10 @@ __device__ __forceinline__ void set_margin(Table &t, float N, uint32_t d, uint32
         e0 += 0x1p-24f * sd * m;
     }
     e1 *= 1.01f;
-    e0 = 1.01f * e0 + (T + 2.0f) * 0x1p-125f;
-    const float eps = (float)(d + 3) * mfma::kU * up;
+    e0 = 1.01f * e0 + (terms + 2.0f) * 0x1p-125f;
+    const float eps = (float)(d + 3) * (f64 ? 0x1p-53f : mfma::kU) * up;
     const float tr0 = __uint_as_float((bits - 23 + 127) << 23), tr = tr0 / (1.0f - tr0) * up;
-    const float under = t.scale * t.scale * (float)d * 0x1p-125f;
+    const float under = f64 ? 0.0f : t.scale * t.scale * (float)d * 0x1p-125f;
     t.t0 = up * (1.01f * ((2.0f + 2.1f * eps) * e0 + 2.0f * under) + 1e-30f);
     t.tX = up * 1.01f * (2.0f + 2.1f * eps) * e1;
     t.tx2 = up * 1.01f * 2.1f * eps;
@@ -181,16 +188,18 @@ __device__ __forceinline__ void set_margin(Table &t, float N, uint32_t d, uint32
 }
 
 // Build the table of cen [d][k] (whole work-group; ends with a barrier).
-template <int P>
-__device__ __forceinline__ Table stage(const float *__restrict__ cen, uint32_t d, uint32_t k, uint32_t ntiles,
-                                       char *lds)
+template <int P, typename T>
+__device__ __forceinline__ Table<T> stage(const T *__restrict__ cen, uint32_t d, uint32_t k, uint32_t ntiles,
+                                          char *lds)
 {
     using Sh = Shape<P>;
-    Table t;
+    constexpr bool f64 = sizeof(T) == 8;
+    constexpr T kMax = f64 ? (T)DBL_MAX : (T)FLT_MAX;
+    Table<T> t;
     u16x8 *ops = reinterpret_cast<u16x8 *>(lds);
     float *norm = reinterpret_cast<float *>(lds + table_bytes<P>(ntiles));
-    float *rows = norm + ntiles * 16;
-    uint32_t *stat = reinterpret_cast<uint32_t *>(rows + rows_bytes<P>(ntiles) / sizeof(float));
+    T *rows = reinterpret_cast<T *>(norm + ntiles * 16);
+    uint32_t *stat = reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(rows) + rows_bytes<P, T>(ntiles));
     const uint32_t tid = threadIdx.x, B = blockDim.x;
     if (tid < kStatWords)
         stat[tid] = 0;
@@ -199,8 +208,15 @@ __device__ __forceinline__ Table stage(const float *__restrict__ cen, uint32_t d
     uint32_t m = 0;
 #pragma unroll 4
     for (uint32_t i = tid; i < d * k; i += B) {
-        const uint32_t u = __float_as_uint(__builtin_fabsf(cen[i]));
-        m = (u < 0x7F800000u && u > m) ? u : m;
+        if constexpr (f64) {
+            // beyond FP32: as its largest value, which no scale takes
+            const double a = __builtin_fabs(cen[i]);
+            const uint32_t u = __float_as_uint((float)(a < (double)FLT_MAX ? a : (double)FLT_MAX));
+            m = (a <= DBL_MAX && u > m) ? u : m;
+        } else {
+            const uint32_t u = __float_as_uint(__builtin_fabsf(cen[i]));
+            m = (u < 0x7F800000u && u > m) ? u : m;
+        }
     }
     for (int o = 32; o >= 1; o /= 2)
         m = max(m, (uint32_t)__shfl_xor((int)m, o));
@@ -223,8 +239,9 @@ __device__ __forceinline__ Table stage(const float *__restrict__ cen, uint32_t d
             const uint32_t f = P == 4 ? j % 4 : f0 + j;
             const bool lo = P == 4 ? j >= 4 : low;
             const bool in = c < k && f < d && (P != 4 || h < 2);
-            float x = cen[in ? (size_t)f * k + c : 0];
-            x = in && __builtin_fabsf(x) <= FLT_MAX ? -2.0f * s * x : 0.0f;
+            const T raw = cen[in ? (size_t)f * k + c : 0];
+            const bool fin = raw <= kMax && raw >= -kMax;
+            const float x = in && fin ? (float)((T)(-2.0f * s) * raw) : 0.0f;
             _Float16 p = (_Float16)x;
             if (lo)
                 p = (_Float16)(x - (float)p);
@@ -235,18 +252,18 @@ __device__ __forceinline__ Table stage(const float *__restrict__ cen, uint32_t d
     if constexpr (P < 32)
         for (uint32_t i = tid; i < k * P; i += B) {
             const uint32_t c = i % k, f = i / k;
-            rows[c * P + f] = f < d ? cen[(size_t)f * k + c] : 0.0f;
+            rows[c * P + f] = f < d ? cen[(size_t)f * k + c] : (T)0;
         }
     uint32_t nmax = 0;
     for (uint32_t c = tid; c < ntiles * 16; c += B) {
         double q = 0.0;
         bool fin = c < k;
-        const float *col = cen + (fin ? c : 0);
+        const T *col = cen + (fin ? c : 0);
 #pragma unroll 8
         for (uint32_t f = 0; f < d; ++f) {
-            const float v = col[(size_t)f * k];
-            fin = fin && __builtin_fabsf(v) <= FLT_MAX;
-            const double w = (double)(v * s);
+            const T v = col[(size_t)f * k];
+            fin = fin && v <= kMax && v >= -kMax;
+            const double w = (double)(v * (T)s);
             q = __builtin_fma(w, w, q);
         }
         norm[c] = fin ? (float)q : kNever;
@@ -275,7 +292,7 @@ __device__ __forceinline__ Table stage(const float *__restrict__ cen, uint32_t d
     while ((1u << bits) < ntiles * 16)
         ++bits;
     t.kmask = (1u << bits) - 1u;
-    set_margin<P>(t, __uint_as_float(stat[1]), d, bits);
+    set_margin<P, T>(t, __uint_as_float(stat[1]), d, bits);
     return t;
 }
 
@@ -298,8 +315,8 @@ struct PointOps {
 // P <= 16: lane = point, coordinates x (past d any of
 // the point's coordinates again: the centroids are 0 there).  buf: this wave's
 // exchange planes.  Returns a bound >= ||s x||^2.
-template <int P>
-__device__ __forceinline__ float build_points(const float (&x)[P], float s, u16x8 *buf, uint32_t lane,
+template <int P, typename T>
+__device__ __forceinline__ float build_points(const T (&x)[P], float s, u16x8 *buf, uint32_t lane,
                                               PointOps<P> &o)
 {
     static_assert(P < 32, "lane = point form");
@@ -307,7 +324,7 @@ __device__ __forceinline__ float build_points(const float (&x)[P], float s, u16x
     uint32_t hi[P / 2], lo[P / 2];
 #pragma unroll
     for (int f = 0; f < P; f += 2) {
-        const float a = x[f] * s, b = x[f + 1] * s;
+        const float a = (float)(x[f] * (T)s), b = (float)(x[f + 1] * (T)s);
         x2 = __builtin_fmaf(a, a, x2);
         x2 = __builtin_fmaf(b, b, x2);
         split2(a, b, hi[f / 2], lo[f / 2]);
@@ -342,14 +359,14 @@ __device__ __forceinline__ float build_points(const float (&x)[P], float s, u16x
             }
         }
     }
-    return x2 * (1.0f + (float)(2 * P + 8) * mfma::kU);
+    return x2 * (1.0f + (float)(2 * P + 12) * mfma::kU);
 }
 
 // P >= 32: lane (q, h) holds raw[g][kb*8 + j] = feature kb*32 + 8h + j of
 // point g*16 + q (past d as above).  Returns a bound >= ||s x||^2 of this
 // lane's own point (lane 16h + q).
-template <int P>
-__device__ __forceinline__ float build_points(const float (&raw)[4][Shape<P>::nkb * 8], float s, uint32_t lane,
+template <int P, typename T>
+__device__ __forceinline__ float build_points(const T (&raw)[4][Shape<P>::nkb * 8], float s, uint32_t lane,
                                               PointOps<P> &o)
 {
     static_assert(P >= 32, "matrix layout");
@@ -362,7 +379,7 @@ __device__ __forceinline__ float build_points(const float (&raw)[4][Shape<P>::nk
             v4u hi, lo;
 #pragma unroll
             for (int j = 0; j < 8; j += 2) {
-                const float a = raw[g][kb * 8 + j] * s, b = raw[g][kb * 8 + j + 1] * s;
+                const float a = (float)(raw[g][kb * 8 + j] * (T)s), b = (float)(raw[g][kb * 8 + j + 1] * (T)s);
                 x2 = __builtin_fmaf(a, a, x2);
                 x2 = __builtin_fmaf(b, b, x2);
                 uint32_t h, l;
@@ -377,7 +394,7 @@ __device__ __forceinline__ float build_points(const float (&raw)[4][Shape<P>::nk
         x2 += __shfl_xor(x2, 32);
         mine = (uint32_t)g == lane / 16 ? x2 : mine;
     }
-    return mine * (1.0f + (float)(2 * P + 8) * mfma::kU);
+    return mine * (1.0f + (float)(2 * P + 12) * mfma::kU);
 }
 
 // The two smallest keys of this lane's own point over all centroids.  A key's
@@ -390,8 +407,8 @@ __device__ __forceinline__ uint32_t centroid_of(float key, uint32_t kmask)
     return (l & ~15u) | ((l & 3u) << 2) | ((l >> 2) & 3u);
 }
 
-template <int P>
-__device__ __forceinline__ void rank_points(const Table &t, const PointOps<P> &x, uint32_t lane, float &best,
+template <int P, typename T>
+__device__ __forceinline__ void rank_points(const Table<T> &t, const PointOps<P> &x, uint32_t lane, float &best,
                                             float &second)
 {
     using Sh = Shape<P>;
@@ -462,7 +479,8 @@ __device__ __forceinline__ void rank_points(const Table &t, const PointOps<P> &x
 }
 
 // Margin test of this lane's own point; lab = the best key's centroid.
-__device__ __forceinline__ bool decide(const Table &t, float x2, float best, float second, uint32_t k, uint32_t &lab)
+template <typename T>
+__device__ __forceinline__ bool decide(const Table<T> &t, float x2, float best, float second, uint32_t k, uint32_t &lab)
 {
     const float X = __builtin_amdgcn_sqrtf(x2);  // within one ulp
     const float ab = __builtin_fabsf(best);
@@ -480,10 +498,14 @@ __device__ __forceinline__ bool decide(const Table &t, float x2, float best, flo
 // centroid while k <= G), sixteen features' loads in flight.  base: the
 // coordinate of feature 0 of the wave's point 0, the rows n apart.  lab of
 // lane i becomes the label of point i.
-__device__ __forceinline__ void exact_scan(uint64_t open, const float *__restrict__ base, uint64_t n,
-                                           const float *__restrict__ cen, uint32_t d, uint32_t k, uint32_t lane,
+template <typename T>
+__device__ __forceinline__ void exact_scan(uint64_t open, const T *__restrict__ base, uint64_t n,
+                                           const T *__restrict__ cen, uint32_t d, uint32_t k, uint32_t lane,
                                            uint32_t &lab)
 {
+    constexpr bool f64 = sizeof(T) == 8;
+    constexpr T kMax = f64 ? (T)DBL_MAX : (T)FLT_MAX;
+    constexpr uint32_t kAhead = f64 ? 8 : 16;
     uint32_t G = 8;
     while (G < k && G < 64)
         G *= 2;
@@ -495,26 +517,29 @@ __device__ __forceinline__ void exact_scan(uint64_t open, const float *__restric
             rest &= rest - 1;
             src = lane / G >= i ? bit : src;  // groups past the last point repeat it
         }
-        const float *x = base + src;
-        float best = FLT_MAX;
+        const T *x = base + src;
+        T best = kMax;
         uint32_t bi = 0;
         for (uint32_t c0 = 0; c0 < k; c0 += G) {
             const uint32_t c = c0 + lane % G;
-            const float *col = cen + min(c, k - 1);
-            float dist = 0.0f;
-            for (uint32_t f0 = 0; f0 < d; f0 += 16) {
-                float xv[16], cv[16];
+            const T *col = cen + min(c, k - 1);
+            T dist = 0;
+            for (uint32_t f0 = 0; f0 < d; f0 += kAhead) {
+                T xv[kAhead], cv[kAhead];
 #pragma unroll
-                for (uint32_t j = 0; j < 16; ++j) {
+                for (uint32_t j = 0; j < kAhead; ++j) {
                     const uint32_t f = min(f0 + j, d - 1);
                     xv[j] = x[(uint64_t)f * n];
                     cv[j] = col[(size_t)f * k];
                 }
 #pragma unroll
-                for (uint32_t j = 0; j < 16; ++j)
+                for (uint32_t j = 0; j < kAhead; ++j)
                     if (f0 + j < d) {
-                        const float u = xv[j] - cv[j];
-                        dist = __builtin_fmaf(u, u, dist);
+                        const T u = xv[j] - cv[j];
+                        if constexpr (f64)
+                            dist = __builtin_fma(u, u, dist);
+                        else
+                            dist = __builtin_fmaf(u, u, dist);
                     }
             }
             if (c < k && dist < best) {
@@ -522,16 +547,16 @@ __device__ __forceinline__ void exact_scan(uint64_t open, const float *__restric
                 bi = c;
             }
         }
-        // smallest distance, lowest index on equal distances; none below
-        // FLT_MAX gives label 0
-        uint32_t hi = __float_as_uint(best);
+        // smallest distance, lowest index on equal distances; none below the
+        // largest value gives label 0
         for (uint32_t o = G / 2; o >= 1; o /= 2) {
-            const uint32_t h2 = (uint32_t)__shfl_xor((int)hi, (int)o), i2 = (uint32_t)__shfl_xor((int)bi, (int)o);
-            const bool take = h2 < hi || (h2 == hi && i2 < bi);
-            hi = take ? h2 : hi;
+            const T b2 = __shfl_xor(best, (int)o);
+            const uint32_t i2 = (uint32_t)__shfl_xor((int)bi, (int)o);
+            const bool take = b2 < best || (b2 == best && i2 < bi);
+            best = take ? b2 : best;
             bi = take ? i2 : bi;
         }
-        const uint32_t found = hi < __float_as_uint(FLT_MAX) ? bi : 0u;
+        const uint32_t found = best < kMax ? bi : 0u;
         for (uint32_t i = 0; i < 64 / G && open; ++i) {
             const uint32_t bit = (uint32_t)__builtin_ctzll(open);
             open &= open - 1;
@@ -539,6 +564,34 @@ __device__ __forceinline__ void exact_scan(uint64_t open, const float *__restric
             lab = lane == bit ? r : lab;
         }
     }
+}
+
+// The reference's scan of this lane's own point x over the staged rows.
+template <int P, typename T>
+__device__ __forceinline__ uint32_t scan_rows(const Table<T> &t, const T (&x)[P], uint32_t d, uint32_t k)
+{
+    T best = sizeof(T) == 8 ? (T)DBL_MAX : (T)FLT_MAX;
+    uint32_t lab = 0;
+    T own[P];
+#pragma unroll
+    for (int f = 0; f < P; ++f)
+        own[f] = f < (int)d ? x[f] : (T)0;
+    for (uint32_t c = 0; c < k; ++c) {
+        const T *row = t.rows + c * P;
+        T dist = 0;
+#pragma unroll
+        for (int f = 0; f < P; ++f) {  // 0 past d: adds fma(0, 0, dist) == dist
+            const T u = own[f] - row[f];
+            if constexpr (sizeof(T) == 8)
+                dist = __builtin_fma(u, u, dist);
+            else
+                dist = __builtin_fmaf(u, u, dist);
+        }
+        const bool lt = dist < best;
+        best = lt ? dist : best;
+        lab = lt ? c : lab;
+    }
+    return lab;
 }
 
 }  // namespace split

@@ -70,3 +70,38 @@ def test_split_scales(gpu_ctx, scale):
     gpu_ctx.labeling(gpu_ctx.config(clkmeans.STAGE_LABELING, "unroll_vector"), d, n, k, dev(pts), dev(cen), labels)
     hip.synchronize()
     np.testing.assert_array_equal(labels.to_host(), O.label(pts, cen))
+
+
+@pytest.mark.parametrize("kind", ["blobs", "lattice", "offset", "special", "huge"])
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "n%d_d%d_k%d" % s)
+def test_split_double(gpu_ctx, shape, kind):
+    """Double points: labels and masses exact; sums within FP64 rounding of a
+    different order (1e-13 of the cell's sum of |x|, as in test_gpu_f64)."""
+    n, d, k = shape
+    p32 = points(n, d, k, "blobs" if kind == "huge" else kind, n + d + k)
+    cen32 = centroids(p32, k, kind)
+    wiggle = np.random.default_rng(d).standard_normal(p32.shape) * 1e-9
+    lattice = kind == "lattice"
+    pts = p32.astype(np.float64) * (1.0 if lattice else 1.0 + wiggle)
+    cen = np.ascontiguousarray(pts[:, np.arange(k) * 2 % n])
+    if kind == "special":
+        cen[~np.isfinite(cen)] = 1.0
+        cen[~np.isfinite(cen32)] = cen32[~np.isfinite(cen32)]
+    if kind == "huge":  # beyond FP32, and one centroid far beyond the others
+        pts, cen = pts * 1e60, cen * 1e60
+        cen[:, k - 1] *= 1e80
+    ref = O.label_f64(pts, cen)
+    labels = dev(np.full(n, 2 ** 64 - 1, np.uint64))
+    gpu_ctx.labeling(gpu_ctx.config(clkmeans.STAGE_LABELING, "unroll_vector"), d, n, k, dev(pts), dev(cen), labels)
+    hip.synchronize()
+    np.testing.assert_array_equal(labels.to_host(), ref)
+    labels = dev(np.full(n, 2 ** 64 - 1, np.uint64))
+    sums, masses = zeros((d, k), np.float64), zeros(k, np.uint64)
+    gpu_ctx.fused(gpu_ctx.config(clkmeans.STAGE_FUSED, "cluster_merge"), d, n, k, dev(pts), dev(cen), sums, labels, masses)
+    hip.synchronize()
+    np.testing.assert_array_equal(labels.to_host(), ref)
+    np.testing.assert_array_equal(masses.to_host(), O.mass_u64(ref, k))
+    if kind != "special":
+        exact = O.sums_f64_dp(pts, ref, k)
+        absx = np.stack([np.bincount(ref.astype(np.int64), weights=np.abs(x), minlength=k) for x in pts])
+        assert np.all(np.abs(sums.to_host() - exact) <= 1e-13 * absx + 1e-300)
