@@ -141,7 +141,7 @@ split_kernel(const T *__restrict__ pts, uint64_t n, uint32_t d, uint32_t k, cons
             }
         }
         if (open)
-            exact_scan(open, pts + bt * 64, n, cen, d, k, lane, lab);
+            exact_scan<P>(open, pts + bt * 64, n, cen, d, k, lane, lab);
         if (p < n)
             stream_store((LabelT)lab, labels + p);
         if constexpr (FUSED) {

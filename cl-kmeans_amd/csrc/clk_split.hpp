@@ -495,17 +495,17 @@ __device__ __forceinline__ bool decide(const Table<T> &t, float x2, float best, 
 
 // The reference's scan, over all centroids, of the wave's points whose bit is
 // set in open: 64 / G points at a time, G lanes each (8 <= G <= 64, a lane per
-// centroid while k <= G), sixteen features' loads in flight.  base: the
+// centroid while k <= G), up to sixteen features' loads in flight.  base: the
 // coordinate of feature 0 of the wave's point 0, the rows n apart.  lab of
 // lane i becomes the label of point i.
-template <typename T>
+template <int P, typename T>
 __device__ __forceinline__ void exact_scan(uint64_t open, const T *__restrict__ base, uint64_t n,
                                            const T *__restrict__ cen, uint32_t d, uint32_t k, uint32_t lane,
                                            uint32_t &lab)
 {
     constexpr bool f64 = sizeof(T) == 8;
     constexpr T kMax = f64 ? (T)DBL_MAX : (T)FLT_MAX;
-    constexpr uint32_t kAhead = f64 ? 8 : 16;
+    constexpr uint32_t kAhead = P == 4 ? 4 : f64 ? 8 : 16;
     uint32_t G = 8;
     while (G < k && G < 64)
         G *= 2;
@@ -573,9 +573,10 @@ __device__ __forceinline__ uint32_t scan_rows(const Table<T> &t, const T (&x)[P]
     T best = sizeof(T) == 8 ? (T)DBL_MAX : (T)FLT_MAX;
     uint32_t lab = 0;
     T own[P];
+    const uint32_t dd = mfma::opaque_s(d);  // no tests kept in scalar registers
 #pragma unroll
     for (int f = 0; f < P; ++f)
-        own[f] = f < (int)d ? x[f] : (T)0;
+        own[f] = f < (int)dd ? x[f] : (T)0;
     for (uint32_t c = 0; c < k; ++c) {
         const T *row = t.rows + c * P;
         T dist = 0;
