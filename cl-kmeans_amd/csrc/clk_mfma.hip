@@ -79,106 +79,133 @@ __global__ void __launch_bounds__(64) mfma_subnormal_check_kernel(float *out)
     }
 }
 
-// Per-iteration centroid tables (three small launches: clear, build, finish):
+// Per-iteration centroid tables, one launch, a work-group per tile of 16
+// centroids:
 //   table[t][kb][lane] = 8 x 16-bit of -2c for centroid t*16 + lane%16,
 //                        features kb*32 + 8*(lane/16) + j (0 past d or k)
 //   norm[c] = RN(||c||^2) (FP32); +inf for a padded or non-finite centroid,
 //             one whose ||c||^2 overflows, or (FP16) whose -2c overflows
 //   cenT[c][f] = the FP32 centroids transposed (ntiles*16 rows of nkb*32, 0
 //             past d or k), for the exact distances of the refinement
-//   stats[0] = C >= max ||c||, stats[1] = N >= max ||c||^2, stats[3] = R >=
-//   max ||c̃ + 2c|| over the others; stats[2] = 1 when a centroid with finite
-//   coordinates had to be left out (its 16-bit or squared norm overflows):
-//   then every point is scanned exactly; stats[4] (as uint32) = refinement
-//   queue length; stats[12..15] = the build's running maxima (FP64 bits of
-//   non-negative values order like the values) and the dropped flag.
-__global__ void __launch_bounds__(64) mfma_prepare_clear_kernel(float *__restrict__ stats)
-{
-    if (threadIdx.x < 16)
-        stats[threadIdx.x] = 0.0f;
-}
+//   tiles[t] = the tile's maxima of ||c||^2 and ||c̃ + 2c||^2 and whether a
+//             centroid with finite coordinates had to be left out (its 16-bit
+//             or squared norm overflows): then every point is scanned exactly
+//   *qlen = 0, and the score offset this labeling will record, hint = 0.
+// The labeling and refinement work-groups reduce tiles[] themselves
+// (load_stats), so there is no launch to clear or finish anything (three
+// launches took 28 us at d = 64, k = 1024).
+struct TileStats {
+    double norm, residual;
+    double dropped;
+};
+constexpr uint32_t kStatFloats = 8;  // load_stats' output
 
 template <bool FP16>
 __global__ void __launch_bounds__(256)
-mfma_prepare_kernel(const float *__restrict__ cen, uint32_t d, uint32_t k, uint32_t ntiles,
-                    uint32_t nkb, u16x8 *__restrict__ table, float *__restrict__ norm,
-                    float *__restrict__ stats, float *__restrict__ cenT)
+mfma_prepare_kernel(const float *__restrict__ cen, uint32_t d, uint32_t k, uint32_t nkb, u16x8 *__restrict__ table,
+                    float *__restrict__ norm, TileStats *__restrict__ tiles, float *__restrict__ cenT,
+                    uint32_t *__restrict__ qlen, float *__restrict__ hint)
 {
-    const uint64_t tid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    const uint64_t entries = (uint64_t)ntiles * nkb * 64;
-    for (uint64_t e = tid; e < entries; e += stride) {
-        const uint32_t lane = (uint32_t)(e % 64);
-        const uint64_t tk = e / 64;
-        const uint32_t kb = (uint32_t)(tk % nkb), t = (uint32_t)(tk / nkb);
+    constexpr uint32_t kParts = 256 / kTile;
+    __shared__ double part_s[kParts][kTile], part_r[kParts][kTile];
+    __shared__ uint32_t part_bad[kParts][kTile];  // bit 0: not finite, bit 1: out of the 16-bit range
+    const uint32_t tid = threadIdx.x, t = blockIdx.x;
+    if (t == 0 && tid == 0) {
+        *qlen = 0;
+        *hint = 0.0f;
+    }
+    for (uint32_t e = tid; e < nkb * 64; e += 256) {
+        const uint32_t lane = e % 64, kb = e / 64;
         const uint32_t c = t * kTile + lane % 16;
         u16x8 v;
+#pragma unroll
         for (int j = 0; j < 8; ++j) {
             const uint32_t f = kb * kKBlock + 8 * (lane / 16) + j;
-            float x = (c < k && f < d) ? -2.0f * cen[(uint64_t)f * k + c] : 0.0f;
+            const bool in = c < k && f < d;
+            float x = in ? -2.0f * cen[(uint64_t)f * k + c] : 0.0f;
             if (!isfinite(x))
                 x = 0.0f;  // such a centroid is excluded through norm = +inf
             v[j] = to16<FP16>(x);
         }
-        table[e] = v;
+        table[(uint64_t)t * nkb * 64 + e] = v;
     }
     const uint32_t P = nkb * kKBlock;
-    for (uint64_t e = tid; e < (uint64_t)ntiles * kTile * P; e += stride) {
-        const uint32_t c = (uint32_t)(e / P), f = (uint32_t)(e % P);
-        cenT[e] = (c < k && f < d) ? cen[(uint64_t)f * k + c] : 0.0f;
+    for (uint32_t e = tid; e < kTile * P; e += 256) {
+        const uint32_t c = t * kTile + e % kTile, f = e / kTile;
+        cenT[(uint64_t)c * P + f] = (c < k && f < d) ? cen[(uint64_t)f * k + c] : 0.0f;
     }
-    double nmax = 0.0, rmax = 0.0;
-    bool dropped = false;  // a centroid with finite coordinates left out
-    for (uint64_t c = tid; c < (uint64_t)ntiles * kTile; c += stride) {
+    {
+        const uint32_t j = tid % kTile, part = tid / kTile, c = t * kTile + j;
         double s = 0.0, r = 0.0;
-        bool fin = c < k, in_range = true;
-        for (uint32_t f = 0; f < d && fin; ++f) {
-            const float v = cen[(uint64_t)f * k + c];
-            fin = isfinite(v);
-            in_range = in_range && (!FP16 || fabs(2.0 * (double)v) < 65504.0);
-            s = fma((double)v, (double)v, s);
-            const double res = (double)from16<FP16>(to16<FP16>(-2.0f * v)) + 2.0 * (double)v;
-            r = fma(res, res, r);
-        }
-        const bool ok = fin && in_range && s < 3.0e38;
-        dropped = dropped || (fin && !ok);
-        norm[c] = ok ? (float)s : INFINITY;
-        if (ok) {
-            nmax = fmax(nmax, s);
-            rmax = fmax(rmax, r);
-        }
+        uint32_t bad = c < k ? 0u : 1u;
+        if (c < k)
+            for (uint32_t f = part; f < d; f += kParts) {
+                const float v = cen[(uint64_t)f * k + c];
+                bad |= isfinite(v) ? 0u : 1u;
+                bad |= (!FP16 || fabs(2.0 * (double)v) < 65504.0) ? 0u : 2u;
+                s = fma((double)v, (double)v, s);
+                const double res = (double)from16<FP16>(to16<FP16>(-2.0f * v)) + 2.0 * (double)v;
+                r = fma(res, res, r);
+            }
+        part_s[part][j] = s;
+        part_r[part][j] = r;
+        part_bad[part][j] = bad;
     }
-    unsigned long long *acc = reinterpret_cast<unsigned long long *>(stats + 12);
-    if (nmax > 0.0)
-        atomicMax(&acc[0], (unsigned long long)__double_as_longlong(nmax));
-    if (rmax > 0.0)
-        atomicMax(&acc[1], (unsigned long long)__double_as_longlong(rmax));
-    if (dropped)
-        atomicOr(reinterpret_cast<uint32_t *>(stats) + 2, 1u);
+    __syncthreads();
+    if (tid >= kTile)
+        return;
+    double s = 0.0, r = 0.0;
+    uint32_t bad = 0;
+    for (uint32_t part = 0; part < kParts; ++part) {
+        s += part_s[part][tid];
+        r += part_r[part][tid];
+        bad |= part_bad[part][tid];
+    }
+    const bool ok = bad == 0 && s < 3.0e38;
+    const bool dropped = (bad & 1u) == 0 && !ok;
+    norm[t * kTile + tid] = ok ? (float)s : INFINITY;
+    double nmax = ok ? s : 0.0, rmax = ok ? r : 0.0, dmax = dropped ? 1.0 : 0.0;
+    for (int o = kTile / 2; o >= 1; o /= 2) {
+        nmax = fmax(nmax, __shfl_xor(nmax, o));
+        rmax = fmax(rmax, __shfl_xor(rmax, o));
+        dmax = fmax(dmax, __shfl_xor(dmax, o));
+    }
+    if (tid == 0)
+        tiles[t] = TileStats{nmax, rmax, dmax};
 }
 
-// stats[5] = the launch-wide score offset K_L for this labeling: 1.02 x the
-// largest per-wave K of the previous labeling on this context (hint[0],
-// reset here for this labeling to record its own), or 0 (none).  A wave
-// whose own K is <= K_L uses K_L with the norms pre-offset in LDS; any K >=
-// ||x||^2 + E is valid, so K_L only changes which waves take that path.
-__global__ void __launch_bounds__(64) mfma_prepare_finish_kernel(float *__restrict__ stats, float *__restrict__ hint)
+// The statistics of a labeling into LDS (wave 0; the caller adds a barrier):
+// stats[0] = C >= max ||c||, stats[1] = N >= max ||c||^2, stats[2] = 1 when
+// every point is scanned exactly, stats[3] = R >= max ||c̃ + 2c||, stats[5] =
+// the launch-wide score offset K_L: 1.02 x the largest per-wave K of the
+// previous labeling on this context (*hint), or 0 (none).  A wave whose own K
+// is <= K_L uses K_L with the norms pre-offset in LDS; any K >= ||x||^2 + E is
+// valid, so K_L only changes which waves take that path.
+__device__ __forceinline__ void load_stats(const TileStats *__restrict__ tiles, uint32_t ntiles, float hint,
+                                           float *stats)
 {
+    if (threadIdx.x >= 64)
+        return;
+    double n = 0.0, r = 0.0, drop = 0.0;
+    for (uint32_t t = threadIdx.x; t < ntiles; t += 64) {
+        n = fmax(n, tiles[t].norm);
+        r = fmax(r, tiles[t].residual);
+        drop = fmax(drop, tiles[t].dropped);
+    }
+    for (int o = 32; o >= 1; o /= 2) {
+        n = fmax(n, __shfl_xor(n, o));
+        r = fmax(r, __shfl_xor(r, o));
+        drop = fmax(drop, __shfl_xor(drop, o));
+    }
     if (threadIdx.x == 0) {
-        const float hv = hint[0];
-        stats[5] = (hv > 0.0f && hv < 1e30f) ? hv * 1.02f : 0.0f;
-        hint[0] = 0.0f;
-        const unsigned long long *acc = reinterpret_cast<const unsigned long long *>(stats + 12);
-        const double n = __longlong_as_double((long long)acc[0]) * (1.0 + 1e-12);
-        const double r = __longlong_as_double((long long)acc[1]);
+        n *= 1.0 + 1e-12;
         stats[0] = (float)(sqrt(n) * (1.0 + 1e-6));
         stats[1] = (float)(n * (1.0 + 1e-6));
-        stats[2] = reinterpret_cast<const uint32_t *>(stats)[2] ? 1.0f : 0.0f;  // 1: exact scan
+        stats[2] = (float)drop;
         stats[3] = (float)(sqrt(r) * (1.0 + 1e-6) + 1e-38);
+        stats[5] = (hint > 0.0f && hint < 1e30f) ? hint * 1.02f : 0.0f;
     }
 }
-
-
 
 // Streaming kernel: work-group of fast_waves(NKB) waves (up to d = 64 three
 // per SIMD sharing one LDS table, so each wave's point loads and LDS reads
@@ -190,24 +217,38 @@ __global__ void __launch_bounds__(64) mfma_prepare_finish_kernel(float *__restri
 // appended to qidx[] / qthr[] (T, above; count at *qlen).
 constexpr int fast_waves(int nkb) { return nkb <= 2 ? 12 : 4; }
 
+struct QueueEntry {
+    uint32_t point;
+    float thr;
+};
+
 // Score offset: each wave needs K >= ||x||^2 + E over its points (wave_bounds).
 // With a launch-wide K_L (stats[5]; 0 = none) the norms are staged a second
 // time as RN(||c||^2 + K_L), and a wave whose own K is <= K_L starts its
 // accumulators from those (no add per tile); the others add their own K.
-// Every wave's own K goes to hint[0] (atomic max of positive float bits) for
+// Every wave's own K goes to *hint_out (atomic max of positive float bits) for
 // the next labeling's K_L.
+// Queue: a wave collects its undecided points in LDS (qbuf, 64 entries) and
+// takes queue slots for up to 64 at a time: the returning atomics on one
+// address cost about 45 ns each, and one for nearly every 64-point step held the
+// kernel back (2M points d=64 k=1024: 317 -> 296 us).  Tables that leave no LDS
+// for it (qbuf_ok false) append step by step.
 template <bool FP16, int NKB, bool FULL>
 __global__ void __launch_bounds__(64 * fast_waves(NKB))
 label_mfma_kernel(const float *__restrict__ pts, uint64_t n, uint32_t d, uint32_t k,
                   const u16x8 *__restrict__ table, const float *__restrict__ norm,
-                  const float *__restrict__ stats, uint32_t ntiles, MfmaParams prm,
+                  const TileStats *__restrict__ tiles, uint32_t ntiles, MfmaParams prm,
                   uint32_t *__restrict__ labels, uint32_t *__restrict__ qidx,
-                  float *__restrict__ qthr, uint32_t *__restrict__ qlen, float *__restrict__ hint,
+                  float *__restrict__ qthr, uint32_t *__restrict__ qlen, const float *__restrict__ hint_in,
+                  float *__restrict__ hint_out, int qbuf_ok,
                   const u16x8 *__restrict__ pin_ops, const f32v4 *__restrict__ pin_x2)
 {
     extern __shared__ __align__(16) u16x8 lds_table[];
+    __shared__ float stats[kStatFloats];
     float *lds_norm = reinterpret_cast<float *>(lds_table + (uint64_t)ntiles * NKB * 64);
     float *lds_normk = lds_norm + (size_t)ntiles * kTile;
+    load_stats(tiles, ntiles, *hint_in, stats);
+    __syncthreads();
     const float KL = stats[5];
     stage_table<NKB>(lds_table, lds_norm, table, norm, ntiles, KL > 0.0f ? lds_normk : nullptr, KL);
     float kmax = 0.0f;  // this wave's largest own K
@@ -218,6 +259,24 @@ label_mfma_kernel(const float *__restrict__ pts, uint64_t n, uint32_t d, uint32_
     const float tr1 = prm.trunc / (1.0f - prm.trunc), ep1 = prm.eps / (1.0f - prm.eps);
 
     constexpr int kWaves = fast_waves(NKB);
+    QueueEntry *const qbuf = reinterpret_cast<QueueEntry *>(lds_normk + (size_t)ntiles * kTile) + wave * 64;
+    uint32_t pending = 0;  // wave-uniform
+    auto take_slots = [&](uint32_t count) -> uint32_t {
+        uint32_t slot0 = 0;
+        if (lane == 0)
+            slot0 = atomicAdd(qlen, count);
+        return (uint32_t)__builtin_amdgcn_readfirstlane((int)slot0);
+    };
+    auto flush_queue = [&]() {
+        const uint32_t slot0 = take_slots(pending);
+        if (lane < pending) {
+            const QueueEntry e = qbuf[lane];
+            qidx[slot0 + lane] = e.point;
+            qthr[slot0 + lane] = e.thr;
+        }
+        wave_lds_order();
+        pending = 0;
+    };
     const uint64_t batches = (n + 63) / 64;
     for (uint64_t bt = (uint64_t)blockIdx.x * kWaves + wave; bt < batches;
          bt += (uint64_t)gridDim.x * kWaves) {
@@ -278,20 +337,29 @@ label_mfma_kernel(const float *__restrict__ pts, uint64_t n, uint32_t d, uint32_
             labels[p] = mine;  // provisional for queued points
         const uint64_t m = __ballot(amb && p < n);
         if (m != 0) {
-            const uint32_t first = (uint32_t)__builtin_ctzll(m);
-            uint32_t slot0 = 0;
-            if (lane == first)
-                slot0 = atomicAdd(qlen, (uint32_t)__builtin_popcountll(m));
-            slot0 = __shfl(slot0, (int)first);
-            if (amb && p < n) {
-                const uint32_t slot = slot0 + lanes_below(m);
-                qidx[slot] = (uint32_t)p;
-                qthr[slot] = T;
+            const uint32_t count = (uint32_t)__builtin_popcountll(m);
+            if (qbuf_ok) {
+                if (pending + count > 64)
+                    flush_queue();
+                if (amb && p < n)
+                    qbuf[pending + lanes_below(m)] = QueueEntry{(uint32_t)p, T};
+                wave_lds_order();
+                pending += count;
+            } else {
+                const uint32_t slot0 = take_slots(count);
+                if (amb && p < n) {
+                    const uint32_t slot = slot0 + lanes_below(m);
+                    qidx[slot] = (uint32_t)p;
+                    qthr[slot] = T;
+                }
             }
         }
     }
-    if (lane == 0 && kmax > 0.0f)
-        atomicMax(reinterpret_cast<uint32_t *>(hint), __float_as_uint(kmax));
+    if (pending)
+        flush_queue();
+    if (lane == 0 && kmax > 0.0f && __float_as_uint(kmax) > __hip_atomic_load(reinterpret_cast<uint32_t *>(hint_out),
+                                                                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMax(reinterpret_cast<uint32_t *>(hint_out), __float_as_uint(kmax));
 }
 
 // The pinned operand copy of points[d][n] (clk_labeling_pin_points): for
@@ -315,7 +383,7 @@ mfma_pin_kernel(const float *__restrict__ pts, uint64_t n, uint32_t d, u16x8 *__
     PointOps<NKB> x;
     float X2[kGroups];
     float unused[kGroups][NKB * 8];
-    load_points_core<FP16, NKB, false, false>(x, X2, pts, n, d, pid, q, h, nullptr, unused);
+    load_points_core<FP16, NKB, false, false>(x, X2, pts, n, d, pid, q, h, unused);
 #pragma unroll
     for (int g = 0; g < kGroups; ++g)
 #pragma unroll
@@ -331,37 +399,47 @@ mfma_pin_kernel(const float *__restrict__ pts, uint64_t n, uint32_t d, u16x8 *__
 
 constexpr uint32_t kPairCap = 1024;  // candidate pairs per wave and flush
 constexpr int kRefineWaves = 4;
+constexpr uint32_t kRowPad = 4;           // a row of points in LDS is shifted by a bank group from the last
 
-// Refinement kernel for the queued points (see the header).  The 16-bit table
-// and norms are read from L2 (tile t+1 prefetched while tile t is scored);
-// LDS holds, per wave, the 64 points' FP32 rows, a pair list, the point ids,
-// the running (distance bits << 32 | centroid) minimum of each point and a
-// pair counter.  cenT = the centroids transposed, [ntiles*16][P] FP32.
+// Refinement kernel for the queued points (see the header): a work-group per
+// batch of 64 points, its waves taking every kRefineWaves-th tile (there are
+// fewer batches than waves on the GPU, and one wave over all tiles of a batch
+// is a chain of L2 loads), and each loading 16 of the points, whose values lie
+// n apart (a cache line each): 2M points d=64 k=1024 100 -> 70 us.  The 16-bit table
+// and norms are read from L2 (the next tile prefetched while this one is
+// scored); LDS holds the 64 points' FP32 rows, their running (distance bits <<
+// 32 | centroid) minima, and per wave a pair list and its counter.  cenT = the
+// centroids transposed, [ntiles*16][P] FP32.
 template <bool FP16, int NKB, bool FULL>
 __global__ void __launch_bounds__(64 * kRefineWaves)
 refine_mfma_kernel(const float *__restrict__ pts, uint64_t n, uint32_t d, uint32_t k,
                    const float *__restrict__ cenT, const u16x8 *__restrict__ table,
-                   const float *__restrict__ norm, const float *__restrict__ stats,
+                   const float *__restrict__ norm, const TileStats *__restrict__ tiles,
                    uint32_t ntiles, MfmaParams prm, uint32_t *__restrict__ labels,
                    const uint32_t *__restrict__ qidx, const float *__restrict__ qthr,
                    const uint32_t *__restrict__ qlen)
 {
-    constexpr uint32_t P = NKB * kKBlock;
+    constexpr uint32_t P = NKB * kKBlock, kRow = P + kRowPad;
+    static_assert(kRefineWaves == kGroups, "a wave loads a group of points");
     const uint32_t qn = *qlen;
     const uint64_t batches = ((uint64_t)qn + 63) / 64;
-    const uint32_t lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+    if (blockIdx.x >= batches)
+        return;
+    const uint32_t lane = threadIdx.x % 64;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / 64));
     extern __shared__ __align__(16) float lds_x[];
-    float *xs = lds_x + wave * 64 * P;
-    uint32_t *pairs = reinterpret_cast<uint32_t *>(lds_x + kRefineWaves * 64 * P) + wave * kPairCap;
-    unsigned long long *lds_min = reinterpret_cast<unsigned long long *>(
-        reinterpret_cast<uint32_t *>(lds_x + kRefineWaves * 64 * P) + kRefineWaves * kPairCap);
-    unsigned long long *wmin = lds_min + wave * 64;
-    uint32_t *wcount = reinterpret_cast<uint32_t *>(lds_min + kRefineWaves * 64) + wave;
+    __shared__ float stats[kStatFloats];
+    float *const xs = lds_x;
+    uint32_t *pairs = reinterpret_cast<uint32_t *>(lds_x + 64 * kRow) + wave * kPairCap;
+    unsigned long long *wmin = reinterpret_cast<unsigned long long *>(
+        reinterpret_cast<uint32_t *>(lds_x + 64 * kRow) + kRefineWaves * kPairCap);
+    uint32_t *wcount = reinterpret_cast<uint32_t *>(wmin + 64) + wave;
+    load_stats(tiles, ntiles, 0.0f, stats);
+    __syncthreads();
     const uint32_t q = lane % 16, h = lane / 16;
     const uint32_t kmask = (1u << prm.key_bits) - 1u;
 
-    for (uint64_t bt = (uint64_t)blockIdx.x * kRefineWaves + wave; bt < batches;
-         bt += (uint64_t)gridDim.x * kRefineWaves) {
+    for (uint64_t bt = blockIdx.x; bt < batches; bt += gridDim.x) {  // the same for every wave
         uint64_t pid[kGroups];
         float thr_in[kGroups];
 #pragma unroll
@@ -373,7 +451,34 @@ refine_mfma_kernel(const float *__restrict__ pts, uint64_t n, uint32_t d, uint32
         }
         PointOps<NKB> x;
         float X2[kGroups];
-        load_points<FP16, NKB, FULL>(x, X2, pts, n, d, pid, q, h, xs);
+        {  // wave g loads group g's rows into LDS; every wave builds all operands from there
+            const uint64_t slot = bt * 64 + wave * 16 + q;
+            float raw[NKB * 8];
+            load_raw<NKB, FULL>(raw, pts, n, d, slot < qn ? (uint64_t)qidx[slot] : ~0ull, h);
+            float *row = xs + (wave * 16 + q) * kRow + 8 * h;
+#pragma unroll
+            for (int v = 0; v < NKB * 2; ++v)
+                *reinterpret_cast<f32v4 *>(row + (v / 2) * kKBlock + (v % 2) * 4) =
+                    f32v4{raw[4 * v], raw[4 * v + 1], raw[4 * v + 2], raw[4 * v + 3]};
+        }
+        if (wave == 0)
+            wmin[lane] = ~0ull;  // slot lane = 16 h + q
+        if (lane == 0)
+            *wcount = 0;
+        __syncthreads();
+#pragma unroll
+        for (int g = 0; g < kGroups; ++g) {
+            const float *row = xs + (g * 16 + q) * kRow + 8 * h;
+            float raw[NKB * 8];
+#pragma unroll
+            for (int v = 0; v < NKB * 2; ++v) {
+                const f32v4 r = *reinterpret_cast<const f32v4 *>(row + (v / 2) * kKBlock + (v % 2) * 4);
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    raw[4 * v + j] = r[j];
+            }
+            X2[g] = build_operands<FP16, NKB>(x.b[g], raw);
+        }
         const WaveBounds w = wave_bounds<NKB, FP16>(X2, stats, prm);
         // candidate threshold on this kernel's scores: T + K' + E', rounded up;
         // NaN or infinite -> every centroid is a candidate
@@ -391,10 +496,6 @@ refine_mfma_kernel(const float *__restrict__ pts, uint64_t n, uint32_t d, uint32
         for (int g = 1; g < kGroups; ++g)
             if ((uint32_t)g == h)
                 mypid = pid[g];
-        wmin[lane] = ~0ull;  // slot lane = 16 h + q
-        if (lane == 0)
-            *wcount = 0;
-        wave_lds_order();
 
         // Exact distances of the collected pairs, the running minimum of
         // (distance bits, centroid) per point; order does not matter.
@@ -402,7 +503,7 @@ refine_mfma_kernel(const float *__restrict__ pts, uint64_t n, uint32_t d, uint32
             for (uint32_t r = lane; r < count; r += 64) {
                 const uint32_t pr = pairs[r];
                 const uint32_t slot = pr >> 20, c = pr & 0xFFFFFu;
-                const float e = exact_dist(xs + slot * P, cenT + (uint64_t)c * P, d);
+                const float e = exact_dist(xs + slot * kRow, cenT + (uint64_t)c * P, d);
                 if (e < FLT_MAX)  // the reference's strict '<' from FLT_MAX
                     atomicMin(&wmin[slot], ((unsigned long long)__float_as_uint(e) << 32) | c);
             }
@@ -412,10 +513,10 @@ refine_mfma_kernel(const float *__restrict__ pts, uint64_t n, uint32_t d, uint32
             wave_lds_order();
         };
         const uint32_t last = ntiles - 1;
-        TileOps<NKB> nxt = load_ops<NKB>(table, norm, 0, lane, h);
-        for (uint32_t t = 0; t < ntiles; ++t) {
+        TileOps<NKB> nxt = load_ops<NKB>(table, norm, min(wave, last), lane, h);
+        for (uint32_t t = wave; t < ntiles; t += kRefineWaves) {
             const TileOps<NKB> cur = nxt;
-            nxt = load_ops<NKB>(table, norm, min(t + 1, last), lane, h);
+            nxt = load_ops<NKB>(table, norm, min(t + kRefineWaves, last), lane, h);
             f32v4 acc[kGroups];
             score_tile<FP16, NKB>(acc, cur, w.K, x);
             uint32_t cmask = 0;  // bit 4g + i: (group g's point, centroid t*16 + 4h + i)
@@ -446,18 +547,22 @@ refine_mfma_kernel(const float *__restrict__ pts, uint64_t n, uint32_t d, uint32
             wave_lds_order();
         }
         flush(min(*wcount, kPairCap));
-        const unsigned long long mn = wmin[lane];
-        if (mypid < n)
-            labels[mypid] = (mn == ~0ull) ? 0u : (uint32_t)mn;
-        wave_lds_order();
+        __syncthreads();
+        if (wave == 0) {
+            const unsigned long long mn = wmin[lane];
+            if (mypid < n)
+                labels[mypid] = (mn == ~0ull) ? 0u : (uint32_t)mn;
+        }
+        __syncthreads();  // wmin and xs are free for the next batch
     }
 }
 
 using LabelKernelM = void (*)(const float *, uint64_t, uint32_t, uint32_t, const u16x8 *,
-                              const float *, const float *, uint32_t, MfmaParams, uint32_t *,
-                              uint32_t *, float *, uint32_t *, float *, const u16x8 *, const f32v4 *);
+                              const float *, const TileStats *, uint32_t, MfmaParams, uint32_t *,
+                              uint32_t *, float *, uint32_t *, const float *, float *, int, const u16x8 *,
+                              const f32v4 *);
 using RefineKernelM = void (*)(const float *, uint64_t, uint32_t, uint32_t, const float *,
-                               const u16x8 *, const float *, const float *, uint32_t, MfmaParams,
+                               const u16x8 *, const float *, const TileStats *, uint32_t, MfmaParams,
                                uint32_t *, const uint32_t *, const float *, const uint32_t *);
 
 template <bool FP16, bool FULL>
@@ -473,7 +578,7 @@ void pick_mfma(uint32_t nkb, LabelKernelM &lk, RefineKernelM &rk)
 
 struct MfmaLayout {
     uint32_t ntiles, nkb;
-    size_t table_bytes, norm_bytes, cent_bytes, refine_lds;
+    size_t table_bytes, norm_bytes, cent_bytes, stats_bytes, refine_lds;
 };
 
 MfmaLayout mfma_layout(uint64_t d, uint64_t k)
@@ -484,8 +589,9 @@ MfmaLayout mfma_layout(uint64_t d, uint64_t k)
     l.table_bytes = (size_t)l.ntiles * l.nkb * 64 * sizeof(u16x8);
     l.norm_bytes = (size_t)l.ntiles * kTile * sizeof(float);
     l.cent_bytes = (size_t)l.ntiles * kTile * l.nkb * kKBlock * sizeof(float);
-    l.refine_lds = kRefineWaves * (64 * l.nkb * kKBlock * sizeof(float) + kPairCap * sizeof(uint32_t) +
-                                   64 * sizeof(unsigned long long) + sizeof(uint32_t));
+    l.stats_bytes = (size_t)l.ntiles * sizeof(TileStats) + 64;  // then the queue length
+    l.refine_lds = 64 * (l.nkb * kKBlock + kRowPad) * sizeof(float) + kRefineWaves * (kPairCap + 1) * sizeof(uint32_t) +
+                   64 * sizeof(unsigned long long);
     return l;
 }
 
@@ -530,7 +636,8 @@ bool mfma_labeling_supported(const clk_context *ctx, uint64_t d, uint64_t n, uin
     if (d == 0 || d > (uint64_t)kMaxKb * kKBlock || k == 0 || k > (1u << 20) || n >= (1ull << 32))
         return false;
     const MfmaLayout l = mfma_layout(d, k);
-    return l.table_bytes + 2 * l.norm_bytes <= ctx->lds_per_block && l.refine_lds <= ctx->lds_per_block;
+    const size_t fixed = kStatFloats * sizeof(float);
+    return l.table_bytes + 2 * l.norm_bytes + fixed <= ctx->lds_per_block && l.refine_lds + fixed <= ctx->lds_per_block;
 }
 
 int launch_labeling_mfma(clk_context *ctx, bool fp16, uint64_t d, uint64_t n, uint64_t k,
@@ -540,34 +647,29 @@ int launch_labeling_mfma(clk_context *ctx, bool fp16, uint64_t d, uint64_t n, ui
     CLK_REQUIRE(mfma_labeling_supported(ctx, d, n, k), CLK_ERR_UNSUPPORTED,
                 "MFMA labeling: needs d <= 128, n < 2^32 and a 16-bit centroid table that fits in LDS");
     const MfmaLayout l = mfma_layout(d, k);
-    CLK_TRY(ensure_scratch(ctx->mfma_tables, l.table_bytes + l.norm_bytes + 64 + l.cent_bytes));
+    CLK_TRY(ensure_scratch(ctx->mfma_tables, l.table_bytes + l.norm_bytes + l.cent_bytes + l.stats_bytes));
     CLK_TRY(ensure_scratch(ctx->mfma_queue, std::max<uint64_t>(n, 1) * 2 * sizeof(uint32_t)));
     u16x8 *table = static_cast<u16x8 *>(ctx->mfma_tables.ptr);
     float *norm = reinterpret_cast<float *>(static_cast<char *>(ctx->mfma_tables.ptr) + l.table_bytes);
-    float *stats = norm + (size_t)l.ntiles * kTile;  // 16 floats
-    float *cenT = stats + 16;
-    uint32_t *qlen = reinterpret_cast<uint32_t *>(stats + 4);
+    float *cenT = norm + (size_t)l.ntiles * kTile;
+    TileStats *tiles = reinterpret_cast<TileStats *>(reinterpret_cast<char *>(cenT) + l.cent_bytes);
+    uint32_t *qlen = reinterpret_cast<uint32_t *>(tiles + l.ntiles);
     if (!ctx->mfma_hint.ptr) {  // no offset hint before the first labeling
         CLK_TRY(ensure_scratch(ctx->mfma_hint, 256));
         CLK_TRY(clk_fill_zero(ctx, ctx->mfma_hint.ptr, 256, stream));
     }
-    float *hint = static_cast<float *>(ctx->mfma_hint.ptr);
+    // two words in turn: the last labeling's offset is read while this one's
+    // is recorded
+    ctx->mfma_turn ^= 1;
+    float *hint_out = static_cast<float *>(ctx->mfma_hint.ptr) + ctx->mfma_turn;
+    const float *hint_in = static_cast<float *>(ctx->mfma_hint.ptr) + (ctx->mfma_turn ^ 1);
     uint32_t *qidx = static_cast<uint32_t *>(ctx->mfma_queue.ptr);
     float *qthr = reinterpret_cast<float *>(qidx + std::max<uint64_t>(n, 1));
     ctx->mfma_qlen = qlen;
     {
         KernelTimer t(ctx, "MfmaPrepare", stream);
-        hipLaunchKernelGGL(mfma_prepare_clear_kernel, dim3(1), dim3(64), 0, stream, stats);
-        const uint64_t work = std::max<uint64_t>((uint64_t)l.ntiles * kTile * l.nkb * kKBlock,
-                                                 (uint64_t)l.ntiles * l.nkb * 64);
-        const unsigned pgrid = (unsigned)std::min<uint64_t>(div_up(work, (uint64_t)256), 1024);
-        if (fp16)
-            hipLaunchKernelGGL(mfma_prepare_kernel<true>, dim3(pgrid), dim3(256), 0, stream, centroids,
-                               (uint32_t)d, (uint32_t)k, l.ntiles, l.nkb, table, norm, stats, cenT);
-        else
-            hipLaunchKernelGGL(mfma_prepare_kernel<false>, dim3(pgrid), dim3(256), 0, stream, centroids,
-                               (uint32_t)d, (uint32_t)k, l.ntiles, l.nkb, table, norm, stats, cenT);
-        hipLaunchKernelGGL(mfma_prepare_finish_kernel, dim3(1), dim3(64), 0, stream, stats, hint);
+        hipLaunchKernelGGL(fp16 ? mfma_prepare_kernel<true> : mfma_prepare_kernel<false>, dim3(l.ntiles), dim3(256), 0,
+                           stream, centroids, (uint32_t)d, (uint32_t)k, l.nkb, table, norm, tiles, cenT, qlen, hint_out);
         CLK_HIP_CHECK(hipGetLastError());
     }
     if (n == 0)
@@ -582,7 +684,11 @@ int launch_labeling_mfma(clk_context *ctx, bool fp16, uint64_t d, uint64_t n, ui
         full ? pick_mfma<true, true>(l.nkb, lk, rk) : pick_mfma<true, false>(l.nkb, lk, rk);
     else
         full ? pick_mfma<false, true>(l.nkb, lk, rk) : pick_mfma<false, false>(l.nkb, lk, rk);
-    const size_t lds = l.table_bytes + 2 * l.norm_bytes;  // table, norms, norms + K_L
+    size_t lds = l.table_bytes + 2 * l.norm_bytes;  // table, norms, norms + K_L
+    const size_t qbuf = (size_t)fast_waves((int)l.nkb) * 64 * sizeof(QueueEntry);
+    const int qbuf_ok = lds + qbuf + kStatFloats * sizeof(float) <= ctx->lds_per_block;
+    if (qbuf_ok)
+        lds += qbuf;
     const size_t lds_r = l.refine_lds;
     CLK_HIP_CHECK(allow_lds((const void *)lk, lds));
     CLK_HIP_CHECK(allow_lds((const void *)rk, lds_r));
@@ -597,8 +703,8 @@ int launch_labeling_mfma(clk_context *ctx, bool fp16, uint64_t d, uint64_t n, ui
         const f32v4 *pin_x2 =
             pinned ? reinterpret_cast<const f32v4 *>(pin_ops + pin_ops_count(n, l.nkb)) : nullptr;
         hipLaunchKernelGGL(lk, dim3((unsigned)grid), dim3(fast_block), lds, stream, points, n,
-                           (uint32_t)d, (uint32_t)k, table, norm, stats, l.ntiles, prm, labels,
-                           qidx, qthr, qlen, hint, pin_ops, pin_x2);
+                           (uint32_t)d, (uint32_t)k, table, norm, tiles, l.ntiles, prm, labels,
+                           qidx, qthr, qlen, hint_in, hint_out, qbuf_ok, pin_ops, pin_x2);
         CLK_HIP_CHECK(hipGetLastError());
     }
     // a resident grid; blocks past the queue return at once
@@ -606,7 +712,7 @@ int launch_labeling_mfma(clk_context *ctx, bool fp16, uint64_t d, uint64_t n, ui
     const uint64_t grid_r = auto_grid(ctx, (const void *)rk, refine_block, lds_r, div_up(n, (uint64_t)64) * 64);
     KernelTimer t(ctx, "LabelingMfmaRefine", stream);
     hipLaunchKernelGGL(rk, dim3((unsigned)grid_r), dim3(refine_block), lds_r, stream, points, n,
-                       (uint32_t)d, (uint32_t)k, cenT, table, norm, stats, l.ntiles, prm, labels,
+                       (uint32_t)d, (uint32_t)k, cenT, table, norm, tiles, l.ntiles, prm, labels,
                        qidx, qthr, qlen);
     CLK_HIP_CHECK(hipGetLastError());
     return CLK_OK;

@@ -230,80 +230,85 @@ __device__ __forceinline__ float exact_dist(const float *xrow, const float *__re
     return dist;
 }
 
+// The operands of one point's raw values in this lane (features kb*32 + 8h + j
+// at kb*8 + j); returns X2 >= ||x||^2 (an FP32 sum over the 4 lanes of a point:
+// at most P/4 + 2 roundings, plus underflow).
+template <bool FP16, int NKB>
+__device__ __forceinline__ float build_operands(u16x8 (&ops)[NKB], const float (&raw)[NKB * 8])
+{
+    float s = 0.0f;
+#pragma unroll
+    for (int kb = 0; kb < NKB; ++kb) {
+        u16x8 vb;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float v = raw[kb * 8 + j];
+            s = __builtin_fmaf(v, v, s);
+            vb[j] = to16<FP16>(v);
+        }
+        ops[kb] = vb;
+    }
+    s += xor_swizzle<16>(s);
+    s += __shfl_xor(s, 32);
+    return s * (1.0f + (float)(2 * NKB * kKBlock + 8) * kU) + 1e-37f;
+}
+
+// This lane's values of point pid (features kb*32 + 8h + j at kb*8 + j; 0 past
+// n or d).  Every load address is in bounds (a missing point reads point n-1,
+// a missing feature reads feature 0; the value is then replaced by 0).
+template <int NKB, bool FULL>
+__device__ __forceinline__ void load_raw(float (&raw)[NKB * 8], const float *__restrict__ pts, uint64_t n,
+                                         uint32_t d, uint64_t pid, uint32_t h)
+{
+    const bool valid = pid < n;
+    const uint64_t pc = valid ? pid : n - 1;
+    const float *row = pts + pc + (uint64_t)(8 * h) * n;  // feature 8h
+#pragma unroll
+    for (int kb = 0; kb < NKB; ++kb)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const uint64_t uoff = (uint64_t)(kb * kKBlock + j) * n;
+            if constexpr (FULL) {
+                const float v = row[uoff];
+                raw[kb * 8 + j] = valid ? v : 0.0f;
+            } else {
+                const bool fv = (uint32_t)(kb * kKBlock + 8 * h + j) < d;
+                const float v = *(fv ? row + uoff : pts + pc);
+                raw[kb * 8 + j] = (valid && fv) ? v : 0.0f;
+            }
+        }
+}
+
 // Load the wave's 64 points and build their operands: lane (q, h) handles,
 // for group g, point pid[g] (>= n: none; zeros), features kb*32 + 8h + j
-// (0 past d).  Every load address is in bounds (a missing point reads point
-// n-1, a missing feature reads feature 0; the value is then replaced by 0).
-// X2[g] >= ||x||^2 (an FP32 sum over the 4 lanes of a point: at most P/4 + 2
-// roundings, plus underflow).
+// (0 past d); X2[g] >= ||x||^2.
 template <bool FP16, int NKB, bool FULL, bool KEEP>
 __device__ __forceinline__ void load_points_core(PointOps<NKB> &x, float (&X2)[kGroups],
                                                  const float *__restrict__ pts, uint64_t n,
                                                  uint32_t d, const uint64_t (&pid)[kGroups],
-                                                 uint32_t q, uint32_t h, float *xs,
+                                                 uint32_t q, uint32_t h,
                                                  float (&keep)[kGroups][NKB * 8])
 {
 #pragma unroll
     for (int g = 0; g < kGroups; ++g) {
-        const bool valid = pid[g] < n;
-        const uint64_t pc = valid ? pid[g] : n - 1;
-        const float *row = pts + pc + (uint64_t)(8 * h) * n;  // feature 8h
         float raw[NKB * 8];
-#pragma unroll
-        for (int kb = 0; kb < NKB; ++kb)
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const uint64_t uoff = (uint64_t)(kb * kKBlock + j) * n;
-                if constexpr (FULL) {
-                    const float v = row[uoff];
-                    raw[kb * 8 + j] = valid ? v : 0.0f;
-                } else {
-                    const bool fv = (uint32_t)(kb * kKBlock + 8 * h + j) < d;
-                    const float v = *(fv ? row + uoff : pts + pc);
-                    raw[kb * 8 + j] = (valid && fv) ? v : 0.0f;
-                }
-            }
-        if (xs) {  // row slot 16g + q, features kb*32 + 8h .. +7
-            float *row = xs + (uint32_t)(g * 16 + q) * (NKB * kKBlock) + 8 * h;
-#pragma unroll
-            for (int kb = 0; kb < NKB; ++kb) {
-                *reinterpret_cast<f32v4 *>(row + kb * kKBlock) =
-                    f32v4{raw[kb * 8 + 0], raw[kb * 8 + 1], raw[kb * 8 + 2], raw[kb * 8 + 3]};
-                *reinterpret_cast<f32v4 *>(row + kb * kKBlock + 4) =
-                    f32v4{raw[kb * 8 + 4], raw[kb * 8 + 5], raw[kb * 8 + 6], raw[kb * 8 + 7]};
-            }
-        }
+        load_raw<NKB, FULL>(raw, pts, n, d, pid[g], h);
         if constexpr (KEEP) {
 #pragma unroll
             for (int j = 0; j < NKB * 8; ++j)
                 keep[g][j] = raw[j];
         }
-        float s = 0.0f;
-#pragma unroll
-        for (int kb = 0; kb < NKB; ++kb) {
-            u16x8 vb;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float v = raw[kb * 8 + j];
-                s = __builtin_fmaf(v, v, s);
-                vb[j] = to16<FP16>(v);
-            }
-            x.b[g][kb] = vb;
-        }
-        s += xor_swizzle<16>(s);
-        s += __shfl_xor(s, 32);
-        X2[g] = s * (1.0f + (float)(2 * NKB * kKBlock + 8) * kU) + 1e-37f;
+        X2[g] = build_operands<FP16, NKB>(x.b[g], raw);
     }
 }
 
 template <bool FP16, int NKB, bool FULL>
 __device__ __forceinline__ void load_points(PointOps<NKB> &x, float (&X2)[kGroups],
                                             const float *__restrict__ pts, uint64_t n, uint32_t d,
-                                            const uint64_t (&pid)[kGroups], uint32_t q, uint32_t h,
-                                            float *xs = nullptr)
+                                            const uint64_t (&pid)[kGroups], uint32_t q, uint32_t h)
 {
     float unused[kGroups][NKB * 8];
-    load_points_core<FP16, NKB, FULL, false>(x, X2, pts, n, d, pid, q, h, xs, unused);
+    load_points_core<FP16, NKB, FULL, false>(x, X2, pts, n, d, pid, q, h, unused);
 }
 
 // As load_points, and keep[g][kb*8 + j] = the FP32 value of feature
@@ -315,7 +320,7 @@ __device__ __forceinline__ void load_points_keep(PointOps<NKB> &x, float (&X2)[k
                                                  uint32_t q, uint32_t h,
                                                  float (&keep)[kGroups][NKB * 8])
 {
-    load_points_core<FP16, NKB, FULL, true>(x, X2, pts, n, d, pid, q, h, nullptr, keep);
+    load_points_core<FP16, NKB, FULL, true>(x, X2, pts, n, d, pid, q, h, keep);
 }
 
 // The loads of load_points alone, for software pipelining: raw[g][kb*8 + j]

@@ -177,6 +177,18 @@ __global__ void __launch_bounds__(1024) reduce_cols_kernel(const T *in, uint64_t
     }
 }
 
+// centroids[f,c] = (float)(sums[f,c] / (double)masses[c]) without a shift: a
+// work-item per value (one work-group over all of them, below, takes 26 us at
+// d=64 k=1024).
+__global__ void __launch_bounds__(256) divide_values_kernel(const double *__restrict__ sums,
+                                                            const uint32_t *__restrict__ masses, uint32_t count,
+                                                            uint32_t k, float *__restrict__ cen)
+{
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i < count)
+        cen[i] = (float)(sums[i] / (double)masses[i % k]);
+}
+
 // centroids[f,c] = (float)(sums[f,c] / (double)masses[c]); optional max
 // centroid shift (FP64) over non-empty clusters.  One block.
 __global__ void __launch_bounds__(1024) divide_kernel(const double *__restrict__ sums,
@@ -625,6 +637,12 @@ extern "C" int clk_matrix_divide_row(clk_context *ctx, uint64_t d, uint64_t k,
                 "divide: old_centroids must not alias centroids");
     hipStream_t s = as_stream(stream);
     KernelTimer t(ctx, "MatrixBinaryOpRow", s);
+    if (!old_centroids || !max_shift) {
+        hipLaunchKernelGGL(divide_values_kernel, dim3((unsigned)div_up(d * k, 256)), dim3(256), 0, s, sums, masses,
+                           (uint32_t)(d * k), (uint32_t)k, centroids);
+        CLK_HIP_CHECK(hipGetLastError());
+        return CLK_OK;
+    }
     unsigned block = 64;
     while (block < 1024 && block < k)
         block *= 2;  // power of two for the tree reduction
