@@ -93,7 +93,7 @@ struct BJob {
     uint32_t bound_ok;
     float *lb;
     float drift;
-    uint32_t pad1;
+    uint32_t keep_due;  // 1: batch_keep_kernel computes the thresholds after this iteration's finish
     // MFMA jobs with d <= 32: the current centroids as rows [k][cen_t_w]
     // (zero-padded to 4/8/16/32 floats), refreshed by the finish kernel, for
     // the keep test and the exact rescan of the tile kernel
@@ -797,10 +797,12 @@ __device__ __forceinline__ double keep_min_rows(const float *__restrict__ cs, ui
 }
 
 // rows_out (optional): the staged rows also written to global memory.
-// thresholds = false: only the rows.
+// thresholds = false: only the rows.  The thresholds of the blocks of 64
+// centroids [first_block, first_block + blocks).
 __device__ __forceinline__ void build_keep_thresholds(const float *__restrict__ cen, uint32_t d, uint32_t k,
                                       float *__restrict__ keep, float *cs, double *red,
-                                      float *__restrict__ rows_out = nullptr, bool thresholds = true)
+                                      float *__restrict__ rows_out, bool thresholds, uint32_t first_block,
+                                      uint32_t blocks)
 {
     const uint32_t tid = threadIdx.x, lane = tid % 64, wave = tid / 64, W = blockDim.x / 64;
     const uint32_t db = keep_row_width(d);
@@ -815,9 +817,9 @@ __device__ __forceinline__ void build_keep_thresholds(const float *__restrict__ 
     __syncthreads();
     if (!thresholds)
         return;
-    const uint32_t nab = (k + 63) / 64;
-    const uint32_t slices = nab >= W ? 1u : W / nab;
-    for (uint32_t ab0 = 0; ab0 < nab; ab0 += W / slices) {
+    const uint32_t slices = blocks >= W ? 1u : W / blocks;
+    const uint32_t nab = first_block + blocks;
+    for (uint32_t ab0 = first_block; ab0 < nab; ab0 += W / slices) {
         const uint32_t ab = ab0 + wave / slices, sl = wave % slices;
         const uint32_t a = ab * 64 + lane;
         const bool mine = ab < nab && a < k;
@@ -865,20 +867,24 @@ __device__ void batch_finalize(BJob &J, double *red)
     float *nxt = J.cen[(J.iter & 1) ^ 1];
     double local = 0.0, moved = 0.0;
     const bool special = J.gmax[d] != 0;  // the job holds NaN / inf: flags may be set
+    // the quotients, a value per lane
+    for (uint32_t i = tid; i < d * k; i += blockDim.x) {
+        // exact sums, or NaN / inf where off-grid values were flagged (the
+        // flags are cleared for the next iteration)
+        const uint32_t fl = special ? J.flags[i] : 0u;
+        if (fl)
+            J.flags[i] = 0u;
+        nxt[i] = (float)((fl ? special_value(fl) : tot[i]) / tot[(size_t)k * d + i % k]);
+    }
+    __syncthreads();
     for (uint32_t c = tid; c < k; c += blockDim.x) {
         const double m = tot[(size_t)k * d + c];
         double sq = 0.0;
         bool fin_new = true, fin_old = true;
+#pragma unroll 8
         for (uint32_t f = 0; f < d; ++f) {
-            // exact sums, or NaN / inf where off-grid values were flagged
-            // (the flags are cleared for the next iteration)
-            const size_t i = (size_t)f * k + c;
-            const uint32_t fl = special ? J.flags[i] : 0u;
-            if (fl)
-                J.flags[i] = 0u;
-            const float v = (float)((fl ? special_value(fl) : tot[i]) / m);
+            const float v = nxt[(size_t)f * k + c];
             const float o = old[(size_t)f * k + c];
-            nxt[(size_t)f * k + c] = v;
             const double diff = (double)v - (double)o;
             sq += diff * diff;
             fin_new = fin_new && __builtin_isfinite(v);
@@ -962,11 +968,15 @@ __device__ __forceinline__ void for_each_tile(const BJob *__restrict__ jobs, con
     }
 }
 
+// The most waves of a tile's work-group whose registers fit; rebuild launches
+// kBatchMaxWaves unless the class has few tiles.
+__host__ __device__ constexpr uint32_t wide_waves(uint32_t dm) { return dm <= 16 ? 16 : dm <= 32 ? 8 : kBatchMaxWaves; }
+
 // Tiles of the jobs of one size class (FP32 labeling, d <= DMAX).
-// d <= 32: at most 168 VGPRs, so three work-groups fit per CU (the
-// prefetched and the current point's 32 features are both live).
+// d <= 32: at most 168 VGPRs, so three work-groups of four waves fit per CU
+// (the prefetched and the current point's 32 features are both live).
 template <int DMAX>
-__global__ void __launch_bounds__(64 * kBatchMaxWaves, DMAX == 32 ? 3 : 1)
+__global__ void __launch_bounds__(64 * wide_waves(DMAX), DMAX == 32 ? 3 : 1)
 batch_tiles_kernel(const BJob *__restrict__ jobs, const BTile *__restrict__ tiles, BCtl *__restrict__ ctl)
 {
     extern __shared__ __align__(16) float lds[];
@@ -978,6 +988,20 @@ batch_tiles_kernel(const BJob *__restrict__ jobs, const BTile *__restrict__ tile
             batch_tile<DMAX, false>(J, index, lds, waves);
         __syncthreads();  // the tables are cleared for the next tile
     });
+}
+
+// The tile kernel of an FP32 size class (c / 2).
+using TilesKernel = void (*)(const BJob *, const BTile *, BCtl *);
+TilesKernel fp32_tiles_kernel(uint32_t bucket)
+{
+    switch (bucket) {
+    case 0: return batch_tiles_kernel<3>;
+    case 1: return batch_tiles_kernel<4>;
+    case 2: return batch_tiles_kernel<8>;
+    case 3: return batch_tiles_kernel<16>;
+    case 4: return batch_tiles_kernel<32>;
+    default: return batch_tiles_kernel<64>;
+    }
 }
 
 // Read in place of a missing point or feature (the loads need no masks).
@@ -1379,12 +1403,28 @@ struct BStatus {
     double shift;
 };
 
+constexpr uint32_t kFinishThreads = 1024;
+
+// Jobs whose keep thresholds have a launch of their own: at 2^18 differences
+// one work-group takes as long as that launch.
+__host__ __device__ inline bool keep_apart(uint32_t d, uint32_t k) { return (uint64_t)k * k * d >= 1u << 18; }
+
+// Whether a job's tiles take the keep test (the finish keeps its thresholds).
+__host__ __device__ inline bool keeps_labels(uint32_t kind, uint32_t d, uint32_t k, uint32_t cen_t_w)
+{
+    return kind == 0 ? k >= kKeepMinK || k * d >= kKeepMinKd : cen_t_w != 0 && (uint64_t)k * cen_t_w <= kKeepStage;
+}
+
+struct BKeepUnit {
+    uint32_t job, block;
+};
+
 template <bool FP16>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(kFinishThreads)
 batch_finish_kernel(BJob *__restrict__ jobs, const uint32_t *__restrict__ active, BCtl *__restrict__ ctl,
                     BStatus *__restrict__ status)
 {
-    __shared__ double red[256];
+    __shared__ double red[kFinishThreads];
     __shared__ float cs[kKeepStage];
     if (blockIdx.x == 0 && threadIdx.x < kClasses)
         ctl[threadIdx.x].next = 0;
@@ -1407,17 +1447,37 @@ batch_finish_kernel(BJob *__restrict__ jobs, const uint32_t *__restrict__ active
     // hide only a cluster that turned empty (finite -> NaN), whose old
     // centroid in the minimum only makes the other thresholds smaller.
     // MFMA jobs with d <= 32 also get their centroid rows every iteration.
-    const bool fp32_keep = J.kind == 0 && (J.k >= kKeepMinK || J.k * J.d >= kKeepMinKd);
-    const bool mfma_keep = J.kind == 1 && J.cen_t_w != 0 && (uint64_t)J.k * J.cen_t_w <= kKeepStage;
-    if (J.state == CLK_JOB_ACTIVE && (fp32_keep || mfma_keep)) {
-        const bool thr = !(J.keep_ok && J.shift == 0.0);
-        if (thr || mfma_keep) {
-            __syncthreads();
-            build_keep_thresholds(J.cen[nxt], J.d, J.k, J.keep, cs, red, mfma_keep ? J.cen_t : nullptr, thr);
-        }
-        if (threadIdx.x == 0)
+    const bool fp32_keep = J.kind == 0 && keeps_labels(J.kind, J.d, J.k, J.cen_t_w);
+    const bool mfma_keep = J.kind == 1 && keeps_labels(J.kind, J.d, J.k, J.cen_t_w);
+    const bool keeps = J.state == CLK_JOB_ACTIVE && (fp32_keep || mfma_keep);
+    const bool due = keeps && !(J.keep_ok && J.shift == 0.0);
+    const bool apart = keep_apart(J.d, J.k);  // batch_keep_kernel computes the thresholds
+    __syncthreads();  // every lane has read the record
+    if (keeps && ((due && !apart) || mfma_keep))
+        build_keep_thresholds(J.cen[nxt], J.d, J.k, J.keep, cs, red, mfma_keep ? J.cen_t : nullptr, due && !apart, 0,
+                              (J.k + 63) / 64);
+    if (threadIdx.x == 0) {
+        J.keep_due = due && apart;
+        if (keeps)
             J.keep_ok = 1;
     }
+}
+
+// The keep thresholds of the jobs with many clusters (keep_apart), a
+// work-group per 64 centroids: k^2 d FP64 differences took one work-group per
+// job 95 us of a 440 us iteration (k = 256, d = 32; finish and this now 24 and
+// 20-30 us).
+__global__ void __launch_bounds__(kFinishThreads)
+batch_keep_kernel(const BJob *__restrict__ jobs, const BKeepUnit *__restrict__ units, const BCtl *__restrict__ ctl)
+{
+    __shared__ double red[kFinishThreads];
+    __shared__ float cs[kKeepStage];
+    if (ctl[0].dry != 0)
+        return;
+    const BKeepUnit u = units[blockIdx.x];
+    const BJob &J = jobs[u.job];
+    if (J.keep_due)
+        build_keep_thresholds(J.cen[J.iter & 1], J.d, J.k, J.keep, cs, red, nullptr, true, u.block, 1);
 }
 
 // Result copies of the serving loop: one work-group per (source, words,
@@ -1433,6 +1493,27 @@ __global__ void __launch_bounds__(256) gather_kernel(const GatherDesc *__restric
     const GatherDesc g = descs[blockIdx.x];
     for (uint64_t i = threadIdx.x; i < g.words; i += blockDim.x)
         g.dst[i] = g.src[i];
+}
+
+// Admission of a round of jobs (serving), a work-group per job: the initial
+// centroids out of device-mapped pinned host memory, the flags and the grid
+// cleared (launch_grid_max_units fills it next).
+struct AdmitDesc {
+    const float *src;
+    float *cen;
+    uint32_t *flags, *gmax;
+    uint32_t dk, d;
+};
+
+__global__ void __launch_bounds__(256) admit_kernel(const AdmitDesc *__restrict__ descs)
+{
+    const AdmitDesc a = descs[blockIdx.x];
+    for (uint32_t i = threadIdx.x; i < a.dk; i += blockDim.x) {
+        a.cen[i] = a.src[i];
+        a.flags[i] = 0u;
+    }
+    for (uint32_t i = threadIdx.x; i <= a.d; i += blockDim.x)
+        a.gmax[i] = 0u;
 }
 
 // Activation of staged jobs (serving): one work-group per slot copies the
@@ -1498,6 +1579,7 @@ size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 using clk::BCtl;
 using clk::BJob;
+using clk::BKeepUnit;
 using clk::BMergeUnit;
 using clk::BTile;
 
@@ -1516,15 +1598,19 @@ struct clk_batch {
     clk_batch_config cfg{};
     bool mfma = false, fp16 = false;
     BJob *d_jobs = nullptr;
+    // what an iteration's launches read, rewritten by rebuild: one device
+    // buffer (d_plan) and its pinned staging copy
+    char *d_plan = nullptr, *h_plan = nullptr;
+    size_t plan_cap = 0;
+    hipEvent_t plan_copied = nullptr;
     BCtl *d_ctl = nullptr;  // one per class
     BTile *d_tiles = nullptr;
-    uint32_t tile_cap = 0;
     uint32_t *d_active = nullptr;  // slots of the active jobs (finish work-groups)
     uint32_t nactive = 0;
     clk::BMergeUnit *d_units = nullptr;  // merge work-groups
-    uint32_t nunits = 0, unit_cap = 0;
-    uint32_t *d_retile = nullptr;  // (slot, tile_pts, ntiles) of jobs rebuild re-tiled
-    uint32_t retile_cap = 0;
+    uint32_t nunits = 0;
+    clk::BKeepUnit *d_keeps = nullptr;  // work-groups of the apart keep thresholds
+    uint32_t nkeeps = 0;
     char *arena = nullptr;
     // host mirror of the job table (device-side fields iter/state/shift are
     // read back by poll / take)
@@ -1549,6 +1635,10 @@ struct clk_batch {
     // status of every slot after its last iteration, written by the finish
     // kernel (pinned, device-mapped): the serving loop reads it in place
     clk::BStatus *h_status = nullptr, *h_status_dev = nullptr;
+    // the admissions of a serving round (pinned, device-mapped; RoundBuffer's
+    // layout) and the end of the kernels that read it last
+    char *h_round = nullptr, *h_round_dev = nullptr;
+    hipEvent_t round_done = nullptr;
 };
 
 namespace {
@@ -1659,16 +1749,8 @@ uint32_t class_of(uint32_t kind, uint32_t d, uint32_t k)
 
 const void *class_kernel(const clk_batch *b, uint32_t c)
 {
-    if (c < clk::kMfmaClass0) {
-        switch (c / 2) {
-        case 0: return (const void *)clk::batch_tiles_kernel<3>;
-        case 1: return (const void *)clk::batch_tiles_kernel<4>;
-        case 2: return (const void *)clk::batch_tiles_kernel<8>;
-        case 3: return (const void *)clk::batch_tiles_kernel<16>;
-        case 4: return (const void *)clk::batch_tiles_kernel<32>;
-        default: return (const void *)clk::batch_tiles_kernel<64>;
-        }
-    }
+    if (c < clk::kMfmaClass0)
+        return (const void *)clk::fp32_tiles_kernel(c / 2);
     const bool nkb2 = c >= clk::kMfmaNkb2Class;
     if (b->fp16)
         return nkb2 ? (const void *)clk::batch_tiles_mfma_kernel<true, 2>
@@ -1782,6 +1864,23 @@ int rebuild(clk_batch *b, hipStream_t stream)
             if (!shrunk)
                 break;
         }
+        // No more tiles than resident work-groups: the class takes as long as
+        // one tile, so a tile gets twice the waves, and all that its registers
+        // allow when there are no more tiles than CUs (serving 128 jobs, n up
+        // to 2^16, d 3-32, k 4-256: d <= 3 tiles 52 -> 35 us with twice the
+        // waves, 45 -> 14 us with four times).
+        if (c < clk::kMfmaClass0 && total <= resident) {
+            const uint32_t most = clk::wide_waves(clk::kFp32Dmax[c / 2]);
+            const uint32_t wide =
+                total <= (uint64_t)b->ctx->num_cus ? most : std::min(most, 2 * clk::kBatchMaxWaves);
+            const size_t lds = class_lds(c, wide, kmax, kdmax, dmax, nullptr);
+            if (wide > C.waves && lds + 4096 <= b->ctx->lds_per_block) {
+                C.waves = wide;
+                C.lds = lds;
+                if (lds > 65536)
+                    CLK_HIP_CHECK(hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+            }
+        }
         for (size_t i = 0; i < mem.size(); ++i) {
             const uint32_t s = mem[i];
             BJob &J = b->jobs[s];
@@ -1800,33 +1899,6 @@ int rebuild(clk_batch *b, hipStream_t stream)
         C.grid = (uint32_t)clk::auto_grid(b->ctx, kern, (int)(64 * C.waves), C.lds,
                                           (uint64_t)C.ntiles * 64 * C.waves);
     }
-    if (!retile.empty()) {  // the device records' tiling
-        const uint32_t count = (uint32_t)(retile.size() / 3);
-        if (retile.size() > b->retile_cap) {
-            if (b->d_retile)
-                CLK_HIP_CHECK(hipFree(b->d_retile));
-            b->retile_cap = (uint32_t)std::max<size_t>(retile.size(), 3 * 1024) * 2;
-            CLK_HIP_CHECK(hipMalloc(&b->d_retile, b->retile_cap * sizeof(uint32_t)));
-        }
-        CLK_HIP_CHECK(hipMemcpyAsync(b->d_retile, retile.data(), retile.size() * sizeof(uint32_t),
-                                     hipMemcpyHostToDevice, stream));
-        hipLaunchKernelGGL(clk::batch_retile_kernel, dim3((count + 255) / 256), dim3(256), 0, stream, b->d_jobs,
-                           b->d_retile, count);
-        CLK_HIP_CHECK(hipGetLastError());
-    }
-    if (tiles.size() > b->tile_cap) {
-        if (b->d_tiles)
-            CLK_HIP_CHECK(hipFree(b->d_tiles));
-        b->tile_cap = (uint32_t)std::max<size_t>(tiles.size(), 1024) * 2;
-        CLK_HIP_CHECK(hipMalloc(&b->d_tiles, b->tile_cap * sizeof(BTile)));
-    }
-    if (!tiles.empty())
-        CLK_HIP_CHECK(hipMemcpyAsync(b->d_tiles, tiles.data(), tiles.size() * sizeof(BTile),
-                                     hipMemcpyHostToDevice, stream));
-    if (!active.empty())
-        CLK_HIP_CHECK(hipMemcpyAsync(b->d_active, active.data(), active.size() * sizeof(uint32_t),
-                                     hipMemcpyHostToDevice, stream));
-    b->nactive = (uint32_t)active.size();
     std::vector<BMergeUnit> units;
     for (uint32_t s : active) {
         const BJob &J = b->jobs[s];
@@ -1840,18 +1912,64 @@ int rebuild(clk_batch *b, hipStream_t stream)
         for (uint32_t e0 = 0; e0 < rl; e0 += per)
             units.push_back({s, e0});
     }
-    if (units.size() > b->unit_cap) {
-        if (b->d_units)
-            CLK_HIP_CHECK(hipFree(b->d_units));
-        b->unit_cap = (uint32_t)std::max<size_t>(units.size(), 1024) * 2;
-        CLK_HIP_CHECK(hipMalloc(&b->d_units, b->unit_cap * sizeof(BMergeUnit)));
+    std::vector<BKeepUnit> keeps;
+    for (uint32_t s : active) {
+        const BJob &J = b->jobs[s];
+        if (clk::keep_apart(J.d, J.k) && clk::keeps_labels(J.kind, J.d, J.k, J.cen_t_w))
+            for (uint32_t block = 0; block < clk::div_up(J.k, 64); ++block)
+                keeps.push_back({s, block});
     }
-    if (!units.empty())
-        CLK_HIP_CHECK(hipMemcpyAsync(b->d_units, units.data(), units.size() * sizeof(BMergeUnit),
-                                     hipMemcpyHostToDevice, stream));
+    // one copy of all of it (a copy each took 10-15 us of an iteration's
+    // start, five times)
+    size_t bytes = 0;
+    auto place = [&](const auto &v) {
+        const size_t at = bytes;
+        bytes += clk::align_up(v.size() * sizeof(v[0]), 256);
+        return at;
+    };
+    const size_t at_ctl = place(ctl), at_tiles = place(tiles), at_active = place(active), at_units = place(units),
+                 at_keeps = place(keeps), at_retile = place(retile);
+    // the last copy may still read h_plan (on another stream too)
+    CLK_HIP_CHECK(hipStreamSynchronize(stream));
+    CLK_HIP_CHECK(hipEventSynchronize(b->plan_copied));
+    if (bytes > b->plan_cap) {
+        if (b->d_plan)
+            (void)hipFree(b->d_plan);
+        if (b->h_plan)
+            (void)hipHostFree(b->h_plan);
+        b->d_plan = b->h_plan = nullptr;
+        b->plan_cap = 0;
+        const size_t cap = std::max<size_t>(2 * bytes, 1u << 16);
+        CLK_HIP_CHECK(hipMalloc((void **)&b->d_plan, cap));
+        CLK_HIP_CHECK(hipHostMalloc((void **)&b->h_plan, cap, hipHostMallocDefault));
+        b->plan_cap = cap;
+    }
+    auto put = [&](const auto &v, size_t at) {
+        if (!v.empty())
+            std::memcpy(b->h_plan + at, v.data(), v.size() * sizeof(v[0]));
+    };
+    put(ctl, at_ctl);
+    put(tiles, at_tiles);
+    put(active, at_active);
+    put(units, at_units);
+    put(keeps, at_keeps);
+    put(retile, at_retile);
+    b->d_ctl = reinterpret_cast<BCtl *>(b->d_plan + at_ctl);
+    b->d_tiles = reinterpret_cast<BTile *>(b->d_plan + at_tiles);
+    b->d_active = reinterpret_cast<uint32_t *>(b->d_plan + at_active);
+    b->d_units = reinterpret_cast<BMergeUnit *>(b->d_plan + at_units);
+    b->d_keeps = reinterpret_cast<BKeepUnit *>(b->d_plan + at_keeps);
+    b->nactive = (uint32_t)active.size();
     b->nunits = (uint32_t)units.size();
-    CLK_HIP_CHECK(hipMemcpyAsync(b->d_ctl, ctl.data(), ctl.size() * sizeof(BCtl), hipMemcpyHostToDevice, stream));
-    CLK_HIP_CHECK(hipStreamSynchronize(stream));  // tiles / ctl are host temporaries
+    b->nkeeps = (uint32_t)keeps.size();
+    CLK_HIP_CHECK(hipMemcpyAsync(b->d_plan, b->h_plan, bytes, hipMemcpyHostToDevice, stream));
+    CLK_HIP_CHECK(hipEventRecord(b->plan_copied, stream));
+    if (!retile.empty()) {  // the device records' tiling
+        const uint32_t count = (uint32_t)(retile.size() / 3);
+        hipLaunchKernelGGL(clk::batch_retile_kernel, dim3((count + 255) / 256), dim3(256), 0, stream, b->d_jobs,
+                           reinterpret_cast<uint32_t *>(b->d_plan + at_retile), count);
+        CLK_HIP_CHECK(hipGetLastError());
+    }
     if (b->exec) {
         (void)hipGraphExecDestroy(b->exec);
         b->exec = nullptr;
@@ -1873,8 +1991,14 @@ int rebuild(clk_batch *b, hipStream_t stream)
 int launch_step(clk_batch *b, hipStream_t stream_main)
 {
     uint32_t used = 0;  // side streams forked so far
-    uint32_t nlaunched = 0;
-    for (uint32_t c = 0; c < clk::kClasses; ++c) {
+    uint32_t nlaunched = 0, nclasses = 0;
+    for (uint32_t c = 0; c < clk::kClasses; ++c)
+        nclasses += b->cls[c].ntiles != 0;
+    if (nclasses > 1)  // before the first class: the others do not wait for it
+        CLK_HIP_CHECK(hipEventRecord(b->fork, stream_main));
+    // the widest classes first: their tiles take longest
+    for (uint32_t r = 0; r < clk::kClasses; ++r) {
+        const uint32_t c = clk::kClasses - 1 - r;
         const BClassState &C = b->cls[c];
         if (C.ntiles == 0)
             continue;
@@ -1884,8 +2008,6 @@ int launch_step(clk_batch *b, hipStream_t stream_main)
         if (slot != 0) {
             const uint32_t si = slot - 1;
             if (si >= used) {
-                if (used == 0)
-                    CLK_HIP_CHECK(hipEventRecord(b->fork, stream_main));
                 CLK_HIP_CHECK(hipStreamWaitEvent(b->side[si], b->fork, 0));
                 used = si + 1;
             }
@@ -1895,14 +2017,7 @@ int launch_step(clk_batch *b, hipStream_t stream_main)
         BCtl *ctl = b->d_ctl + c;
         const dim3 g(C.grid), t(64 * C.waves);
         if (c < clk::kMfmaClass0) {
-            switch (c / 2) {
-            case 0: hipLaunchKernelGGL(clk::batch_tiles_kernel<3>, g, t, C.lds, stream, b->d_jobs, tl, ctl); break;
-            case 1: hipLaunchKernelGGL(clk::batch_tiles_kernel<4>, g, t, C.lds, stream, b->d_jobs, tl, ctl); break;
-            case 2: hipLaunchKernelGGL(clk::batch_tiles_kernel<8>, g, t, C.lds, stream, b->d_jobs, tl, ctl); break;
-            case 3: hipLaunchKernelGGL(clk::batch_tiles_kernel<16>, g, t, C.lds, stream, b->d_jobs, tl, ctl); break;
-            case 4: hipLaunchKernelGGL(clk::batch_tiles_kernel<32>, g, t, C.lds, stream, b->d_jobs, tl, ctl); break;
-            default: hipLaunchKernelGGL(clk::batch_tiles_kernel<64>, g, t, C.lds, stream, b->d_jobs, tl, ctl); break;
-            }
+            hipLaunchKernelGGL(clk::fp32_tiles_kernel(c / 2), g, t, C.lds, stream, b->d_jobs, tl, ctl);
         } else if (b->fp16) {
             if (c >= clk::kMfmaNkb2Class)
                 hipLaunchKernelGGL((clk::batch_tiles_mfma_kernel<true, 2>), g, t, C.lds, stream, b->d_jobs, tl,
@@ -1930,13 +2045,18 @@ int launch_step(clk_batch *b, hipStream_t stream_main)
                            b->d_units, b->d_ctl);
         CLK_HIP_CHECK(hipGetLastError());
     }
-    const dim3 fg(std::max<uint32_t>(b->nactive, 1)), fb(256);
+    const dim3 fg(std::max<uint32_t>(b->nactive, 1)), fb(clk::kFinishThreads);
     if (b->fp16)
         hipLaunchKernelGGL(clk::batch_finish_kernel<true>, fg, fb, 0, stream, b->d_jobs, b->d_active, b->d_ctl,
                            b->h_status_dev);
     else
         hipLaunchKernelGGL(clk::batch_finish_kernel<false>, fg, fb, 0, stream, b->d_jobs, b->d_active, b->d_ctl,
                            b->h_status_dev);
+    if (b->nkeeps > 0) {
+        CLK_HIP_CHECK(hipGetLastError());
+        hipLaunchKernelGGL(clk::batch_keep_kernel, dim3(b->nkeeps), dim3(clk::kFinishThreads), 0, stream, b->d_jobs,
+                           b->d_keeps, b->d_ctl);
+    }
     CLK_HIP_CHECK(hipGetLastError());
     return CLK_OK;
 }
@@ -1994,20 +2114,18 @@ extern "C" int clk_batch_create(clk_context *ctx, const clk_batch_config *cfg, c
     b->off.assign(cfg->max_jobs, 0);
     b->bytes.assign(cfg->max_jobs, 0);
     hipError_t e1 = hipMalloc(&b->d_jobs, cfg->max_jobs * sizeof(BJob));
-    hipError_t e2 = hipMalloc(&b->d_ctl, clk::kClasses * sizeof(BCtl));
-    hipError_t e3 = hipMalloc(&b->arena, cfg->arena_bytes);
-    hipError_t e4 = hipMalloc(&b->d_active, cfg->max_jobs * sizeof(uint32_t));
-    hipError_t e5 = hipHostMalloc((void **)&b->h_status, cfg->max_jobs * sizeof(clk::BStatus), hipHostMallocDefault);
-    if (e5 == hipSuccess)
-        e5 = hipHostGetDevicePointer((void **)&b->h_status_dev, b->h_status, 0);
-    if (e1 != hipSuccess || e2 != hipSuccess || e3 != hipSuccess || e4 != hipSuccess || e5 != hipSuccess) {
+    hipError_t e2 = hipMalloc(&b->arena, cfg->arena_bytes);
+    hipError_t e3 = hipHostMalloc((void **)&b->h_status, cfg->max_jobs * sizeof(clk::BStatus), hipHostMallocDefault);
+    if (e3 == hipSuccess)
+        e3 = hipHostGetDevicePointer((void **)&b->h_status_dev, b->h_status, 0);
+    if (e1 != hipSuccess || e2 != hipSuccess || e3 != hipSuccess) {
         clk_batch_destroy(b);
         clk::set_error("clk_batch_create: device allocation failed");
         return CLK_ERR_NOMEM;
     }
     CLK_HIP_CHECK(hipMemset(b->d_jobs, 0, cfg->max_jobs * sizeof(BJob)));
-    CLK_HIP_CHECK(hipMemset(b->d_ctl, 0, clk::kClasses * sizeof(BCtl)));
-    bool ok = hipEventCreateWithFlags(&b->fork, hipEventDisableTiming) == hipSuccess;
+    bool ok = hipEventCreateWithFlags(&b->fork, hipEventDisableTiming) == hipSuccess &&
+              hipEventCreateWithFlags(&b->plan_copied, hipEventDisableTiming) == hipSuccess;
     for (int i = 0; i < clk_batch::kSide && ok; ++i)
         ok = hipStreamCreateWithFlags(&b->side[i], hipStreamNonBlocking) == hipSuccess &&
              hipEventCreateWithFlags(&b->join[i], hipEventDisableTiming) == hipSuccess;
@@ -2032,18 +2150,18 @@ extern "C" int clk_batch_destroy(clk_batch *b)
         (void)hipGraphDestroy(b->graph);
     if (b->d_jobs)
         (void)hipFree(b->d_jobs);
-    if (b->d_ctl)
-        (void)hipFree(b->d_ctl);
-    if (b->d_tiles)
-        (void)hipFree(b->d_tiles);
-    if (b->d_active)
-        (void)hipFree(b->d_active);
-    if (b->d_units)
-        (void)hipFree(b->d_units);
-    if (b->d_retile)
-        (void)hipFree(b->d_retile);
+    if (b->plan_copied)
+        (void)hipEventDestroy(b->plan_copied);
+    if (b->d_plan)
+        (void)hipFree(b->d_plan);
+    if (b->h_plan)
+        (void)hipHostFree(b->h_plan);
     if (b->h_rec)
         (void)hipHostFree(b->h_rec);
+    if (b->h_round) {
+        (void)hipEventDestroy(b->round_done);
+        (void)hipHostFree(b->h_round);
+    }
     if (b->h_status)
         (void)hipHostFree(b->h_status);
     if (b->arena)
@@ -2069,9 +2187,62 @@ namespace {
 // Stage a job: a free slot and arena range, the job record, and the copies of
 // its points and initial centroids (async on stream).  The slot is not yet
 // visible to the kernels.
+// The device side of a serving round's admissions, collected by stage_job and
+// launched once for all of them: by itself each job takes a copy of its
+// centroids, three fills and the pass over its points for the sum grid, about
+// 35 us of calls (128 jobs in one round, traced: 7.3 -> 0.6 ms).  Jobs beyond the buffer, and
+// all while the last round's kernels may still read it, are prepared singly.
+struct AdmitRound {
+    static constexpr size_t kDescs = 1024, kUnits = 8192, kFloats = 1u << 17;
+    static constexpr size_t kUnitsAt = kDescs * sizeof(clk::AdmitDesc),
+                            kFloatsAt = kUnitsAt + kUnits * sizeof(clk::GridUnit),
+                            kBytes = kFloatsAt + kFloats * sizeof(float);
+    clk_batch *b;
+    bool open;
+    size_t descs = 0, units = 0, floats = 0;
+
+    explicit AdmitRound(clk_batch *batch)
+        : b(batch), open(batch->h_round != nullptr && hipEventQuery(batch->round_done) == hipSuccess)
+    {
+    }
+    // false: no room
+    bool add(const BJob &J, const float *host_centroids)
+    {
+        const size_t dk = (size_t)J.d * J.k, nu = clk::div_up(J.n, clk::kGridUnitValues) * J.d;
+        if (!open || descs == kDescs || units + nu > kUnits || floats + dk > kFloats)
+            return false;
+        const size_t at = kFloatsAt + floats * sizeof(float);
+        std::memcpy(b->h_round + at, host_centroids, dk * sizeof(float));
+        reinterpret_cast<clk::AdmitDesc *>(b->h_round)[descs++] = clk::AdmitDesc{
+            reinterpret_cast<const float *>(b->h_round_dev + at), J.cen[0], J.flags, J.gmax, (uint32_t)dk, J.d};
+        clk::GridUnit *u = reinterpret_cast<clk::GridUnit *>(b->h_round + kUnitsAt) + units;
+        for (uint32_t f = 0; f < J.d; ++f)
+            for (uint64_t first = 0; first < J.n; first += clk::kGridUnitValues)
+                *u++ = clk::GridUnit{J.pts + (size_t)f * J.n + first, J.gmax + f, J.gmax + J.d,
+                                     (uint32_t)std::min<uint64_t>(clk::kGridUnitValues, J.n - first)};
+        units += nu;
+        floats += dk;
+        return true;
+    }
+    int launch(hipStream_t st)
+    {
+        if (descs == 0)
+            return CLK_OK;
+        hipLaunchKernelGGL(clk::admit_kernel, dim3((unsigned)descs), dim3(256), 0, st,
+                           reinterpret_cast<const clk::AdmitDesc *>(b->h_round_dev));
+        CLK_HIP_CHECK(hipGetLastError());
+        CLK_TRY(clk::launch_grid_max_units(b->ctx, reinterpret_cast<const clk::GridUnit *>(b->h_round_dev + kUnitsAt),
+                                           (uint32_t)units, st));
+        CLK_HIP_CHECK(hipEventRecord(b->round_done, st));
+        return CLK_OK;
+    }
+};
+
+// round: the serving round to join if its buffer has room (the outputs of its
+// jobs are not cleared: the first iteration writes both).
 int stage_job(clk_batch *b, uint64_t n, uint32_t d, uint32_t k, const float *host_points,
               const float *host_centroids, uint32_t max_iterations, double tolerance, int32_t *slot,
-              hipStream_t st, bool device_points = false, bool zero_outputs = true)
+              hipStream_t st, bool device_points = false, AdmitRound *round = nullptr)
 {
     CLK_REQUIRE(n >= 1 && n <= (1ull << 30) && n * d <= (1ull << 30), CLK_ERR_SIZE,
                 "clk_batch_add: n must be >= 1 with n*d <= 2^30 (32-bit byte offsets into the points)");
@@ -2165,12 +2336,14 @@ int stage_job(clk_batch *b, uint64_t n, uint32_t d, uint32_t k, const float *hos
     if (!device_points)
         CLK_HIP_CHECK(
             hipMemcpyAsync(const_cast<float *>(J.pts), host_points, n * d * 4, hipMemcpyHostToDevice, st));
-    CLK_HIP_CHECK(hipMemcpyAsync(J.cen[0], host_centroids, (size_t)d * k * 4, hipMemcpyHostToDevice, st));
     // the job's sum grid (the one clk_sum_grid_from_points computes for these
     // points) and cleared flags
-    CLK_TRY(clk::launch_grid_max(b->ctx, d, n, J.pts, J.gmax, st));
-    CLK_HIP_CHECK(hipMemsetAsync(J.flags, 0, (size_t)d * k * 4, st));
-    if (zero_outputs || max_iterations == 0) {  // else the first iteration writes both
+    if (!round || !round->add(J, host_centroids)) {
+        CLK_HIP_CHECK(hipMemcpyAsync(J.cen[0], host_centroids, (size_t)d * k * 4, hipMemcpyHostToDevice, st));
+        CLK_TRY(clk::launch_grid_max(b->ctx, d, n, J.pts, J.gmax, st));
+        CLK_HIP_CHECK(hipMemsetAsync(J.flags, 0, (size_t)d * k * 4, st));
+    }
+    if (!round || max_iterations == 0) {  // else the first iteration writes both
         CLK_HIP_CHECK(hipMemsetAsync(J.masses, 0, (size_t)k * 4, st));
         CLK_HIP_CHECK(hipMemsetAsync(J.labels, 0, n * 4, st));
     }
@@ -2192,6 +2365,27 @@ int ensure_pinned_records(clk_batch *b)
     CLK_HIP_CHECK(hipHostMalloc((void **)&b->h_rec, b->jobs.size() * sizeof(BJob), hipHostMallocDefault));
     CLK_HIP_CHECK(hipHostGetDevicePointer((void **)&b->h_rec_dev, b->h_rec, 0));
     return CLK_OK;
+}
+
+// The serving rounds' buffer; without it (no pinned memory left) every job is
+// prepared singly.
+void ensure_round_buffer(clk_batch *b)
+{
+    if (b->h_round)
+        return;
+    char *p = nullptr, *dev = nullptr;
+    hipEvent_t ev = nullptr;
+    if (hipHostMalloc((void **)&p, AdmitRound::kBytes, hipHostMallocDefault) == hipSuccess &&
+        hipHostGetDevicePointer((void **)&dev, p, 0) == hipSuccess &&
+        hipEventCreateWithFlags(&ev, hipEventDisableTiming) == hipSuccess) {
+        b->h_round = p;
+        b->h_round_dev = dev;
+        b->round_done = ev;
+        return;
+    }
+    (void)hipGetLastError();
+    if (p)
+        (void)hipHostFree(p);
 }
 
 // Make a staged job visible: its record in the device job table and, for the
@@ -2534,6 +2728,8 @@ extern "C" int clk_serve_run(clk_batch *b, clk_serve_job *jobs, uint32_t count, 
         fail(CLK_ERR_INVALID_ARGUMENT);
     if (rc == CLK_OK && ensure_pinned_records(b) != CLK_OK)
         fail(CLK_ERR_HIP);
+    if (rc == CLK_OK)
+        ensure_round_buffer(b);
     const auto t0 = std::chrono::steady_clock::now();
     uint32_t next = 0, finished = 0, active = 0;
     bool inflight = false;
@@ -2545,11 +2741,12 @@ extern "C" int clk_serve_run(clk_batch *b, clk_serve_job *jobs, uint32_t count, 
         // 1. stage the arrived jobs in arrival order while slots and arena allow
         //    (their copies overlap the iteration in flight)
         const size_t round0 = staged.size();
+        AdmitRound round(b);
         while (next < count && jobs[next].arrival <= now) {
             clk_serve_job &j = jobs[next];
             int32_t s = -1;
             const int r = stage_job(b, j.n, j.d, j.k, j.points, j.centroids, j.max_iterations, j.tolerance, &s, cs,
-                                    j.device_points != 0, false);
+                                    j.device_points != 0, &round);
             if (r == CLK_ERR_NOMEM)
                 break;
             if (r != CLK_OK) {
@@ -2563,6 +2760,11 @@ extern "C" int clk_serve_run(clk_batch *b, clk_serve_job *jobs, uint32_t count, 
         }
         if (rc != CLK_OK)
             break;
+        const int launched = round.launch(cs);
+        if (launched != CLK_OK) {
+            fail(launched);
+            break;
+        }
         if (staged.size() > round0) {  // one event marks this round's copies
             hipEvent_t ev = nullptr;
             if (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess ||

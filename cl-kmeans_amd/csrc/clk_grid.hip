@@ -13,21 +13,15 @@ namespace {
 
 constexpr int kGridBlock = 1024;
 
-// blockIdx.y = feature; the work-items of blockIdx.x stride over the row,
-// four 128-bit loads in flight each.  NaN and +-inf are skipped.  The
-// work-group's maximum (bits of non-negative floats order like their values)
-// goes to gmax[f] with at most one atomicMax: device atomics on one address
-// take about 45 ns each, and one per wave bounded the pass.  Launch included,
-// before -> now: 2^20 points d=4 51 -> 14 us; 2.5M d=7 60 -> 29; 10M d=5
-// 81 -> 45; 2^27 d=4 382 -> 320 (6.7 TB/s).
-__global__ void __launch_bounds__(kGridBlock)
-grid_max_kernel(const float *__restrict__ pts, uint64_t n, uint32_t *__restrict__ gmax, uint32_t d)
+// The maximum of n values of a row over the work-items t0, t0 + stride, ...
+// (four 128-bit loads in flight each; NaN and +-inf are skipped), into *gmax:
+// bits of non-negative floats order like their values; NaN or +-inf set
+// *special_seen.  At most one atomicMax per work-group: device atomics on one
+// address take about 45 ns each.
+__device__ __forceinline__ void grid_max_row(const float *__restrict__ row, uint64_t n, uint64_t t0, uint64_t stride,
+                                             uint32_t *__restrict__ gmax, uint32_t *__restrict__ special_seen)
 {
     __shared__ uint32_t wave_max[kGridBlock / kWave];
-    const uint32_t f = blockIdx.y;
-    const float *row = pts + (uint64_t)f * n;
-    const uint64_t stride = (uint64_t)gridDim.x * kGridBlock;
-    const uint64_t t0 = (uint64_t)blockIdx.x * kGridBlock + threadIdx.x;
     uint32_t m = 0;
     bool special = false;  // a NaN or an infinity seen
     auto take = [&](float x) {
@@ -78,10 +72,29 @@ grid_max_kernel(const float *__restrict__ pts, uint64_t n, uint32_t *__restrict_
         flags |= wave_max[w];
     }
     // plain look first: most work-groups have nothing to raise
-    if (best > __hip_atomic_load(&gmax[f], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-        atomicMax(&gmax[f], best);
-    if ((flags & 0x80000000u) && !__hip_atomic_load(&gmax[d], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-        atomicOr(&gmax[d], 1u);
+    if (best > __hip_atomic_load(gmax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMax(gmax, best);
+    if ((flags & 0x80000000u) && !__hip_atomic_load(special_seen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicOr(special_seen, 1u);
+}
+
+// blockIdx.y = feature; the work-items of blockIdx.x stride over the row.  With
+// one atomic per work-group (one per wave bounded the pass), launch included,
+// before -> now: 2^20 points d=4 51 -> 14 us; 2.5M d=7 60 -> 29; 10M d=5
+// 81 -> 45; 2^27 d=4 382 -> 320 (6.7 TB/s).
+__global__ void __launch_bounds__(kGridBlock)
+grid_max_kernel(const float *__restrict__ pts, uint64_t n, uint32_t *__restrict__ gmax, uint32_t d)
+{
+    const uint32_t f = blockIdx.y;
+    grid_max_row(pts + (uint64_t)f * n, n, (uint64_t)blockIdx.x * kGridBlock + threadIdx.x,
+                 (uint64_t)gridDim.x * kGridBlock, gmax + f, gmax + d);
+}
+
+// Slices of rows of several point sets (cleared gmax), one per work-group.
+__global__ void __launch_bounds__(kGridBlock) grid_max_units_kernel(const GridUnit *__restrict__ units)
+{
+    const GridUnit u = units[blockIdx.x];
+    grid_max_row(u.values, u.count, threadIdx.x, kGridBlock, u.gmax, u.special_seen);
 }
 
 }  // namespace
@@ -100,6 +113,14 @@ int launch_grid_max(clk_context *ctx, uint64_t d, uint64_t n, const float *point
     KernelTimer t(ctx, "SumGrid", stream);
     hipLaunchKernelGGL(grid_max_kernel, dim3((unsigned)std::max<uint64_t>(gx, 1), (unsigned)d),
                        dim3(kGridBlock), 0, stream, points, n, gmax, (uint32_t)d);
+    CLK_HIP_CHECK(hipGetLastError());
+    return CLK_OK;
+}
+
+int launch_grid_max_units(clk_context *ctx, const GridUnit *units, uint32_t count, hipStream_t stream)
+{
+    KernelTimer t(ctx, "SumGrid", stream);
+    hipLaunchKernelGGL(grid_max_units_kernel, dim3(count), dim3(kGridBlock), 0, stream, units);
     CLK_HIP_CHECK(hipGetLastError());
     return CLK_OK;
 }

@@ -143,6 +143,19 @@ __device__ __forceinline__ void lds_or(uint32_t *p, uint32_t v)
 int launch_grid_max(clk_context *ctx, uint64_t d, uint64_t n, const float *points, uint32_t *gmax,
                     hipStream_t stream);
 
+// A slice of a row for launch_grid_max_units: count <= kGridUnitValues values,
+// their row's maximum (cleared before) and the NaN / inf word.
+struct GridUnit {
+    const float *values;
+    uint32_t *gmax, *special_seen;
+    uint32_t count;
+};
+constexpr uint64_t kGridUnitValues = 65536;
+
+// The grids of several point sets in one launch (units: device address, read
+// by the kernel).
+int launch_grid_max_units(clk_context *ctx, const GridUnit *units, uint32_t count, hipStream_t stream);
+
 // The grid the sum-accumulating ops of ctx use for (d, n, points): the
 // pinned one (clk_sum_grid_from_*) when set, else computed now into the
 // context's scratch.  out->own: computed now, or pinned from these points.

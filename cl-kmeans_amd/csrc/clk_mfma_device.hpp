@@ -624,20 +624,31 @@ __device__ void build_table_block(const float *__restrict__ cen, uint32_t d, uin
     }
     double nmax = 0.0, rmax = 0.0;
     bool dropped = false;
-    for (uint32_t c = tid; c < ntiles * kTile; c += blockDim.x) {
+    // four neighbouring lanes a centroid (blockDim.x is a multiple of 64, and
+    // so is ntiles * kTile * 4: whole quads take part in the exchanges)
+    for (uint32_t e = tid; e < ntiles * kTile * 4; e += blockDim.x) {
+        const uint32_t c = e / 4;
         double s = 0.0, r = 0.0;
-        bool fin = c < k, in_range = true;
-        for (uint32_t f = 0; f < d && fin; ++f) {
-            const float v = cen[(uint64_t)f * k + c];
-            fin = isfinite(v);
-            in_range = in_range && (!FP16 || fabs(2.0 * (double)v) < 65504.0);
-            s = fma((double)v, (double)v, s);
-            const double res = (double)from16<FP16>(to16<FP16>(-2.0f * v)) + 2.0 * (double)v;
-            r = fma(res, res, r);
+        uint32_t bad = c < k ? 0u : 1u;  // bit 0: not finite, bit 1: out of the 16-bit range
+        if (c < k)
+#pragma unroll 4
+            for (uint32_t f = e % 4; f < d; f += 4) {
+                const float v = cen[(uint64_t)f * k + c];
+                bad |= isfinite(v) ? 0u : 1u;
+                bad |= (!FP16 || fabs(2.0 * (double)v) < 65504.0) ? 0u : 2u;
+                s = fma((double)v, (double)v, s);
+                const double res = (double)from16<FP16>(to16<FP16>(-2.0f * v)) + 2.0 * (double)v;
+                r = fma(res, res, r);
+            }
+        for (int o = 1; o <= 2; o *= 2) {
+            s += __shfl_xor(s, o);
+            r += __shfl_xor(r, o);
+            bad |= __shfl_xor(bad, o);
         }
-        const bool ok = fin && in_range && s < 3.0e38;
-        dropped = dropped || (fin && !ok);
-        norm[c] = ok ? (float)s : INFINITY;
+        const bool ok = bad == 0 && s < 3.0e38;
+        dropped = dropped || ((bad & 1u) == 0 && !ok);
+        if (e % 4 == 0)
+            norm[c] = ok ? (float)s : INFINITY;
         if (ok) {
             nmax = fmax(nmax, s);
             rmax = fmax(rmax, r);
