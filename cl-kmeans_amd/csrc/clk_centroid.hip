@@ -305,7 +305,9 @@ cu_feature_sum_kernel(const float *__restrict__ pts, uint64_t n, uint32_t d, uin
 // consecutive points per step (lane = point: F coalesced loads and the label)
 // and adds each point's grid integers into its cluster's cells with ds_add_u64
 // (exact, so no ordering between lanes or waves is needed); R replicas (lane
-// mod R) thin out the same-cell additions of a wave when k is small.
+// mod R) thin out the same-cell additions of a wave when k is small.  The
+// slice's values go to the work-group's partial row, or (direct, one
+// work-group per slice) are added to the sums.
 // Bound by the points' bytes from a few million points on: 16M points d=64
 // k=1024 648 us (6.4 TB/s; 32-bit flags, four features per slice and a quarter
 // more label reads took 730), d=32 k=256 339 us (6.2 TB/s).  Against the
@@ -322,7 +324,7 @@ size_t cell_lds_bytes(uint32_t F, uint64_t k, uint32_t R)
 template <int F>
 __global__ void __launch_bounds__(64 * kCellWaves)
 cu_cell_kernel(const float *__restrict__ pts, uint64_t n, uint32_t d, uint32_t k, const uint32_t *__restrict__ labels,
-               GridRef grid, uint32_t R, double *__restrict__ part)
+               GridRef grid, uint32_t R, double *__restrict__ part, int direct)
 {
     extern __shared__ __align__(16) char lds_cell[];
     constexpr uint32_t B = 64 * kCellWaves;
@@ -418,11 +420,12 @@ cu_cell_kernel(const float *__restrict__ pts, uint64_t n, uint32_t d, uint32_t k
         long long q = 0;
         for (uint32_t r = 0; r < R; ++r)
             q += acc[(size_t)r * cells + i];
-        row[i] = cell_value(q, grid_unit(scl[i / k]), (flg[i / 4] >> 8 * (i % 4)) & 7u);
+        const double value = cell_value(q, grid_unit(scl[i / k]), (flg[i / 4] >> 8 * (i % 4)) & 7u);
+        row[i] = direct ? row[i] + value : value;
     }
 }
 
-using CellKernel = void (*)(const float *, uint64_t, uint32_t, uint32_t, const uint32_t *, GridRef, uint32_t, double *);
+using CellKernel = void (*)(const float *, uint64_t, uint32_t, uint32_t, const uint32_t *, GridRef, uint32_t, double *, int);
 
 struct CellPlan {
     CellKernel kern = nullptr;
@@ -596,14 +599,22 @@ int run_centroid_update(clk_context *ctx, const clk_kernel_config *cfg, uint64_t
         uint64_t gxs = auto_grid(ctx, (const void *)cells.kern, 64 * kCellWaves, cells.lds, n * gy) / gy;
         gxs = std::min<uint64_t>(gxs, div_up(n, std::max<uint64_t>(4 * k, 64 * kCellWaves)));
         gxs = std::max<uint64_t>(1, std::min<uint64_t>(gxs, 65535));
-        CLK_TRY(ensure_scratch(ctx->part_sums, gxs * dk * sizeof(double)));
-        double *ps = static_cast<double *>(ctx->part_sums.ptr);
+        // Few points: one work-group per slice, which adds its sums itself --
+
+        const bool direct = n * cells.F <= 32768 && n <= 16384;
+        if (direct)
+            gxs = 1;
+        else
+            CLK_TRY(ensure_scratch(ctx->part_sums, gxs * dk * sizeof(double)));
+        double *ps = direct ? sums : static_cast<double *>(ctx->part_sums.ptr);
         {
             KernelTimer t(ctx, kCellNames[strategy], stream);
             hipLaunchKernelGGL(cells.kern, dim3((unsigned)gxs, (unsigned)gy), dim3(64 * kCellWaves), cells.lds,
-                               stream, points, n, (uint32_t)d, (uint32_t)k, labels, sg, cells.R, ps);
+                               stream, points, n, (uint32_t)d, (uint32_t)k, labels, sg, cells.R, ps, direct);
             CLK_HIP_CHECK(hipGetLastError());
         }
+        if (direct)
+            return CLK_OK;
         return launch_merge_sums(ctx, ps, gxs, dk, sums, stream);
     }
     if (!kern)

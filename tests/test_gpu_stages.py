@@ -34,6 +34,8 @@ def test_mass_histogram(gpu_ctx, n, k):
 @pytest.mark.parametrize("n,d,k", [
     (1, 1, 1), (63, 2, 3), (65, 3, 2), (1000, 5, 33), (4097, 9, 1), (5000, 16, 300), (5001, 17, 700), (6000, 70, 40),
     (30001, 4, 5000), (3000, 3, 17000), (3000, 2, 20000), (600003, 6, 10),
+    # one work-group per slice adds to the sums itself, and one point more
+    (16384, 1, 30), (16385, 2, 7), (8192, 3, 10), (8193, 4, 10), (4096, 7, 300), (4097, 8, 5), (2048, 33, 40), (2049, 64, 9),
 ])
 def test_centroid_cells(gpu_ctx, n, d, k, special):
     rng = np.random.default_rng(n + d + k)
