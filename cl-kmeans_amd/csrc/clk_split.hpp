@@ -241,7 +241,11 @@ __device__ __forceinline__ Table<T> stage(const T *__restrict__ cen, uint32_t d,
             const bool in = c < k && f < d && (P != 4 || h < 2);
             const T raw = cen[in ? (size_t)f * k + c : 0];
             const bool fin = raw <= kMax && raw >= -kMax;
-            const float x = in && fin ? (float)((T)(-2.0f * s) * raw) : 0.0f;
+            float x = in && fin ? (float)((T)(-2.0f * s) * raw) : 0.0f;
+            // both parts come from the FP32 value: the compiler would round a
+            // double to FP16 at once for the high part, and not to the same
+            // neighbour when the FP32 value lies between two
+            asm("" : "+v"(x));
             _Float16 p = (_Float16)x;
             if (lo)
                 p = (_Float16)(x - (float)p);

@@ -105,3 +105,28 @@ def test_split_double(gpu_ctx, shape, kind):
         exact = O.sums_f64_dp(pts, ref, k)
         absx = np.stack([np.bincount(ref.astype(np.int64), weights=np.abs(x), minlength=k) for x in pts])
         assert np.all(np.abs(sums.to_host() - exact) <= 1e-13 * absx + 1e-300)
+
+
+@pytest.mark.parametrize("n,d,k", [(100003, 3, 60), (100003, 4, 128), (20000, 7, 100), (20000, 16, 64), (20000, 24, 64), (20000, 48, 100)])
+def test_double_centroids_between_two_halves(gpu_ctx, n, d, k):
+    # coordinates whose FP32 rounding, scaled by a power of two, is exactly
+    # between two FP16 values, while the double lies to one side: both parts
+    # of the operand must come from the same rounding.  The points lie near
+    # the planes between each centroid and its neighbour.
+    rng = np.random.default_rng(d + k)
+    cen = rng.uniform(1.0, 2.0, (d, k))
+    cen = np.floor(cen * 1024) / 1024  # on the FP16 grid of [1, 2)
+    cen += 2.0 ** -11  # between two of its values (the spacing is 2^-10)
+    cen *= 1 + rng.choice([-1.0, 1.0], (d, k)) * 2.0 ** -27  # and a little off
+    cen[0, 0] = 3.5
+    a = rng.integers(0, k, n)
+    other = cen[:, a]
+    dist = ((cen[:, :, None] - cen[:, None, :]) ** 2).sum(0) + 1e9 * np.eye(k)
+    near = dist.argmin(1)[a]
+    t = 0.5 + rng.uniform(-1e-3, 1e-3, n)
+    pts = np.ascontiguousarray(other * t + cen[:, near] * (1 - t))
+    cfg = gpu_ctx.config(clkmeans.STAGE_LABELING, "unroll_vector")
+    dl = zeros(n, np.uint64)
+    gpu_ctx.labeling(cfg, d, n, k, dev(pts), dev(cen), dl)
+    hip.synchronize()
+    np.testing.assert_array_equal(dl.to_host(), O.label_f64(pts, np.ascontiguousarray(cen)))
