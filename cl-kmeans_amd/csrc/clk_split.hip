@@ -128,7 +128,8 @@ split_kernel(const T *__restrict__ pts, uint64_t n, uint32_t d, uint32_t k, cons
             x2 = build_points<P, T>(x, t.scale, lane, ops);
         rank_points<P, T>(t, ops, lane, best, second);
         uint32_t lab;
-        const bool sure = decide(t, x2, best, second, k, lab);
+        float limit;
+        const bool sure = decide(t, x2, best, second, k, lab, limit);
         uint64_t open = __ballot(!sure && p < n);
         if constexpr (P < 32) {
             // Many undecided points against few centroids: every lane scans
@@ -138,6 +139,18 @@ split_kernel(const T *__restrict__ pts, uint64_t n, uint32_t d, uint32_t k, cons
                 const uint32_t scanned = scan_rows<P, T>(t, x[0], d, k);
                 lab = sure ? lab : scanned;
                 open = 0;
+            }
+        }
+        if constexpr (P >= 32 && !(f64 && !FUSED && P == 32)) {  // (its registers spill)
+            // Scoring the tiles again and one exact distance a lane for each
+            // tile with candidates, against the rounds of the full scan: 188k
+            // points d=53 k=290 with clusters sharing blobs 640 -> 203 us.
+            const uint64_t known = __ballot(!sure && p < n && limit == limit);
+            const uint32_t m = (uint32_t)__builtin_popcountll(known);
+            const uint32_t full = k > 32 ? m * ((k + 63) / 64) : k > 16 ? (m + 1) / 2 : (m + 3) / 4;
+            if (full > min(ntiles, 2 * m) + ntiles / 8 + 1) {
+                candidate_scan<P>(t, ops, known, limit, pts + bt * 64, n, cen, d, k, lane, lab);
+                open &= ~known;
             }
         }
         if (open)
@@ -327,10 +340,11 @@ bool split_labeling_pays(const clk_context *ctx, const clk_kernel_config *cfg, u
     // stay below the ranking's.  Fused step: d=4 k=3 33 / 34, k=10 25 / 29,
     // k=50 36 / 47; d=16 k=5 61 / 50, k=10 52 / 73; d=32 k=32 88 / 190; 300k
     // points d=4 k=5 14 / 19, d=16 k=3 22 / 35; 20k points d=4 k=5 11 / 16.
-    // One feature and many clusters: the gaps sink below the keys' truncation
-    // (274k points k=238: 81 / 45) and the plain scan costs 5 per centroid.
+    // One feature: the gaps sink below the keys' truncation (2M points k=8 20 /
+    // 11, k=20 26 / 12, 274k k=238 81 / 45); the plain scan takes 5 operations
+    // a centroid.
     if (fused)
-        return (k >= 6 || (n <= (1u << 20) && k >= 2)) && (d > 1 || k <= 32) &&
+        return (k >= 6 || (n <= (1u << 20) && k >= 2)) && d > 1 &&
                split_plan<true, float>(ctx, d, k).kern != nullptr;
     const uint64_t bucket = split_bucket(d);
     return n >= 4096 && d >= 3 && k * (2 * bucket + 3) >= 300 + 20 * bucket &&

@@ -11,7 +11,9 @@
 // K = 32 of one 16x16x32 MFMA holds, for P padded features:
 //   P = 4, 8 all four products xh ch, xh cl, xl ch, xl cl of the features;
 //   P = 16   two MFMAs, (ch | cl) against (xh | xh) and (xl | xl);
-//   P >= 32  three MFMAs per 32 features: xh ch, xl ch, xh cl.
+//   P >= 32  three MFMAs per 32 features: xl ch, xh cl of all features from 0,
+//            the norm added, then xh ch -- so that the small products are
+//            summed while the sum is small, and round a third as much.
 // Scores may be negative: they are ranked as floats.  A key is the score with
 // its low bits replaced by an index.
 //
@@ -23,7 +25,10 @@
 //                (2^-10 X + 2^-24 sqrt(d)) (2^-11 2C + 2^-25 sqrt(d))
 //   summation    g (N + 1.004 X 2C), g = 2(T+1)u / (1 - 2(T+1)u) for the T
 //                products that are not padding (adding 0 is exact), each
-//                addition rounding or truncating
+//                addition rounding or truncating.  P >= 32: T = d (xh ch, on
+//                top of the norm and the small products), the addition of the
+//                norm 2u (N + their sum), and theirs, g' with T = 2d of
+//                (2^-10 X + 2^-24 sqrt(d)) 2C (1 + 2^-11) + X (2^-11 2C + 2^-25 sqrt(d))
 //   norm         2u N
 // E = 1.01 x the sum + a bound on flushed denormals.  An FP16 subnormal must
 // reach the product: every launch checks that the matrix core keeps them, and
@@ -63,7 +68,7 @@ template <int P>
 struct Shape {
     static constexpr int nkb = P < 32 ? 1 : P / 32;       // K-blocks of 32 features
     static constexpr int nops = P < 32 ? 1 : 2 * nkb;     // operand vectors per tile of 16 centroids
-    static constexpr int terms = P < 32 ? 4 : 3;  // products per feature
+    static constexpr int terms = P < 32 ? 4 : 1;  // products per feature in the sum with the norm
     static constexpr int planes = P < 32 ? P / 4 : 0;  // LDS exchange, u16x8 [64] each
 };
 
@@ -175,9 +180,16 @@ __device__ __forceinline__ void set_margin(Table<T> &t, float N, uint32_t d, uin
         const float m = 0x1p-11f * C2 + 0x1p-25f * sd;
         e1 += 0x1p-10f * m;
         e0 += 0x1p-24f * sd * m;
+        // the small products' sum is at most s1 X + s0; g2 their summation,
+        // the norm's addition to it and its part in the last one
+        const float s1 = 1.01f * (0x1p-10f * C2 + m), s0 = 1.01f * 0x1p-24f * sd * C2;
+        const float g2 = 4.0f * ((float)d + 1.0f) * mfma::kU / (1.0f - 4.0f * ((float)d + 1.0f) * mfma::kU) * up +
+                         2.0f * mfma::kU + gamma;
+        e1 += g2 * s1;
+        e0 += g2 * s0 + 2.0f * mfma::kU * N;
     }
     e1 *= 1.01f;
-    e0 = 1.01f * e0 + (terms + 2.0f) * 0x1p-125f;
+    e0 = 1.01f * e0 + (4.0f * (float)d + 2.0f) * 0x1p-125f;
     const float eps = (float)(d + 3) * (f64 ? 0x1p-53f : mfma::kU) * up;
     const float tr0 = __uint_as_float((bits - 23 + 127) << 23), tr = tr0 / (1.0f - tr0) * up;
     const float under = f64 ? 0.0f : t.scale * t.scale * (float)d * 0x1p-125f;
@@ -401,6 +413,46 @@ __device__ __forceinline__ float build_points(const T (&raw)[4][Shape<P>::nkb * 
     return mine * (1.0f + (float)(2 * P + 12) * mfma::kU);
 }
 
+// The scores of a tile: acc[g][i] of point 16g + q and centroid 16 tile + 4h + i.
+template <int P, typename T>
+__device__ __forceinline__ void score_tile(const Table<T> &t, const PointOps<P> &x, uint32_t tile, uint32_t lane,
+                                           f32v4 (&acc)[4])
+{
+    using Sh = Shape<P>;
+    const f32v4 nrm = *reinterpret_cast<const f32v4 *>(t.norm + tile * 16 + 4 * (lane / 16));
+    if constexpr (P < 32) {
+        const u16x8 a = t.ops[tile * 64 + lane];
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+            acc[g] = mfma::mma16<true>(a, x.hi[g][0], nrm);
+        if constexpr (P == 16)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                acc[g] = mfma::mma16<true>(a, x.lo[g][0], acc[g]);
+    } else {
+        u16x8 ah[Sh::nkb];
+#pragma unroll
+        for (int kb = 0; kb < Sh::nkb; ++kb) {
+            ah[kb] = t.ops[(tile * Sh::nops + 2 * kb) * 64 + lane];
+            const u16x8 al = t.ops[(tile * Sh::nops + 2 * kb + 1) * 64 + lane];
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                acc[g] = mfma::mma16<true>(ah[kb], x.lo[g][kb], kb == 0 ? f32v4{0.0f, 0.0f, 0.0f, 0.0f} : acc[g]);
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                acc[g] = mfma::mma16<true>(al, x.hi[g][kb], acc[g]);
+        }
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+            acc[g] += nrm;
+#pragma unroll
+        for (int kb = 0; kb < Sh::nkb; ++kb)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                acc[g] = mfma::mma16<true>(ah[kb], x.hi[g][kb], acc[g]);
+    }
+}
+
 // The two smallest keys of this lane's own point over all centroids.  A key's
 // low bits hold (4 tile + i) * 4 + h for row 4h + i of a tile: the tile and
 // row parts are the same for all lanes (scalar operands), h is put in once
@@ -415,7 +467,6 @@ template <int P, typename T>
 __device__ __forceinline__ void rank_points(const Table<T> &t, const PointOps<P> &x, uint32_t lane, float &best,
                                             float &second)
 {
-    using Sh = Shape<P>;
     const uint32_t h = lane / 16;
     float b[4], s[4];
 #pragma unroll
@@ -423,33 +474,8 @@ __device__ __forceinline__ void rank_points(const Table<T> &t, const PointOps<P>
         b[g] = s[g] = FLT_MAX;
     const uint32_t vkeep = mfma::opaque_v(~t.kmask);
     for (uint32_t tile = 0; tile < t.ntiles; ++tile) {
-        const f32v4 nrm = *reinterpret_cast<const f32v4 *>(t.norm + tile * 16 + 4 * h);
         f32v4 acc[4];
-#pragma unroll
-        for (int kb = 0; kb < Sh::nkb; ++kb) {
-            if constexpr (P < 32) {
-                const u16x8 a = t.ops[tile * 64 + lane];
-#pragma unroll
-                for (int g = 0; g < 4; ++g)
-                    acc[g] = mfma::mma16<true>(a, x.hi[g][0], nrm);
-                if constexpr (P == 16)
-#pragma unroll
-                    for (int g = 0; g < 4; ++g)
-                        acc[g] = mfma::mma16<true>(a, x.lo[g][0], acc[g]);
-            } else {
-                const u16x8 ah = t.ops[(tile * Sh::nops + 2 * kb) * 64 + lane];
-                const u16x8 al = t.ops[(tile * Sh::nops + 2 * kb + 1) * 64 + lane];
-#pragma unroll
-                for (int g = 0; g < 4; ++g)
-                    acc[g] = mfma::mma16<true>(ah, x.hi[g][kb], kb == 0 ? nrm : acc[g]);
-#pragma unroll
-                for (int g = 0; g < 4; ++g)
-                    acc[g] = mfma::mma16<true>(ah, x.lo[g][kb], acc[g]);
-#pragma unroll
-                for (int g = 0; g < 4; ++g)
-                    acc[g] = mfma::mma16<true>(al, x.hi[g][kb], acc[g]);
-            }
-        }
+        score_tile<P>(t, x, tile, lane, acc);
         uint32_t idx[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i)
@@ -482,19 +508,27 @@ __device__ __forceinline__ void rank_points(const Table<T> &t, const PointOps<P>
     second = s[0];
 }
 
-// Margin test of this lane's own point; lab = the best key's centroid.
+// Margin test of this lane's own point; lab = the best key's centroid.  limit:
+// a centroid whose key v has v - t.tk |v| > limit is farther than the best
+// key's by the reference's arithmetic (NaN, which nothing exceeds, where the
+// bounds do not hold).
 template <typename T>
-__device__ __forceinline__ bool decide(const Table<T> &t, float x2, float best, float second, uint32_t k, uint32_t &lab)
+__device__ __forceinline__ bool decide(const Table<T> &t, float x2, float best, float second, uint32_t k, uint32_t &lab,
+                                       float &limit)
 {
     const float X = __builtin_amdgcn_sqrtf(x2);  // within one ulp
     const float ab = __builtin_fabsf(best);
-    float tau = __builtin_fmaf(t.tX, X, t.t0);
-    tau = __builtin_fmaf(t.tx2, x2, tau);
-    tau = __builtin_fmaf(t.tk, ab + __builtin_fabsf(second), tau);
+    float base = __builtin_fmaf(t.tX, X, t.t0);
+    base = __builtin_fmaf(t.tx2, x2, base);
+    const float tau = __builtin_fmaf(t.tk, ab + __builtin_fabsf(second), base);
     lab = centroid_of(best, t.kmask);
     // NaN fails every test; 4.2e9 < 65504^2; a key of denormal size is not
     // trusted to keep its index
-    return t.ok && x2 < 4.2e9f && best < 1e37f && ab > 1e-30f && second - best > tau && lab < k;
+    const bool holds = t.ok && x2 < 4.2e9f && best < 1e37f && ab > 1e-30f && lab < k;
+    base = __builtin_fmaf(t.tk, ab, base);
+    // rounded up: by more than this sum's and the test's own roundings
+    limit = holds ? best + base + 8.0f * mfma::kU * (ab + base) : __builtin_nanf("");
+    return holds && second - best > tau;
 }
 
 // The reference's scan, over all centroids, of the wave's points whose bit is
@@ -567,6 +601,92 @@ __device__ __forceinline__ void exact_scan(uint64_t open, const T *__restrict__ 
             const uint32_t r = (uint32_t)__builtin_amdgcn_readlane((int)found, (int)(i * G));
             lab = lane == bit ? r : lab;
         }
+    }
+}
+
+// The points of open settled among the centroids that their limits leave
+// (usually two or three): the tiles are scored again, and every lane takes the
+// exact distances of its rows' candidates, its own point and centroid each.
+// base as in exact_scan.
+template <int P, typename T>
+__device__ __forceinline__ void candidate_scan(const Table<T> &t, const PointOps<P> &ops, uint64_t open, float limit,
+                                               const T *__restrict__ base, uint64_t n, const T *__restrict__ cen,
+                                               uint32_t d, uint32_t k, uint32_t lane, uint32_t &lab)
+{
+    constexpr bool f64 = sizeof(T) == 8;
+    constexpr T kMax = f64 ? (T)DBL_MAX : (T)FLT_MAX;
+    constexpr uint32_t kAhead = f64 || P > 64 ? 8 : 16;
+    const uint32_t q = lane % 16, h = lane / 16;
+    float lim[4];
+    T best[4];
+    uint32_t at[4];
+    uint32_t live = 0;  // bits 4g .. 4g+3: this lane's point of group g is open
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        lim[g] = __shfl(limit, g * 16 + (int)q);
+        live |= (open >> (g * 16 + q)) & 1 ? 15u << (4 * g) : 0u;
+        best[g] = kMax;
+        at[g] = 0;
+    }
+    for (uint32_t tile = 0; tile < t.ntiles; ++tile) {
+        f32v4 acc[4];
+        score_tile<P>(t, ops, tile, lane, acc);
+        uint32_t cand = 0;
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                // the score itself: its key is within t.tk of it
+                const float v = acc[g][i];
+                const bool in = v - 2.0f * t.tk * __builtin_fabsf(v) <= lim[g] && tile * 16 + 4 * h + i < k;
+                cand |= (in ? 1u : 0u) << (4 * g + i);
+            }
+        cand &= live;
+        while (cand) {
+            const uint32_t bit = (uint32_t)__builtin_ctz(cand), g = bit / 4;
+            cand &= cand - 1;
+            const uint32_t c = tile * 16 + 4 * h + bit % 4;
+            const T *x = base + g * 16 + q, *col = cen + c;
+            T dist = 0;
+            for (uint32_t f0 = 0; f0 < d; f0 += kAhead) {
+                T xv[kAhead], cv[kAhead];
+#pragma unroll
+                for (uint32_t j = 0; j < kAhead; ++j) {
+                    const uint32_t f = min(f0 + j, d - 1);
+                    xv[j] = x[(uint64_t)f * n];
+                    cv[j] = col[(size_t)f * k];
+                }
+#pragma unroll
+                for (uint32_t j = 0; j < kAhead; ++j)
+                    if (f0 + j < d) {
+                        const T u = xv[j] - cv[j];
+                        if constexpr (f64)
+                            dist = __builtin_fma(u, u, dist);
+                        else
+                            dist = __builtin_fmaf(u, u, dist);
+                    }
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i)  // ascending centroids: strict
+                if ((uint32_t)i == g && dist < best[i]) {
+                    best[i] = dist;
+                    at[i] = c;
+                }
+        }
+    }
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        T b = best[g];
+        uint32_t c = at[g];
+        for (int o = 16; o <= 32; o *= 2) {
+            const T b2 = __shfl_xor(b, o);
+            const uint32_t c2 = (uint32_t)__shfl_xor((int)c, o);
+            const bool take = b2 < b || (b2 == b && c2 < c);
+            b = take ? b2 : b;
+            c = take ? c2 : c;
+        }
+        if ((uint32_t)g == h && ((open >> lane) & 1))
+            lab = c;
     }
 }
 

@@ -130,3 +130,33 @@ def test_double_centroids_between_two_halves(gpu_ctx, n, d, k):
     gpu_ctx.labeling(cfg, d, n, k, dev(pts), dev(cen), dl)
     hip.synchronize()
     np.testing.assert_array_equal(dl.to_host(), O.label_f64(pts, np.ascontiguousarray(cen)))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n,d,k", [(4101, 17, 290), (4164, 32, 129), (5000, 33, 200), (4099, 53, 290), (4097, 64, 300),
+                                   (4100, 96, 100), (4097, 128, 90)])
+def test_split_many_undecided(gpu_ctx, n, d, k, dtype):
+    # far from the origin in every direction, two or more centroids close
+    # together: most points stay undecided between a few of them.  Some points
+    # and centroids that no score can order.
+    rng = np.random.default_rng(n + d)
+    centres = rng.uniform(-50, 50, (d, max(k // 3, 2)))
+    pts = centres[:, rng.integers(0, centres.shape[1], n)] + rng.standard_normal((d, n)) * 0.3
+    pts = np.ascontiguousarray(pts.astype(dtype))
+    cen = np.ascontiguousarray(pts[:, :k])
+    cen[:, k // 2] = cen[:, 1]  # ties
+    cen[d - 1, k - 2] = np.nan
+    pts[0, n - 1], pts[d // 2, n - 7], pts[0, 900] = np.nan, np.inf, 1e30
+    f64 = dtype == np.float64
+    ref = O.label_f64(pts, cen) if f64 else O.label(pts, cen)
+    whole = np.uint64 if f64 else np.uint32
+    dl = zeros(n, whole)
+    gpu_ctx.labeling(gpu_ctx.config(clkmeans.STAGE_LABELING, "unroll_vector"), d, n, k, dev(pts), dev(cen), dl)
+    hip.synchronize()
+    np.testing.assert_array_equal(dl.to_host(), ref)
+    if not f64 and d <= 32:
+        dl, sums, masses = zeros(n, whole), zeros((d, k), np.float64), zeros(k, np.uint32)
+        gpu_ctx.fused(gpu_ctx.config(clkmeans.STAGE_FUSED, "feature_sum"), d, n, k, dev(pts), dev(cen), sums, dl, masses)
+        hip.synchronize()
+        np.testing.assert_array_equal(dl.to_host(), ref)
+        np.testing.assert_array_equal(masses.to_host(), O.mass(ref, k))
