@@ -382,8 +382,11 @@ int run_fused(clk_context *ctx, const clk_kernel_config *cfg, uint64_t d, uint64
                        priv_plain <= ctx->lds_per_block;
     // The bounded pass needs k keep thresholds beside the private tile; where
     // they do not fit it runs as "cluster_merge" (the same results).
-    const bool run_bounded = bounded && use_private && priv_plain + thr_bytes <= ctx->lds_per_block;
+    bool run_bounded = bounded && use_private && priv_plain + thr_bytes <= ctx->lds_per_block;
     const uint64_t priv_bytes = priv_plain + (run_bounded ? thr_bytes : 0);
+    const char *name = !use_private  ? "FusedFeatureSum"
+                       : run_bounded ? "FusedClusterMergeBounded"
+                                     : "FusedClusterMerge";
     bool use_shared = dmax && !use_private && k * d < (1ull << 24) && shared_bytes <= ctx->lds_per_block;
 
     CLK_REQUIRE(!ext || use_private || use_shared || n == 0, CLK_ERR_UNSUPPORTED,
@@ -410,12 +413,24 @@ int run_fused(clk_context *ctx, const clk_kernel_config *cfg, uint64_t d, uint64
 
     const bool b256 = (B == 256);
     const bool exact = (uint64_t)dmax == d;
+    // Up to four features the private columns pay on large data only, with two
+    // work-groups per CU: clearing and flushing them costs more than the shared
+    // cells' atomics below (private / shared, us: 20k points d=2 k=10 13.4 /
+    // 6.8; 1M d=4 k=10 19.6 / 13.0, d=3 k=5 22 / 12; 3M d=4 k=10 26.9 / 25.1;
+    // but 16M d=4 k=10 84 / 101, d=2 k=10 54 / 66; one work-group, d=4 k=24
+    // 241 / 120).  An explicit launch geometry names the strategy's kernel.
+    const bool two_groups = 2 * priv_bytes <= ctx->lds_per_block;
+    const bool geometry = cfg && (cfg->global_size[0] || (cfg->local_size[0] && cfg->local_size[0] != 256));
+    if (d <= 4 && !geometry && use_private && !(n >= (4u << 20) && two_groups)) {
+        use_private = run_bounded = false;
+        use_shared = true;
+    }
     // The bounded pass is the faster one on settled labels where it keeps two
     // work-groups per CU and the points dwarf its fixed costs (16M points,
     // d=4 k=10: 84 us against 110-124 with split labels; d=8 k=8 123 / 146-188;
     // but d=4 k=16, one work-group: 185 / 105-125, and 1M points d=4 k=10:
     // 26 / 18-20).
-    const bool split = !(run_bounded && n >= (4u << 20) && 2 * priv_bytes <= ctx->lds_per_block) &&
+    const bool split = !(run_bounded && n >= (4u << 20) && two_groups) &&
                        split_labeling_pays(ctx, cfg, d, n, k, true);
     FusedKernel kern = !use_private ? pick_fused<false, false>(dmax, exact, vec, b256)
                        : run_bounded ? pick_fused<true, true>(dmax, exact, vec, b256)
@@ -457,9 +472,6 @@ int run_fused(clk_context *ctx, const clk_kernel_config *cfg, uint64_t d, uint64
         CLK_TRY(ensure_scratch(ctx->part_sums, grid * (d + 1) * k * sizeof(double)));
         part = static_cast<double *>(ctx->part_sums.ptr);
     }
-    const char *name = !use_private  ? "FusedFeatureSum"
-                       : run_bounded ? "FusedClusterMergeBounded"
-                                     : "FusedClusterMerge";
     if (split) {
         CLK_TRY(launch_fused_split(ctx, name, d, n, k, points, old_centroids, labels, sgrid, grid, part, max_shift,
                                    stream));

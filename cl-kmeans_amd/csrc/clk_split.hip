@@ -343,9 +343,14 @@ bool split_labeling_pays(const clk_context *ctx, const clk_kernel_config *cfg, u
     // One feature: the gaps sink below the keys' truncation (2M points k=8 20 /
     // 11, k=20 26 / 12, 274k k=238 81 / 45); the plain scan takes 5 operations
     // a centroid.
+    // Up to four features the plain pass (shared cells) is the faster one
+    // until the scan is long: 3M points d=4 k=10 26.0 / 25.1, k=24 30.8 / 30.5,
+    // k=48 36 / 45; 300k d=4 k=24 12.3 / 9.9, k=48 12.8 / 12.6; d=3 k=32 11.9 /
+    // 10.6, k=48 12.8 / 12.2, 3M 36 / 41; d=2 k=150 3M 79 / 67.
+    if (fused && d <= 4)
+        return d >= 3 && k >= 48 && split_plan<true, float>(ctx, d, k).kern != nullptr;
     if (fused)
-        return (k >= 6 || (n <= (1u << 20) && k >= 2)) && d > 1 &&
-               split_plan<true, float>(ctx, d, k).kern != nullptr;
+        return (k >= 6 || (n <= (1u << 20) && k >= 2)) && split_plan<true, float>(ctx, d, k).kern != nullptr;
     const uint64_t bucket = split_bucket(d);
     return n >= 4096 && d >= 3 && k * (2 * bucket + 3) >= 300 + 20 * bucket &&
            split_plan<false, float>(ctx, d, k).kern != nullptr;
