@@ -337,9 +337,8 @@ bool split_labeling_pays(const clk_context *ctx, const clk_kernel_config *cfg, u
     // unless said).  Labeling: d=4 k=20 18.3 / 13.7, k=32 17.6 / 18.7; d=8
     // k=16 17.8 / 20.8; d=16 k=16 31 / 39; d=32 k=10 60 / 55, k=16 55 / 65;
     // with one or two features the plain scan's 2d + 3 operations per centroid
-    // stay below the ranking's.  Fused step: d=4 k=3 33 / 34, k=10 25 / 29,
-    // k=50 36 / 47; d=16 k=5 61 / 50, k=10 52 / 73; d=32 k=32 88 / 190; 300k
-    // points d=4 k=5 14 / 19, d=16 k=3 22 / 35; 20k points d=4 k=5 11 / 16.
+    // stay below the ranking's.  Fused step: d=16 k=5 61 / 50, k=10 52 / 73; d=32 k=32 88 / 190; 300k
+    // points d=16 k=3 22 / 35.
     // One feature: the gaps sink below the keys' truncation (2M points k=8 20 /
     // 11, k=20 26 / 12, 274k k=238 81 / 45); the plain scan takes 5 operations
     // a centroid.
