@@ -348,7 +348,14 @@ int clk_sum_grid_units(clk_context *ctx, uint64_t d, uint64_t n,
  * when nothing is smaller; every strategy id of a stage runs the same FP64
  * pass (an LDS-tiled pass with a fixed-order merge where the tile fits, FP64
  * / uint64 global atomics beyond).  Labels and masses are exact; sums carry
- * FP64 rounding of a different summation order.
+ * FP64 rounding of a different summation order.  Within a work-group that
+ * order is the order of arrival, so two equal calls may differ in the sums'
+ * last bits.  max_shift is the largest move between the centroids as they are
+ * returned; once no label changes any more it is therefore not exactly zero
+ * but a difference of two roundings, another one on every call, at most about
+ * 2^-52 times the mass and the mean |x| of a cluster (in practice a few times
+ * 2^-52 |x|): a stopping tolerance for double points has to lie above that.
+ * (For float points the sums are exact, and a settled max_shift is 0.)
  */
 int clk_fused_f64(clk_context *ctx, const clk_kernel_config *cfg, uint64_t d,
                   uint64_t n, uint64_t k, const double *points,
