@@ -25,6 +25,10 @@ using namespace split;
 // registers.
 constexpr uint32_t split_waves(int P) { return P >= 96 ? 4 : 8; }
 
+// Waves per SIMD that the registers have to leave room for: two work-groups to
+// a CU up to 8 features, and of the four-wave ones at 96 (float points).
+constexpr uint32_t split_occupancy(int P, bool f64) { return P <= 8 ? 4 : P <= 64 || (P == 96 && !f64) ? 2 : 1; }
+
 // LDS after the table of a fused pass: scales [P] | cells [R][d*k] | flags
 // [d*k] | counts [R][k].  Float points: int64 cells of grid integers
 // (clk_grid.hpp); double points: FP64 cells, no scales or flags.  R replicas
@@ -41,7 +45,7 @@ __host__ __device__ inline size_t fused_tail_bytes(uint32_t P, uint32_t d, uint3
 // (q, h) holds features 8h .. 8h+7 of each K-block of the points q, 16+q,
 // 32+q, 48+q (the matrix core's layout).
 template <int P, bool FUSED, typename T, typename LabelT>
-__global__ void __launch_bounds__(64 * split_waves(P))
+__global__ void __launch_bounds__(64 * split_waves(P), split_occupancy(P, sizeof(T) == 8))
 split_kernel(const T *__restrict__ pts, uint64_t n, uint32_t d, uint32_t k, const T *__restrict__ cen,
              LabelT *__restrict__ labels, uint32_t ntiles, GridRef grid, uint32_t R, double *__restrict__ part,
              double *__restrict__ max_shift)
@@ -123,38 +127,52 @@ split_kernel(const T *__restrict__ pts, uint64_t n, uint32_t d, uint32_t k, cons
         PointOps<P> ops;
         float x2, best, second;
         if constexpr (P < 32)
-            x2 = build_points<P, T>(x[0], t.scale, buf, lane, ops);
+            x2 = build_points<P, T>(t, x[0], buf, lane, ops);
         else
-            x2 = build_points<P, T>(x, t.scale, lane, ops);
+            x2 = build_points<P, T>(t, x, lane, ops);
         rank_points<P, T>(t, ops, lane, best, second);
         uint32_t lab;
         float limit;
         const bool sure = decide(t, x2, best, second, k, lab, limit);
-        uint64_t open = __ballot(!sure && p < n);
+        uint64_t open = __ballot(!sure && p < n);  // points that the wave scans one by one
+        const uint32_t m = (uint32_t)__builtin_popcountll(open), rounds = (k + 63) / 64;
+        bool all = false;  // every lane scans for its own point, and the ones that are not sure take that
         if constexpr (P < 32) {
-            // Many undecided points against few centroids: every lane scans
-            // for its own point (about k (2P + 3) instructions in all, against
-            // about 150 for each point that the wave scans together).
-            if (open && k * (2 * P + 3) <= 150u * (uint32_t)__builtin_popcountll(open)) {
-                const uint32_t scanned = scan_rows<P, T>(t, x[0], d, k);
-                lab = sure ? lab : scanned;
-                open = 0;
+            // about k (2P + 3) instructions, against about 150 for each point
+            // and 64 centroids that the wave scans together (double points: the
+            // rows take twice the LDS reads; 150k points d=8 k=700 172 / 243 us
+            // without that)
+            all = open && k * (2 * P + 3) <= 150u * m * (f64 ? (rounds + 1) / 2 : rounds);
+        } else if (open) {
+            all = m > 5;  // (block_scan)
+            if constexpr (!(f64 && !FUSED && P == 32)) {  // (its registers spill)
+                // Scoring the tiles again and one exact distance a lane for each
+                // tile with candidates, against the rounds of the full scan:
+                // 188k points d=53 k=290 with clusters sharing blobs 640 ->
+                // 203 us.
+                const uint64_t known = __ballot(!sure && p < n && limit == limit);
+                const uint32_t mk = (uint32_t)__builtin_popcountll(known);
+                const uint32_t full = k > 32 ? mk * rounds : k > 16 ? (mk + 1) / 2 : (mk + 3) / 4;
+                if (m - mk <= 5 && full > min(ntiles, 2 * mk) + ntiles / 8 + 1)
+                    if (candidate_scan<P>(t, ops, known, limit, pts + bt * 64, n, cen, d, k, lane, lab)) {
+                        open &= ~known;
+                        all = false;
+                    }
             }
         }
-        if constexpr (P >= 32 && !(f64 && !FUSED && P == 32)) {  // (its registers spill)
-            // Scoring the tiles again and one exact distance a lane for each
-            // tile with candidates, against the rounds of the full scan: 188k
-            // points d=53 k=290 with clusters sharing blobs 640 -> 203 us.
-            const uint64_t known = __ballot(!sure && p < n && limit == limit);
-            const uint32_t m = (uint32_t)__builtin_popcountll(known);
-            const uint32_t full = k > 32 ? m * ((k + 63) / 64) : k > 16 ? (m + 1) / 2 : (m + 3) / 4;
-            if (full > min(ntiles, 2 * m) + ntiles / 8 + 1) {
-                candidate_scan<P>(t, ops, known, limit, pts + bt * 64, n, cen, d, k, lane, lab);
-                open &= ~known;
+        if (all) {
+            uint32_t scanned;
+            if constexpr (P < 32) {
+                scanned = scan_rows<P, T>(t, x[0], d, k);
+            } else {
+                const uint64_t left = n - 1 - bt * 64;
+                const T *own = pts + bt * 64 + min(lane, left < 63 ? (uint32_t)left : 63u);
+                scanned = block_scan(own, n, cen, d, k, lane);
             }
-        }
-        if (open)
+            lab = sure ? lab : scanned;
+        } else if (open) {
             exact_scan<P>(open, pts + bt * 64, n, cen, d, k, lane, lab);
+        }
         if (p < n)
             stream_store((LabelT)lab, labels + p);
         if constexpr (FUSED) {
@@ -275,7 +293,7 @@ SplitPlan<T> plan_for(const clk_context *ctx, uint64_t d, uint64_t k)
 template <bool FUSED, typename T>
 SplitPlan<T> split_plan(const clk_context *ctx, uint64_t d, uint64_t k)
 {
-    if (d == 0 || k == 0 || k > 65536)
+    if (d == 0 || k < 2 || k > 65536)
         return {};
     if (d <= 4)
         return plan_for<4, FUSED, T>(ctx, d, k);

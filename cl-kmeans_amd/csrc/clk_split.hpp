@@ -4,10 +4,15 @@
 // centroids in LDS.  The labels equal the sequential-fma scan's
 // (lloyd_fused_feature_sum.cl:213-239, kmeans_naive.cpp:49-63) bit for bit.
 //
-// Scores.  With a power of two s that puts max |c| into [2^12, 2^13), every
-// coordinate is split into two FP16 parts: s x = xh + xl (toward zero),
-// -2 s c = ch + cl (to nearest).  The MFMA accumulator starts at
-// RN(||s c||^2), so S_c = ||s c||^2 - 2 s^2 x.c up to a bounded error.
+// Scores.  Points and centroids are taken relative to a point m, the mean of
+// eight centroids: below, x and c stand for x - m and c - m.  (Relative to the
+// origin the scores of data far from it cancel, and nearly every point took
+// the exact scan: 150k points d=11 k=300 around 300 labeling 703 -> 28 us, 3M
+// d=8 k=64 126 -> 48; m costs about 1 us of every launch.)
+// With a power of two s that puts max |c| into [2^12, 2^13), every coordinate
+// is split into two FP16 parts: s x = xh + xl (toward zero), -2 s c = ch + cl
+// (to nearest).  The MFMA accumulator starts at RN(||s c||^2), so S_c =
+// ||s c||^2 - 2 s^2 x.c up to a bounded error.
 // K = 32 of one 16x16x32 MFMA holds, for P padded features:
 //   P = 4, 8 all four products xh ch, xh cl, xl ch, xl cl of the features;
 //   P = 16   two MFMAs, (ch | cl) against (xh | xh) and (xl | xl);
@@ -18,9 +23,11 @@
 // its low bits replaced by an index.
 //
 // Error of one score (u = 2^-24, X >= ||s x|| over the padded features, C >= max ||s c||, N >= C^2):
-//   split of x   Rx = 2^-20 X + 1.01 * 2^-24 sqrt(d)  (toward zero: 2^-10
-//                relative per part, subnormal spacing 2^-24)
-//   split of c   Rc = 2^-22 2C + 1.01 * 2^-25 sqrt(d)
+//   split of x   Rx = 1.125 * 2^-20 X + 1.01 * 2^-24 sqrt(d)  (toward zero:
+//                2^-10 relative per part, subnormal spacing 2^-24; and the
+//                rounding of x - m, 2^-24 relative)
+//   split of c   Rc = 1.3125 * 2^-22 2C + 1.01 * 2^-25 sqrt(d)  (with that of
+//                c - m)
 //   inputs       (X + Rx) Rc + Rx 2C; P >= 32 also the dropped xl cl:
 //                (2^-10 X + 2^-24 sqrt(d)) (2^-11 2C + 2^-25 sqrt(d))
 //   summation    g (N + 1.004 X 2C), g = 2(T+1)u / (1 - 2(T+1)u) for the T
@@ -29,7 +36,7 @@
 //                top of the norm and the small products), the addition of the
 //                norm 2u (N + their sum), and theirs, g' with T = 2d of
 //                (2^-10 X + 2^-24 sqrt(d)) 2C (1 + 2^-11) + X (2^-11 2C + 2^-25 sqrt(d))
-//   norm         2u N
+//   norm         4u N  (of coordinates rounded to FP32)
 // E = 1.01 x the sum + a bound on flushed denormals.  An FP16 subnormal must
 // reach the product: every launch checks that the matrix core keeps them, and
 // without that every point takes the exact scan.
@@ -42,10 +49,13 @@
 // tr' = tr / (1 - tr),
 // makes c_b the strict, unique minimum of e_c.  Every other point -- and every
 // point with a coordinate that is not finite or too large for FP16 -- scans
-// all centroids with the reference's arithmetic.
+// all centroids, or its candidates, with the reference's arithmetic: one by
+// one (exact_scan, candidate_scan), or all points of the wave at once
+// (scan_rows, block_scan), by what they cost.
 //
-// Double points (T = double): s x and -2 s c are rounded to FP32 first, 2^-24
-// relative, which Rx and Rc include; eps = (d+3) 2^-53 and the scans are FP64.
+// Double points (T = double): x - m and c - m are taken in FP64 and then
+// rounded to FP32, one rounding as well; eps = (d+3) 2^-53 and the scans are
+// FP64.
 #pragma once
 
 #include "clk_common.hpp"
@@ -73,7 +83,8 @@ struct Shape {
 };
 
 // LDS of one work-group of `waves` waves: table, norms, centroids as they are
-// (P < 32: [k][P], 0 past d), statistics, exchange.
+// (P < 32: [k][P], 0 past d), m (past d that of feature d - 1), statistics,
+// exchange.
 template <int P>
 __host__ __device__ constexpr size_t table_bytes(uint32_t ntiles)
 {
@@ -88,7 +99,7 @@ __host__ __device__ constexpr size_t rows_bytes(uint32_t ntiles)
 template <int P, typename T>
 __host__ __device__ constexpr size_t lds_bytes(uint32_t ntiles, uint32_t waves)
 {
-    return table_bytes<P>(ntiles) + rows_bytes<P, T>(ntiles) + (size_t)ntiles * 16 * sizeof(float) +
+    return table_bytes<P>(ntiles) + rows_bytes<P, T>(ntiles) + (size_t)ntiles * 16 * sizeof(float) + P * sizeof(T) +
            kStatWords * sizeof(float) +
            (size_t)waves * Shape<P>::planes * 64 * sizeof(u16x8);
 }
@@ -153,6 +164,7 @@ struct Table {
     const u16x8 *ops;
     const float *norm;
     const T *rows;
+    const T *mean;  // m
     uint32_t ntiles, kmask;
     float scale;    // s
     // the margin: t0 + tX ||s x|| + tx2 ||s x||^2 + tk (|vb| + |vs|)
@@ -171,11 +183,11 @@ __device__ __forceinline__ void set_margin(Table<T> &t, float N, uint32_t d, uin
     const float terms = (float)(Shape<P>::terms * d);
     const float g0 = 2.0f * (terms + 1.0f) * mfma::kU;
     const float gamma = g0 / (1.0f - g0) * up;
-    constexpr float alpha = f64 ? 0x1.2p-20f : 0x1p-20f;
+    constexpr float alpha = 0x1.2p-20f;
     const float beta = 1.01f * 0x1p-24f * sd;
-    const float Rc = (f64 ? 0x1.5p-22f : 0x1p-22f) * C2 + 1.01f * 0x1p-25f * sd;
+    const float Rc = 0x1.5p-22f * C2 + 1.01f * 0x1p-25f * sd;
     float e1 = (1.0f + alpha) * Rc + alpha * C2 + gamma * 1.004f * C2;
-    float e0 = beta * (Rc + C2) + (gamma + 2.0f * mfma::kU) * N;
+    float e0 = beta * (Rc + C2) + (gamma + 4.0f * mfma::kU) * N;
     if constexpr (P >= 32) {
         const float m = 0x1p-11f * C2 + 0x1p-25f * sd;
         e1 += 0x1p-10f * m;
@@ -211,25 +223,45 @@ __device__ __forceinline__ Table<T> stage(const T *__restrict__ cen, uint32_t d,
     u16x8 *ops = reinterpret_cast<u16x8 *>(lds);
     float *norm = reinterpret_cast<float *>(lds + table_bytes<P>(ntiles));
     T *rows = reinterpret_cast<T *>(norm + ntiles * 16);
-    uint32_t *stat = reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(rows) + rows_bytes<P, T>(ntiles));
-    const uint32_t tid = threadIdx.x, B = blockDim.x;
+    T *mean = reinterpret_cast<T *>(reinterpret_cast<char *>(rows) + rows_bytes<P, T>(ntiles));
+    uint32_t *stat = reinterpret_cast<uint32_t *>(mean + P);
+    const uint32_t tid = threadIdx.x, B = blockDim.x, dk = d * k;
     if (tid < kStatWords)
         stat[tid] = 0;
-    __syncthreads();
-    // stat[0]: max |c| over the finite coordinates
-    uint32_t m = 0;
-#pragma unroll 4
-    for (uint32_t i = tid; i < d * k; i += B) {
-        if constexpr (f64) {
-            // beyond FP32: as its largest value, which no scale takes
-            const double a = __builtin_fabs(cen[i]);
-            const uint32_t u = __float_as_uint((float)(a < (double)FLT_MAX ? a : (double)FLT_MAX));
-            m = (a <= DBL_MAX && u > m) ? u : m;
-        } else {
-            const uint32_t u = __float_as_uint(__builtin_fabsf(cen[i]));
-            m = (u < 0x7F800000u && u > m) ? u : m;
+    // m: the mean of 8 centroids (an eighth of each: no sum overflows)
+    constexpr uint32_t kSample = 8, kFirst = 4;
+    T first[kFirst];  // of the next pass, loaded with them
+#pragma unroll
+    for (uint32_t j = 0; j < kFirst; ++j)
+        first[j] = cen[min(tid + j * B, dk - 1)];
+    if (tid < P) {
+        T sum = 0;
+#pragma unroll
+        for (uint32_t j = 0; j < kSample; ++j) {
+            const T v = cen[min(tid, d - 1) * k + j * k / kSample];
+            sum += __builtin_fabs(v) <= kMax ? v * (T)(1.0 / kSample) : (T)0;
         }
+        mean[tid] = sum;
     }
+    __syncthreads();
+    // stat[0]: max |c - m| over the finite coordinates; beyond FP32 its largest
+    // value, which no scale takes
+    uint32_t m = 0;
+    const float per_row = 1.0f / (float)k;
+    // i / k: i < 2^18, so the product is off by less than the half added
+    auto row_of = [&](uint32_t i) { return (uint32_t)(((float)i + 0.5f) * per_row); };
+    auto take = [&](T v, uint32_t i) {
+        const T a = v - mean[row_of(i)];
+        const uint32_t u = min(__float_as_uint(__builtin_fabsf((float)a)), 0x7F7FFFFFu);
+        m = (__builtin_fabs(v) <= kMax && u > m) ? u : m;
+    };
+#pragma unroll
+    for (uint32_t j = 0; j < kFirst; ++j)
+        if (tid + j * B < dk)
+            take(first[j], tid + j * B);
+#pragma unroll 2
+    for (uint32_t i = tid + kFirst * B; i < dk; i += B)
+        take(cen[i], i);
     for (int o = 32; o >= 1; o /= 2)
         m = max(m, (uint32_t)__shfl_xor((int)m, o));
     if (tid % 64 == 0 && m)
@@ -250,10 +282,9 @@ __device__ __forceinline__ Table<T> stage(const T *__restrict__ cen, uint32_t d,
             // P = 4: (ch | cl) in the first two quarters, zeros in the others
             const uint32_t f = P == 4 ? j % 4 : f0 + j;
             const bool lo = P == 4 ? j >= 4 : low;
-            const bool in = c < k && f < d && (P != 4 || h < 2);
-            const T raw = cen[in ? (size_t)f * k + c : 0];
-            const bool fin = raw <= kMax && raw >= -kMax;
-            float x = in && fin ? (float)((T)(-2.0f * s) * raw) : 0.0f;
+            const T raw = cen[min(f * k + c, dk - 1)];
+            const bool in = c < k && f < d && (P != 4 || h < 2) && __builtin_fabs(raw) <= kMax;
+            float x = in ? -2.0f * s * (float)(T)(raw - mean[f]) : 0.0f;
             // both parts come from the FP32 value: the compiler would round a
             // double to FP16 at once for the high part, and not to the same
             // neighbour when the FP32 value lies between two
@@ -267,19 +298,18 @@ __device__ __forceinline__ Table<T> stage(const T *__restrict__ cen, uint32_t d,
     }
     if constexpr (P < 32)
         for (uint32_t i = tid; i < k * P; i += B) {
-            const uint32_t c = i % k, f = i / k;
-            rows[c * P + f] = f < d ? cen[(size_t)f * k + c] : (T)0;
+            const uint32_t f = row_of(i), c = i - f * k;
+            rows[c * P + f] = f < d ? cen[min(i, dk - 1)] : (T)0;
         }
     uint32_t nmax = 0;
     for (uint32_t c = tid; c < ntiles * 16; c += B) {
         double q = 0.0;
         bool fin = c < k;
-        const T *col = cen + (fin ? c : 0);
 #pragma unroll 8
         for (uint32_t f = 0; f < d; ++f) {
-            const T v = col[(size_t)f * k];
-            fin = fin && v <= kMax && v >= -kMax;
-            const double w = (double)(v * (T)s);
+            const T v = cen[min(f * k + c, dk - 1)];
+            fin = fin && __builtin_fabs(v) <= kMax;
+            const double w = f64 ? (double)(v - mean[f]) * (double)s : (double)((float)(v - mean[f]) * s);
             q = __builtin_fma(w, w, q);
         }
         norm[c] = fin ? (float)q : kNever;
@@ -303,6 +333,7 @@ __device__ __forceinline__ Table<T> stage(const T *__restrict__ cen, uint32_t d,
     t.ops = ops;
     t.norm = norm;
     t.rows = rows;
+    t.mean = mean;
     t.ntiles = ntiles;
     uint32_t bits = 4;
     while ((1u << bits) < ntiles * 16)
@@ -332,7 +363,7 @@ struct PointOps {
 // the point's coordinates again: the centroids are 0 there).  buf: this wave's
 // exchange planes.  Returns a bound >= ||s x||^2.
 template <int P, typename T>
-__device__ __forceinline__ float build_points(const T (&x)[P], float s, u16x8 *buf, uint32_t lane,
+__device__ __forceinline__ float build_points(const Table<T> &t, const T (&x)[P], u16x8 *buf, uint32_t lane,
                                               PointOps<P> &o)
 {
     static_assert(P < 32, "lane = point form");
@@ -340,7 +371,7 @@ __device__ __forceinline__ float build_points(const T (&x)[P], float s, u16x8 *b
     uint32_t hi[P / 2], lo[P / 2];
 #pragma unroll
     for (int f = 0; f < P; f += 2) {
-        const float a = (float)(x[f] * (T)s), b = (float)(x[f + 1] * (T)s);
+        const float a = (float)(x[f] - t.mean[f]) * t.scale, b = (float)(x[f + 1] - t.mean[f + 1]) * t.scale;
         x2 = __builtin_fmaf(a, a, x2);
         x2 = __builtin_fmaf(b, b, x2);
         split2(a, b, hi[f / 2], lo[f / 2]);
@@ -382,11 +413,12 @@ __device__ __forceinline__ float build_points(const T (&x)[P], float s, u16x8 *b
 // point g*16 + q (past d as above).  Returns a bound >= ||s x||^2 of this
 // lane's own point (lane 16h + q).
 template <int P, typename T>
-__device__ __forceinline__ float build_points(const T (&raw)[4][Shape<P>::nkb * 8], float s, uint32_t lane,
+__device__ __forceinline__ float build_points(const Table<T> &t, const T (&raw)[4][Shape<P>::nkb * 8], uint32_t lane,
                                               PointOps<P> &o)
 {
     static_assert(P >= 32, "matrix layout");
     float mine = 0.0f;
+    const T *const mean = t.mean + 8 * (lane / 16);
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
         float x2 = 0.0f;
@@ -395,7 +427,8 @@ __device__ __forceinline__ float build_points(const T (&raw)[4][Shape<P>::nkb * 
             v4u hi, lo;
 #pragma unroll
             for (int j = 0; j < 8; j += 2) {
-                const float a = (float)(raw[g][kb * 8 + j] * (T)s), b = (float)(raw[g][kb * 8 + j + 1] * (T)s);
+                const float a = (float)(raw[g][kb * 8 + j] - mean[kb * 32 + j]) * t.scale;
+                const float b = (float)(raw[g][kb * 8 + j + 1] - mean[kb * 32 + j + 1]) * t.scale;
                 x2 = __builtin_fmaf(a, a, x2);
                 x2 = __builtin_fmaf(b, b, x2);
                 uint32_t h, l;
@@ -604,12 +637,86 @@ __device__ __forceinline__ void exact_scan(uint64_t open, const T *__restrict__ 
     }
 }
 
+// Lane I of this lane's row of 16.
+template <int I, typename T>
+__device__ __forceinline__ T row_lane(T v)
+{
+    constexpr int kRowNewBcast = 0x150;
+    if constexpr (sizeof(T) == 8)
+        return __builtin_amdgcn_update_dpp(v, v, kRowNewBcast + I, 0xf, 0xf, true);
+    else
+        return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), kRowNewBcast + I, 0xf, 0xf, true));
+}
+
+template <int I, int CB, typename T>
+__device__ __forceinline__ void add_squares(T xv, T cv, T (&dist)[CB])
+{
+    const T u = row_lane<I>(cv) - xv;  // the square of x - c, whichever its sign
+    if constexpr (sizeof(T) == 8)
+        dist[I] = __builtin_fma(u, u, dist[I]);
+    else
+        dist[I] = __builtin_fmaf(u, u, dist[I]);
+    if constexpr (I + 1 < CB)
+        add_squares<I + 1, CB>(xv, cv, dist);
+}
+
+// The reference's scan, over all centroids, of all the wave's points: lane =
+// point (x: its feature 0, the rows n apart), 16 centroids at a time, one in
+// every lane of each row of 16 lanes, from where the subtraction broadcasts
+// it; the loads four features ahead.  Vector operations bound it, 2 k d for
+// the 64 points, where exact_scan takes 2 d loads for each point and 64
+// centroids: it is the faster one from about six points on (1M equal points
+// d=20 k=130, double, labeling 4185 -> 409 us; 1M d=32 k=64 out of the scores'
+// range 1351 -> 191, the plain kernel 113).
+template <typename T>
+__device__ __forceinline__ uint32_t block_scan(const T *__restrict__ x, uint64_t n, const T *__restrict__ cen,
+                                               uint32_t d, uint32_t k, uint32_t lane)
+{
+    constexpr int kBlock = 16;
+    constexpr uint32_t kAhead = 4;
+    T best = sizeof(T) == 8 ? (T)DBL_MAX : (T)FLT_MAX;
+    uint32_t lab = 0;
+    for (uint32_t c0 = 0; c0 < k; c0 += kBlock) {
+        const T *const col = cen + min(c0 + lane % kBlock, k - 1);  // the last centroid again: never less than itself
+        T dist[kBlock], xv[kAhead], cv[kAhead];
+#pragma unroll
+        for (int i = 0; i < kBlock; ++i)
+            dist[i] = 0;
+        auto load = [&](uint32_t j, uint32_t f) {
+            xv[j] = x[(uint64_t)min(f, d - 1) * n];
+            cv[j] = col[(size_t)min(f, d - 1) * k];
+        };
+#pragma unroll
+        for (uint32_t j = 0; j < kAhead; ++j)
+            load(j, j);
+        uint32_t f = 0;
+        for (; f + kAhead <= d; f += kAhead)
+#pragma unroll
+            for (uint32_t j = 0; j < kAhead; ++j) {
+                add_squares<0, kBlock>(xv[j], cv[j], dist);
+                load(j, f + kAhead + j);
+            }
+#pragma unroll
+        for (uint32_t j = 0; j < kAhead - 1; ++j)
+            if (f + j < d)
+                add_squares<0, kBlock>(xv[j], cv[j], dist);
+#pragma unroll
+        for (int i = 0; i < kBlock; ++i)
+            if (dist[i] < best) {
+                best = dist[i];
+                lab = c0 + i;
+            }
+    }
+    return lab;
+}
+
 // The points of open settled among the centroids that their limits leave
 // (usually two or three): the tiles are scored again, and every lane takes the
 // exact distances of its rows' candidates, its own point and centroid each.
-// base as in exact_scan.
+// base as in exact_scan.  false, with lab as it was: a lane has more than six
+// candidates in a tile, the scan of all centroids is the cheaper one.
 template <int P, typename T>
-__device__ __forceinline__ void candidate_scan(const Table<T> &t, const PointOps<P> &ops, uint64_t open, float limit,
+__device__ __forceinline__ bool candidate_scan(const Table<T> &t, const PointOps<P> &ops, uint64_t open, float limit,
                                                const T *__restrict__ base, uint64_t n, const T *__restrict__ cen,
                                                uint32_t d, uint32_t k, uint32_t lane, uint32_t &lab)
 {
@@ -642,6 +749,8 @@ __device__ __forceinline__ void candidate_scan(const Table<T> &t, const PointOps
                 cand |= (in ? 1u : 0u) << (4 * g + i);
             }
         cand &= live;
+        if (__ballot(__builtin_popcount(cand) > 6))
+            return false;
         while (cand) {
             const uint32_t bit = (uint32_t)__builtin_ctz(cand), g = bit / 4;
             cand &= cand - 1;
@@ -688,6 +797,7 @@ __device__ __forceinline__ void candidate_scan(const Table<T> &t, const PointOps
         if ((uint32_t)g == h && ((open >> lane) & 1))
             lab = c;
     }
+    return true;
 }
 
 // The reference's scan of this lane's own point x over the staged rows.
