@@ -707,9 +707,11 @@ int launch_labeling_mfma(clk_context *ctx, bool fp16, uint64_t d, uint64_t n, ui
                            qidx, qthr, qlen, hint_in, hint_out, qbuf_ok, pin_ops, pin_x2);
         CLK_HIP_CHECK(hipGetLastError());
     }
-    // a resident grid; blocks past the queue return at once
+    // a resident grid, a work-group per batch of 64 points (8000 points d=24
+    // k=16, all queued: 25 us with a quarter of them, 10 now); those past the
+    // queue return at once
     const int refine_block = 64 * kRefineWaves;
-    const uint64_t grid_r = auto_grid(ctx, (const void *)rk, refine_block, lds_r, div_up(n, (uint64_t)64) * 64);
+    const uint64_t grid_r = auto_grid(ctx, (const void *)rk, refine_block, lds_r, div_up(n, (uint64_t)64) * refine_block);
     KernelTimer t(ctx, "LabelingMfmaRefine", stream);
     hipLaunchKernelGGL(rk, dim3((unsigned)grid_r), dim3(refine_block), lds_r, stream, points, n,
                        (uint32_t)d, (uint32_t)k, cenT, table, norm, tiles, l.ntiles, prm, labels,
