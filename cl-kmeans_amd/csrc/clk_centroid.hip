@@ -433,17 +433,25 @@ struct CellPlan {
     size_t lds = 0;
 };
 
+// Points of a work-group at least: it writes F*k doubles.
+uint64_t cell_points(uint64_t k) { return std::max<uint64_t>(4 * k, 64 * kCellWaves); }
+
 // The widest slice whose cells leave a CU two work-groups (every wave slot):
 // each slice reads the labels again, and loads of more features overlap.
-// Else the narrowest slice that fits at all.  Replicas as far as a CU keeps
-// its two work-groups and k is small enough for a wave's labels to meet.
-CellPlan cell_plan(const clk_context *ctx, uint64_t d, uint64_t k)
+// Else the narrowest slice that fits at all.  Narrower where the points give
+// the slices less than half a work-group per CU: a few work-groups then take
+// one wave's additions after another (3000 points d=64 k=300 12 -> 4.6 us, all
+// in one cluster 24 -> 6.3; d=128 k=130 10.9 -> 5.8).  Replicas as far as a CU
+// keeps its two work-groups and k is small enough for a wave's labels to meet.
+CellPlan cell_plan(const clk_context *ctx, uint64_t d, uint64_t n, uint64_t k)
 {
     CellPlan p;
     const uint32_t widest = d >= 16 ? 16 : d > 4 ? 8 : d > 2 ? 4 : (uint32_t)d;
     for (uint32_t F = widest; F >= 1 && !p.F; F /= 2)
         if (cell_lds_bytes(F, k, 1) <= ctx->lds_per_block / 2 || (F == 1 && cell_lds_bytes(1, k, 1) <= ctx->lds_per_block))
             p.F = F;
+    while (p.F > 1 && div_up(d, p.F) * (n / cell_points(k)) < (uint64_t)ctx->num_cus / 2)
+        p.F /= 2;
     switch (p.F) {
     case 1: p.kern = cu_cell_kernel<1>; break;
     case 2: p.kern = cu_cell_kernel<2>; break;
@@ -543,7 +551,7 @@ int run_centroid_update(clk_context *ctx, const clk_kernel_config *cfg, uint64_t
     // a launch geometry of the caller's names the strategy's own kernel
     const bool automatic = !(cfg && (cfg->global_size[0] || (cfg->local_size[0] && cfg->local_size[0] != 256)));
     const bool private_fits = dmax && dk < (1ull << 24) && head + dk * B * 4 <= ctx->lds_per_block;
-    const CellPlan cells = cell_plan(ctx, d, k);
+    const CellPlan cells = cell_plan(ctx, d, n, k);
     const bool take_cells = cells.kern && automatic && !(private_fits && private_pays(ctx, n, dk, head + dk * B * 4));
     if (!take_cells && private_fits && (automatic || strategy == CLK_CENTROID_CLUSTER_MERGE)) {
         const int vec = std::min(pick_vector_width(cfg ? cfg->vector_length : 4), cm_vec_cap(dmax));
@@ -593,14 +601,21 @@ int run_centroid_update(clk_context *ctx, const clk_kernel_config *cfg, uint64_t
         if (cells.lds > 65536)
             CLK_HIP_CHECK(hipFuncSetAttribute((const void *)cells.kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                                               (int)cells.lds));
-        // a resident grid over the slices; a work-group takes at least 4k
-        // points (it writes F*k doubles)
+        // A resident grid over the slices; a work-group takes at least
+        // cell_points, up to 16k points where one per CU is enough (each writes
+        // F*k doubles, which the merge reads: 400k points d=32 k=256 26 -> 21
+        // us, 50k d=128 k=130 17.6 -> 14.5).
         const uint64_t gy = div_up(d, (uint64_t)cells.F);
         uint64_t gxs = auto_grid(ctx, (const void *)cells.kern, 64 * kCellWaves, cells.lds, n * gy) / gy;
-        gxs = std::min<uint64_t>(gxs, div_up(n, std::max<uint64_t>(4 * k, 64 * kCellWaves)));
+        uint64_t share = cell_points(k);
+        while (gy * div_up(n, share) > (uint64_t)ctx->num_cus && share < 16 * k)
+            share *= 2;
+        gxs = std::min<uint64_t>(gxs, div_up(n, share));
         gxs = std::max<uint64_t>(1, std::min<uint64_t>(gxs, 65535));
-        // Few points: one work-group per slice, which adds its sums itself --
-
+        // Few points: one work-group per slice, which adds its sums itself.
+        // Its waves take the points one after another, so it pays up to about
+        // what the merge's launch costs: 8192 points d=4 k=10 33.6 us a step
+        // through the separate operators against 35.8, 16k d=8 k=30 even.
         const bool direct = n * cells.F <= 32768 && n <= 16384;
         if (direct)
             gxs = 1;
