@@ -355,8 +355,9 @@ bool split_labeling_pays(const clk_context *ctx, const clk_kernel_config *cfg, u
     // unless said).  Labeling: d=4 k=20 18.3 / 13.7, k=32 17.6 / 18.7; d=8
     // k=16 17.8 / 20.8; d=16 k=16 31 / 39; d=32 k=10 60 / 55, k=16 55 / 65;
     // with one or two features the plain scan's 2d + 3 operations per centroid
-    // stay below the ranking's.  Fused step: d=16 k=5 61 / 50, k=10 52 / 73; d=32 k=32 88 / 190; 300k
-    // points d=16 k=3 22 / 35.
+    // stay below the ranking's.  Fused step: d=16 k=5 61 / 50, k=10 52 / 73;
+    // d=32 k=32 88 / 190; 300k points d=16 k=3 22 / 35, but two clusters of more
+    // than 16 features 400k d=32 75 / 54, 1M d=20 57 / 48.
     // One feature: the gaps sink below the keys' truncation (2M points k=8 20 /
     // 11, k=20 26 / 12, 274k k=238 81 / 45); the plain scan takes 5 operations
     // a centroid.
@@ -367,7 +368,8 @@ bool split_labeling_pays(const clk_context *ctx, const clk_kernel_config *cfg, u
     if (fused && d <= 4)
         return d >= 3 && k >= 48 && split_plan<true, float>(ctx, d, k).kern != nullptr;
     if (fused)
-        return (k >= 6 || (n <= (1u << 20) && k >= 2)) && split_plan<true, float>(ctx, d, k).kern != nullptr;
+        return (k >= 6 || (n <= (1u << 20) && k >= (d > 16 ? 3u : 2u))) &&
+               split_plan<true, float>(ctx, d, k).kern != nullptr;
     const uint64_t bucket = split_bucket(d);
     return n >= 4096 && d >= 3 && k * (2 * bucket + 3) >= 300 + 20 * bucket &&
            split_plan<false, float>(ctx, d, k).kern != nullptr;
