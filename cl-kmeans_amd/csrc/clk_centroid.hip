@@ -10,11 +10,11 @@
 //   feature_sum         one LDS accumulator [d][k] shared by the work-group,
 //                       work-items stride over the flattened feature-major
 //                       matrix (coalesced rows)
-// With an automatic launch geometry every strategy takes the kernel that is
-// fastest for the sizes (the results are the same): cluster_merge's private
+// With every launch key at its default (names_kernel) each strategy takes the
+// kernel that is fastest for the sizes (the results are the same): cluster_merge's private
 // tile for a few cells, else the cell kernel below, which shares the
 // accumulators of a slice of features; the strategies' own kernels serve the
-// launch geometries that name them.
+// launch keys that name them.
 // Every coordinate is rounded to its grid integer and added exactly
 // (clk_grid.hpp): the private int32 columns flush into the work-group's
 // int64 accumulator (ds_add_u64) at least every 64 values, shared
@@ -548,8 +548,7 @@ int run_centroid_update(clk_context *ctx, const clk_kernel_config *cfg, uint64_t
     uint32_t tf = 1;
     uint64_t gx = 0;
 
-    // a launch geometry of the caller's names the strategy's own kernel
-    const bool automatic = !(cfg && (cfg->global_size[0] || (cfg->local_size[0] && cfg->local_size[0] != 256)));
+    const bool automatic = !names_kernel(cfg);
     const bool private_fits = dmax && dk < (1ull << 24) && head + dk * B * 4 <= ctx->lds_per_block;
     const CellPlan cells = cell_plan(ctx, d, n, k);
     const bool take_cells = cells.kern && automatic && !(private_fits && private_pays(ctx, n, dk, head + dk * B * 4));

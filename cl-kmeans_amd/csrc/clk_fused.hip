@@ -387,7 +387,7 @@ int run_fused(clk_context *ctx, const clk_kernel_config *cfg, uint64_t d, uint64
     const char *name = !use_private  ? "FusedFeatureSum"
                        : run_bounded ? "FusedClusterMergeBounded"
                                      : "FusedClusterMerge";
-    bool use_shared = dmax && !use_private && k * d < (1ull << 24) && shared_bytes <= ctx->lds_per_block;
+    const bool use_shared = dmax && !use_private && k * d < (1ull << 24) && shared_bytes <= ctx->lds_per_block;
 
     CLK_REQUIRE(!ext || use_private || use_shared || n == 0, CLK_ERR_UNSUPPORTED,
                 "lloyd_step_noalloc: k*d beyond the work-group LDS tiles (the separate stages allocate)");
@@ -418,18 +418,14 @@ int run_fused(clk_context *ctx, const clk_kernel_config *cfg, uint64_t d, uint64
     // cells' atomics below (private / shared, us: 20k points d=2 k=10 13.4 /
     // 6.8; 1M d=4 k=10 19.6 / 13.0, d=3 k=5 22 / 12; 3M d=4 k=10 26.9 / 25.1;
     // but 16M d=4 k=10 84 / 101, d=2 k=10 54 / 66; one work-group, d=4 k=24
-    // 241 / 120).  An explicit launch geometry names the strategy's kernel.
+    // 241 / 120).  A launch key off its default names the strategy's kernel.
     const bool two_groups = 2 * priv_bytes <= ctx->lds_per_block;
-    const bool geometry = cfg && (cfg->global_size[0] || (cfg->local_size[0] && cfg->local_size[0] != 256));
-    if (d <= 4 && !geometry && use_private && !(n >= (4u << 20) && two_groups)) {
+    if (d <= 4 && !names_kernel(cfg) && use_private && !(n >= (4u << 20) && two_groups))
         use_private = run_bounded = false;
-        use_shared = true;
-    }
     // The bounded pass is the faster one on settled labels where it keeps two
-    // work-groups per CU and the points dwarf its fixed costs (16M points,
-    // d=4 k=10: 84 us against 110-124 with split labels; d=8 k=8 123 / 146-188;
-    // but d=4 k=16, one work-group: 185 / 105-125, and 1M points d=4 k=10:
-    // 26 / 18-20).
+    // work-groups per CU and the points dwarf its fixed costs (16M points, d=8
+    // k=8: 123 us against 146-188 with split labels; d <= 4 takes those from k
+    // = 48 only, where one private tile fills the CU).
     const bool split = !(run_bounded && n >= (4u << 20) && two_groups) &&
                        split_labeling_pays(ctx, cfg, d, n, k, true);
     FusedKernel kern = !use_private ? pick_fused<false, false>(dmax, exact, vec, b256)

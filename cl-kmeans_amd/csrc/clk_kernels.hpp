@@ -20,6 +20,16 @@ inline int dmax_bucket(uint64_t d)
     return ((uint64_t)b >= d) ? b : 0;
 }
 
+// Whether a launch key is off its default and so names the strategy's own
+// kernel; else the fastest kernel for the sizes may stand in for it (the same
+// results).  A local_size of 256 is the default and cannot be told from it.
+inline bool names_kernel(const clk_kernel_config *cfg)
+{
+    return cfg && (cfg->global_size[0] || (cfg->local_size[0] && cfg->local_size[0] != 256) ||
+                   (cfg->vector_length && pick_vector_width(cfg->vector_length) != 4) || cfg->local_features > 1 ||
+                   cfg->thread_features > 1);
+}
+
 // Labels every point with the reference arithmetic; used by the fused ops
 // for the global-accumulation variant and by clk_labeling.
 // bounded: the "unroll_vector_bounded" variant (labels read first, kept

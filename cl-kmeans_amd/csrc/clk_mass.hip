@@ -212,12 +212,12 @@ int run_mass_update(clk_context *ctx, const clk_kernel_config *cfg, uint64_t n, 
     const int vec = pick_vector_width(cfg ? cfg->vector_length : 4);
     const uint64_t user_grid = (cfg && cfg->global_size[0]) ? div_up(cfg->global_size[0], B) : 0;
 
-    // An automatic launch geometry takes the histogram kernel under every
+    // Launch keys at their defaults take the histogram kernel under every
     // strategy (the counts are exact integers): the per-label global atomics of
     // global_atomic and part_global meet on a few addresses, at about 45 ns
     // each (20M labels, k=36: 50 ms per call; this kernel and the merge about
     // 35 us).
-    const bool automatic = !(cfg && (cfg->global_size[0] || (cfg->local_size[0] && cfg->local_size[0] != 256)));
+    const bool automatic = !names_kernel(cfg);
     if (automatic && strategy >= CLK_MASS_GLOBAL_ATOMIC && strategy <= CLK_MASS_PART_PRIVATE &&
         k * 4 <= 65536) {
         uint32_t R = 1;

@@ -346,8 +346,7 @@ int launch_split(clk_context *ctx, const SplitPlan<T> &p, const char *name, uint
 bool split_labeling_pays(const clk_context *ctx, const clk_kernel_config *cfg, uint64_t d, uint64_t n, uint64_t k,
                          bool fused)
 {
-    // an explicit launch geometry names the plain kernels' one
-    if (cfg && (cfg->global_size[0] || (cfg->local_size[0] && cfg->local_size[0] != 256)))
+    if (names_kernel(cfg))
         return false;
     if (d > 16 && n * d > (1ull << 30))  // 32-bit row offsets
         return false;

@@ -97,6 +97,12 @@ typedef struct clk_context clk_context;
  * mass_update_configuration.hpp:18-25, centroid_update_configuration.hpp:18-27)
  * minus platform/device.  A size of 0 means "choose for this GPU".
  * global_size counts work-items (threads), as in the reference.
+ * With every key at its default (global_size 0, local_size 0 or 256,
+ * vector_length 0, 4 or 8, local_features and thread_features 0 or 1) the
+ * library takes the kernel that is fastest for the sizes, whichever strategy
+ * is named: the results are the same, and timing records keep the strategy's
+ * name.  To time a strategy's own kernel, set one of the keys (for instance
+ * global_size).
  */
 typedef struct clk_kernel_config {
     int32_t stage;
