@@ -616,10 +616,11 @@ int run_centroid_update(clk_context *ctx, const clk_kernel_config *cfg, uint64_t
         // what the merge's launch costs: 8192 points d=4 k=10 33.6 us a step
         // through the separate operators against 35.8, 16k d=8 k=30 even.
         const bool direct = n * cells.F <= 32768 && n <= 16384;
+        // (the global atomics need no scratch memory)
         if (direct)
             gxs = 1;
-        else
-            CLK_TRY(ensure_scratch(ctx->part_sums, gxs * dk * sizeof(double)));
+        else if (!try_scratch(ctx->part_sums, gxs * dk * sizeof(double), stream))
+            return launch_accumulate_global(ctx, d, n, k, points, labels, sg, sums, nullptr, stream);
         double *ps = direct ? sums : static_cast<double *>(ctx->part_sums.ptr);
         {
             KernelTimer t(ctx, kCellNames[strategy], stream);

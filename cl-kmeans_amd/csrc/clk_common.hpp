@@ -99,6 +99,9 @@ int enter(clk_context *ctx);
 
 // Grow a scratch buffer to at least `bytes` (hipMalloc; never shrinks).
 int ensure_scratch(Scratch &s, size_t bytes);
+// For ops that can do without: false, and no error, where the buffer is too
+// small and cannot grow now (no memory left, or stream is being captured).
+bool try_scratch(Scratch &s, size_t bytes, hipStream_t stream);
 
 // Bracket one kernel launch with timing events when profiling is on.
 struct KernelTimer {

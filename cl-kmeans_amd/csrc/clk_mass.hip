@@ -229,10 +229,15 @@ int run_mass_update(clk_context *ctx, const clk_kernel_config *cfg, uint64_t n, 
         // straight into the masses (same-address atomics: 32 x 45 ns, against
         // the merge's launch).
         uint64_t grid = auto_grid(ctx, (const void *)mass_hist_kernel<false>, 64 * kHistWaves, lds, div_up(n, 16));
-        const bool direct = grid <= 32;
+        bool direct = grid <= 32;
+        const size_t bytes = grid * k * sizeof(uint32_t);
+        // global_atomic needs no scratch memory: where there is none, every
+        // work-group adds straight into the masses
+        if (!direct && strategy == CLK_MASS_GLOBAL_ATOMIC)
+            direct = !try_scratch(ctx->part_masses, bytes, stream);
         uint32_t *out = masses;
         if (!direct) {
-            CLK_TRY(ensure_scratch(ctx->part_masses, grid * k * sizeof(uint32_t)));
+            CLK_TRY(ensure_scratch(ctx->part_masses, bytes));
             out = static_cast<uint32_t *>(ctx->part_masses.ptr);
         }
         {

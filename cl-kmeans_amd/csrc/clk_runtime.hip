@@ -43,6 +43,18 @@ int ensure_scratch(Scratch &s, size_t bytes)
     return CLK_OK;
 }
 
+bool try_scratch(Scratch &s, size_t bytes, hipStream_t stream)
+{
+    if (s.bytes >= bytes)
+        return true;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    const bool free_stream = hipStreamIsCapturing(stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone;
+    const bool grown = free_stream && ensure_scratch(s, bytes) == CLK_OK;
+    if (!grown)
+        (void)hipGetLastError();
+    return grown;
+}
+
 static hipEvent_t take_event(clk_context *ctx)
 {
     if (!ctx->event_pool.empty()) {
