@@ -67,8 +67,7 @@ struct clk_context {
     clk::Scratch part_masses;     // per-block uint32 partial masses
     clk::Scratch mfma_tables;     // 16-bit centroid operand table, norms, bounds
     clk::Scratch mfma_queue;      // point ids queued for exact refinement
-    clk::Scratch mfma_hint;       // largest per-wave score offset K of the last two MFMA labelings
-    uint32_t mfma_turn = 0;       // which of them the last one recorded
+    clk::Scratch mfma_hint;       // largest per-wave score offset K of the last MFMA labeling, and of the one before
     uint32_t *mfma_qlen = nullptr;  // device queue length inside mfma_tables
     clk::Scratch mfma_pin;        // pinned 16-bit operand copy of points (clk_labeling_pin_points)
     const void *mfma_pin_src = nullptr;  // the points it was built from (null: none)

@@ -90,7 +90,9 @@ __global__ void __launch_bounds__(64) mfma_subnormal_check_kernel(float *out)
 //   tiles[t] = the tile's maxima of ||c||^2 and ||c̃ + 2c||^2 and whether a
 //             centroid with finite coordinates had to be left out (its 16-bit
 //             or squared norm overflows): then every point is scanned exactly
-//   *qlen = 0, and the score offset this labeling will record, hint = 0.
+//   *qlen = 0; hint[1] = the score offset that the last labeling recorded in
+//   hint[0], which is cleared for this one (handed over on the device, so that
+//   a captured labeling finds that of its last replay).
 // The labeling and refinement work-groups reduce tiles[] themselves
 // (load_stats), so there is no launch to clear or finish anything (three
 // launches took 28 us at d = 64, k = 1024).
@@ -112,7 +114,8 @@ mfma_prepare_kernel(const float *__restrict__ cen, uint32_t d, uint32_t k, uint3
     const uint32_t tid = threadIdx.x, t = blockIdx.x;
     if (t == 0 && tid == 0) {
         *qlen = 0;
-        *hint = 0.0f;
+        hint[1] = hint[0];  // the last labeling's, for this one
+        hint[0] = 0.0f;
     }
     for (uint32_t e = tid; e < nkb * 64; e += 256) {
         const uint32_t lane = e % 64, kb = e / 64;
@@ -658,18 +661,14 @@ int launch_labeling_mfma(clk_context *ctx, bool fp16, uint64_t d, uint64_t n, ui
         CLK_TRY(ensure_scratch(ctx->mfma_hint, 256));
         CLK_TRY(clk_fill_zero(ctx, ctx->mfma_hint.ptr, 256, stream));
     }
-    // two words in turn: the last labeling's offset is read while this one's
-    // is recorded
-    ctx->mfma_turn ^= 1;
-    float *hint_out = static_cast<float *>(ctx->mfma_hint.ptr) + ctx->mfma_turn;
-    const float *hint_in = static_cast<float *>(ctx->mfma_hint.ptr) + (ctx->mfma_turn ^ 1);
+    float *hint = static_cast<float *>(ctx->mfma_hint.ptr);
     uint32_t *qidx = static_cast<uint32_t *>(ctx->mfma_queue.ptr);
     float *qthr = reinterpret_cast<float *>(qidx + std::max<uint64_t>(n, 1));
     ctx->mfma_qlen = qlen;
     {
         KernelTimer t(ctx, "MfmaPrepare", stream);
         hipLaunchKernelGGL(fp16 ? mfma_prepare_kernel<true> : mfma_prepare_kernel<false>, dim3(l.ntiles), dim3(256), 0,
-                           stream, centroids, (uint32_t)d, (uint32_t)k, l.nkb, table, norm, tiles, cenT, qlen, hint_out);
+                           stream, centroids, (uint32_t)d, (uint32_t)k, l.nkb, table, norm, tiles, cenT, qlen, hint);
         CLK_HIP_CHECK(hipGetLastError());
     }
     if (n == 0)
@@ -704,7 +703,7 @@ int launch_labeling_mfma(clk_context *ctx, bool fp16, uint64_t d, uint64_t n, ui
             pinned ? reinterpret_cast<const f32v4 *>(pin_ops + pin_ops_count(n, l.nkb)) : nullptr;
         hipLaunchKernelGGL(lk, dim3((unsigned)grid), dim3(fast_block), lds, stream, points, n,
                            (uint32_t)d, (uint32_t)k, table, norm, tiles, l.ntiles, prm, labels,
-                           qidx, qthr, qlen, hint_in, hint_out, qbuf_ok, pin_ops, pin_x2);
+                           qidx, qthr, qlen, hint + 1, hint, qbuf_ok, pin_ops, pin_x2);
         CLK_HIP_CHECK(hipGetLastError());
     }
     // a resident grid, a work-group per batch of 64 points (8000 points d=24

@@ -1,7 +1,9 @@
-"""Operators that need no scratch memory of their own are captured into a graph
-on a context that has none yet (where growing it would break the capture): the
-global-atomic mass update and the centroid update of many clusters.  Every
-replay gives the eager result, with the program's own eager work between."""
+"""Captured operators.  Those that need no scratch memory of their own (the
+global-atomic mass update, the centroid update of many clusters) are captured
+into a graph on a context that has none yet, where growing it would break the
+capture; a graph of one MFMA labeling, whose replays hand the score offset on.
+Every replay gives the eager result, with the program's own eager work
+between."""
 import ctypes
 
 import numpy as np
@@ -75,5 +77,31 @@ def test_centroid_update(n, d, k):
         hip.synchronize()
         g.launch()
         np.testing.assert_array_equal(sums.to_host(), O.sums_grid(pts, lab, k, O.grid_scales(pts)))
+    g.close()
+    ctx.close()
+
+
+@pytest.mark.parametrize("strategy", ["mfma_fp16", "mfma_bf16"])
+@pytest.mark.parametrize("warm", [1, 2])
+def test_mfma_labeling(strategy, warm):
+    n, d, k = 30000, 40, 100
+    ctx = clkmeans.Context(0)
+    pts, _ = clkmeans.generate_blobs(n, d, k, sigma=1.0, box=3.0, seed=5)
+    cen = np.ascontiguousarray(pts[:, :k])
+    dp, dc, dl = dev(pts), dev(cen), zeros(n, np.uint32)
+    cfg = ctx.config(clkmeans.STAGE_LABELING, strategy)
+    for _ in range(warm):  # the scratch memory
+        ctx.labeling(cfg, d, n, k, dp, dc, dl)
+    g = Graph(lambda st: ctx.labeling(cfg, d, n, k, dp, dc, dl, stream=st))
+    for scale in (1.0, 50.0, 0.01, 1.0):  # the offset of one replay does not fit the next one's data
+        p = (pts * np.float32(scale)).astype(np.float32)
+        c = np.ascontiguousarray(p[:, :k])
+        dp.copy_from(p)
+        dc.copy_from(c)
+        for _ in range(2):
+            hip.synchronize()
+            g.launch()
+            np.testing.assert_array_equal(dl.to_host(), O.label(p, c))
+        ctx.labeling(cfg, d, n, k, dp, dc, dl)
     g.close()
     ctx.close()
