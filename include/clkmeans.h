@@ -195,7 +195,7 @@ int clk_lloyd_step(clk_context *ctx, const clk_kernel_config *cfg, uint64_t d,
  * calls that overlap in time on one GPU race (order them on one stream).
  * No profiling records are taken.
  */
-#define CLK_NOALLOC_SCRATCH_BYTES (8u << 20)
+#define CLK_NOALLOC_SCRATCH_BYTES (12u << 20)
 int clk_lloyd_step_noalloc(clk_context *ctx, const clk_kernel_config *cfg, uint64_t d,
                            uint64_t n, uint64_t k, const float *points,
                            const float *old_centroids, float *new_centroids, double *sums,
