@@ -45,7 +45,10 @@ TimedEvent TimedEvent::begin(hipStream_t s)
 void TimedEvent::finish(hipStream_t s)
 {
     end = make_event(hipEventDefault);
-    (void)hipEventRecord(end.get(), s);
+    // the operator's completion event too: a wait for one that was never
+    // recorded would return at once
+    if (hipEventRecord(end.get(), s) != hipSuccess)
+        throw std::runtime_error("hipEventRecord failed");
 }
 
 uint64_t TimedEvent::duration_ns() const
