@@ -2,9 +2,9 @@
 // for the sizes where the sequential-fma scan is bound by its vector
 // operations: 2 per feature and centroid plus the argmin, against 2.5 per
 // centroid for ranking matrix-core scores.  Measured with the launches
-// included, before -> now: fused step 2.5M points d=7 k=33 71 -> 44 us (13 of
-// them the points' bytes), 700k d=24 k=48 113 -> 45; 2^20 d=4 k=10 21.5 -> 18;
-// labeling 400k d=32 k=256 183 -> 44 us.  What is left is issue-bound: about
+// included, before -> now: fused step 2.5M points d=7 k=33 71 -> 45 us (13 of
+// them the points' bytes), 700k d=24 k=48 113 -> 45, 5M double d=4 k=10 58 ->
+// 53; labeling 400k d=32 k=256 187 -> 53 us.  What is left is issue-bound: about
 // 150 vector instructions per 64 points and 60 per tile of 16 centroids, the
 // matrix core (64 cycles per tile at P <= 8) only partly under them.
 #include "clk_common.hpp"
